@@ -6,6 +6,10 @@ table of the start position to depth 7 and depth 8, plus 16 seeded random
 positions (start position + 10..60 uniform-random legal plies) to depth 6 --
 107.2e9 leaves per step, every count checked against the reference's values.
 
+The step enumerates every board (pg_set_dedup off), as the reference's path
+without a table does; `merged` in the output is the same step with equal
+boards of a ply merged, which is what pg_perft does by default.
+
 Prints one JSON line: leaves/s over the timed steps, per-variant timings,
 the leaf kernel's roofline (integer VALU issue against the chip's vector
 peak, HBM bytes beside it) and the CPU baseline (the reference's own CPU
@@ -487,8 +491,9 @@ def main():
     counters = leg_counters(pg) if "counters" in legs_wanted else None
 
     jobs = load_workload(pg)
-    # headline steps: each perft is one graph launch (no per-kernel events)
+    # headline steps: no per-kernel events, every board enumerated
     dev = pg.Device(0, arena_bytes=48 << 30)
+    dev.set_dedup(False)
     _, _, _, clk_khz, cus = dev.issue_rate(0, 16)
 
     # per-variant pass (the slider choice for this path); skipped when a
@@ -511,6 +516,18 @@ def main():
         leaves += run_step(dev, jobs, best)
     elapsed = max(time.perf_counter() - t0, 1e-9)
     value = leaves / elapsed
+
+    # the same step as pg_perft runs it by default: equal boards of a ply merged
+    dev.set_dedup(True)
+    merged = None
+    if args.steps > 0 and best != pg.SLIDER_MAGIC_BYTE:   # (the byte-lookup variant does not merge)
+        run_step(dev, jobs, best)
+        t = time.perf_counter()
+        for _ in range(args.steps):
+            n = run_step(dev, jobs, best)
+        dt = (time.perf_counter() - t) / args.steps
+        merged = {"leaves_per_s": n / dt, "ms_per_step": dt * 1e3}
+        log("equal boards merged: %.2f ms per step" % (dt * 1e3))
 
     # roofline pass: the same step once more on a context that brackets every
     # leaf-kernel launch with HIP events on its launch stream (the host-driven
@@ -568,7 +585,7 @@ def main():
         "config": {"workload": "plain GPU BFS perft, no TT: start position d7 + d8 and 16 seeded random "
                                "positions (ply 10-60) at d6", "leaves_per_step": leaves // max(1, args.steps),
                    "slider": pg.SLIDER_NAMES[best], "exact": True},
-        "variants": variants, "roofline": roofline,
+        "variants": variants, "merged": merged, "roofline": roofline,
         "leaf_totals": {"launches": acc["launches"], "items": acc["items"], "parents": acc["parents"],
                         "grandparents": acc["grandparents"], "ms": acc["ms"]},
     }

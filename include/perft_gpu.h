@@ -68,12 +68,13 @@ typedef struct pg_stats {
     double total_ms;          /* wall time of the last perft call */
     double leaf_kernel_ms;    /* summed duration of leaf-kernel launches (timing=1) */
     uint64_t leaf_launches;   /* leaf-kernel launches in the last call */
-    uint64_t leaf_items;      /* (parent, move) items the leaf kernels consumed */
+    uint64_t leaf_items;      /* (parent, move) items the leaf kernels consumed (merged boards once) */
     uint64_t leaf_parents;    /* parent boards the leaf kernels read */
     uint64_t leaves;          /* the perft result */
     uint64_t splits;          /* level splits forced by the arena budget */
     uint64_t peak_arena;      /* peak arena bytes in use */
-    uint64_t nodes[16];       /* boards materialized per ply below the root */
+    uint64_t nodes[16];       /* pg_perft: perft(ply), each ply's boards (merged boards as many times as
+                                 they are reached); pg_perft_tt: boards made per ply */
 } pg_stats;
 
 /* ------------------------------------------------------------ host side */
@@ -132,7 +133,11 @@ int pg_set_slider(pg_ctx *ctx, int slider);
 
 /* perftLauncher, no-TT branch (launcher.h:1455-1503) driving
  * perft_bb_driver_gpu / perft_bb_gpu_simple (perft_bb.h:1027-1220):
- * breadth-first perft of one position; returns the leaf count. */
+ * breadth-first perft of one position; returns the leaf count.  Unless
+ * pg_set_dedup is off, equal boards of a ply are merged and counted once,
+ * times the paths that reach them (boards are compared in full: the count
+ * is exact).  The byte-lookup variant, timing = 1 and leaf_mode = 1 take
+ * every board by itself. */
 int pg_perft(pg_ctx *ctx, const pg_pos48 *pos, uint32_t depth, int slider, uint64_t *out);
 /* No counterpart in the reference.  pg_perft for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
@@ -244,7 +249,8 @@ int pg_perft_records(pg_ctx *ctx, pg_tt *tt, const char *in_path, uint32_t depth
  * pseudo-random words; lookups must then miss, never return garbage. */
 int pg_tt_poison(pg_tt *tt, uint64_t seed);
 /* FIND_DUPLICATES_IN_BFS (switches.h:52): 1 (default) collapses identical
- * positions within a level before expanding them. */
+ * positions within a level before expanding them, in pg_perft and
+ * pg_perft_tt. */
 int pg_set_dedup(pg_ctx *ctx, int on);
 
 /* ------------------------------------------------------------- batches */

@@ -189,8 +189,7 @@ static __global__ __launch_bounds__(SCAN_WG) void kd_scan_down(Plan *P, int l) {
 }
 
 // allocate level l+1 (children of l) and the transient arrays; a total-only
-// search keeps just boards and counts per level, and for its last expansion
-// (total == 2) only the moves and parents: the leaf makes those children.
+// search (total == 1) keeps just boards and counts per level.
 // total == 3: the last level of a search with per-board results and keys
 // keeps no boards or counts, only keys, perfts, states and owners; the moves
 // and parents stay until the leaf, which makes the children from them.
@@ -224,13 +223,6 @@ __device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int tot
             return;
         }
         C.n = m;
-        return;
-    }
-    if (total == 2) {
-        L.release = P->top;
-        L.mv = (u16 *)plan_alloc(P, m * 2);
-        L.par = (u32 *)plan_alloc(P, m * 4);
-        if (!P->overflow) C.n = m;
         return;
     }
     C.b = (Pos *)plan_alloc(P, m * sizeof(Pos));
@@ -450,15 +442,14 @@ static __global__ __launch_bounds__(LIVE_WG) void kd_live(Plan *P, int l) {
     }
 }
 
-// perft(2) of the boards of level l, fused (see leaf_tiles): per board into
-// the level's perft array, or (TOTAL, a single-root search that only needs
-// the sum) added to the plan's total
-template <int V, bool TOTAL>
+// perft(2) of the boards of level l, fused (see leaf_tiles), per board into
+// the level's perft array
+template <int V>
 __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void kd_leaf(Plan *P, int l, Tables t) {
     const DLevel L = P->lv[l];
-    const bool listed = !TOTAL && L.live;
-    leaf_tiles<V, !TOTAL>(L.b, L.cnt, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft, L.state,
-                          l == 0 ? P->bias : 0, &P->err, &P->ovf, t, listed ? L.live : nullptr);
+    const bool listed = L.live;
+    leaf_tiles<V, true>(L.b, L.cnt, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft, L.state,
+                        l == 0 ? P->bias : 0, &P->err, &P->ovf, t, listed ? L.live : nullptr);
 }
 
 // perft(2) of the children of level l-1 that form level l when level l keeps
@@ -473,17 +464,6 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL
     leaf_tiles<V, true, true>(A.b, nullptr, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft,
                               listed ? nullptr : L.state, 0, &P->err, &P->ovf, t, listed ? L.live : nullptr, A.par,
                               A.mv);
-}
-
-// perft(3) of the boards of level l summed into the plan's total: the
-// children of level l (its move list) are made, counted and expanded inside
-// the fused leaf (leaf_tiles, MOVES)
-template <int V>
-__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void kd_leaf_moves(
-    Plan *P, int l, Tables t) {
-    const DLevel L = P->lv[l];
-    leaf_tiles<V, false, true>(L.b, nullptr, P->lv[l + 1].n, &P->acc, &P->leafItems, nullptr, nullptr, 0, &P->err,
-                               &P->ovf, t, nullptr, L.par, L.mv);
 }
 
 // the plan's total += the move counts of level l (perft(1) of a total-only search)

@@ -28,10 +28,18 @@ int scratch_setup(int device, u8 **out);  // device address of the static scratc
     default: fn<SL_BYTE>(__VA_ARGS__); break;        \
     }
 
+// the variants whose tables leave the LDS to the fused leaf (not the byte lookup)
+#define PG_VARIANT_CALL_LDS(v, fn, ...)              \
+    switch (v) {                                     \
+    case SL_KOGGE: fn<SL_KOGGE>(__VA_ARGS__); break; \
+    case SL_PLAIN: fn<SL_PLAIN>(__VA_ARGS__); break; \
+    default: fn<SL_FANCY>(__VA_ARGS__); break;       \
+    }
 
 struct TTable;
 struct Slot;
 struct Server;
+struct Single;
 
 struct Engine {
     int device = 0, cus = 0, bpc = 8, slider = SL_KOGGE;
@@ -73,6 +81,8 @@ struct Engine {
 
     // batched searches (graph.hip)
     Slot *batchSlot = nullptr;
+    // single-root searches (single.hip)
+    Single *single = nullptr;
     // tables and slot servers created on this context; pg_shutdown releases
     // those still alive
     std::vector<TTable *> tts;
@@ -92,6 +102,8 @@ void slot_delete(Slot *sl);
 void slot_forget_tt(Slot &sl, const TTable *tt);  // drop graphs that bake this table in
 int batch_perft(Engine &e, Slot &sl, TTable *tt, const Pos *roots, u64 n, u32 depth, int v, int dedup, int bpc,
                 u64 *out, pg_batch_stats *bs);
+int perft_single(Engine &e, const Pos &root, u32 depth, int v, bool collapse, u64 *out, bool *fits);
+void single_delete(Single *s);
 int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fits);
 void tt_free(TTable *t);      // release a table (no users left)
 void server_free(Server *s);  // release a slot server

@@ -278,14 +278,21 @@ int Engine::perft(const Pos &root, u32 depth, int v, u64 *out) {
     top = 0;
     peak = 0;
     if (depth == 0) { *out = 1; return PG_OK; }
-    // Whole search as one graph launch (no host round trip between levels)
-    // unless each leaf launch is to be timed with events, the materialized
-    // leaf is asked for, or the call must not allocate (its plan and graphs
-    // are created on first use).  A search whose levels do not fit the arena
-    // falls back to the host-driven loop below, which splits levels.
+    // Whole search without a host round trip between levels unless each leaf
+    // launch is to be timed with events, the materialized leaf is asked for,
+    // or the call must not allocate (its plan is created on first use).  The
+    // collapsing search takes more arena per board of its last ply than the
+    // plain one, so that is tried next; a search that fits neither way falls
+    // back to the host-driven loop below, which splits levels.
     if (!timing && leafMode == 0 && graphPerft) {
         bool fits = false;
-        const int rc = perft_graph(*this, root, depth, v, out, &fits);
+        int rc;
+        if (v == SL_BYTE) {
+            rc = perft_graph(*this, root, depth, v, out, &fits);
+        } else {
+            rc = perft_single(*this, root, depth, v, dedup, out, &fits);
+            if (!rc && !fits && dedup) rc = perft_single(*this, root, depth, v, false, out, &fits);
+        }
         if (rc) return rc;
         if (fits) {
             stats.leaves = *out;
@@ -450,6 +457,8 @@ void pg_shutdown(pg_ctx *c) {
     while (!c->tts.empty()) tt_free(c->tts.back());
     slot_delete(c->batchSlot);
     c->batchSlot = nullptr;
+    single_delete(c->single);
+    c->single = nullptr;
     if (c->arena) (void)hipFree(c->arena);
     if (c->dTables) (void)hipFree(c->dTables);
     if (c->dSmall) (void)hipFree(c->dSmall);

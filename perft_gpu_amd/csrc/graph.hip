@@ -98,10 +98,7 @@ template <int V> static void cap_expand(hipStream_t s, Plan *P, int l, const TTV
     kd_expand<V><<<g, wg_size<V>(), 0, s>>>(P, l, tt, rc, ctr, t);
 }
 template <int V> static void cap_leaf(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
-    if constexpr (V != SL_BYTE) kd_leaf<V, false><<<g, LEAF_WG, 0, s>>>(P, l, t);
-}
-template <int V> static void cap_leaf_total(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
-    if constexpr (V != SL_BYTE) kd_leaf<V, true><<<g, LEAF_WG, 0, s>>>(P, l, t);
+    if constexpr (V != SL_BYTE) kd_leaf<V><<<g, LEAF_WG, 0, s>>>(P, l, t);
 }
 template <int V> static void cap_expand_keys(hipStream_t s, Plan *P, int l, const TTView &tt, int rc, TTCounters *ctr,
                                              int g, const Tables &t) {
@@ -110,37 +107,24 @@ template <int V> static void cap_expand_keys(hipStream_t s, Plan *P, int l, cons
 template <int V> static void cap_leaf_keys(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
     if constexpr (V != SL_BYTE) kd_leaf_keys<V><<<g, LEAF_WG, 0, s>>>(P, l, t);
 }
-template <int V> static void cap_leaf_moves(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
-    if constexpr (V != SL_BYTE) kd_leaf_moves<V><<<g, LEAF_WG, 0, s>>>(P, l, t);
-}
 
-// The search of one root when only its perft is wanted: per level just
-// boards and counts (no keys, table or per-board sums), the leaf adds into the
-// plan's total.
+// The search of one root when only its perft is wanted, for the byte-lookup
+// variant (the others run single.hip): per level just boards and counts (no
+// keys, table or per-board sums), down to the boards whose counts are summed.
 static void enqueue_total(const Engine &e, hipStream_t s, Plan *P, const GraphShape &sh) {
     const int D = sh.depth, v = sh.v;
     const Grids G = grids_for(e, sh);
     const int gWork = G.work, gScan = G.scan, gv = G.v;
     PG_VARIANT_CALL(v, cap_count, s, P, gv, e.dt);
-    const int lastExpand = v == SL_BYTE ? D - 2 : D - 3;
-    for (int l = 0; l <= lastExpand; l++) {
-        // with the fused leaf the last expansion lists moves only: the leaf
-        // makes and counts those children itself (kd_leaf_moves)
-        const bool movesOnly = v != SL_BYTE && l == lastExpand;
+    for (int l = 0; l <= D - 2; l++) {
         kd_plan_scan<<<1, 64, 0, s>>>(P, l);
         kd_scan_reduce<<<gScan, SCAN_WG, 0, s>>>(P, l);
-        kd_scan_spine<<<1, 1024, 0, s>>>(P, l, 0, 0, movesOnly ? 2 : 1);
+        kd_scan_spine<<<1, 1024, 0, s>>>(P, l, 0, 0, 1);
         kd_scan_down<<<gScan, SCAN_WG, 0, s>>>(P, l);
         PG_VARIANT_CALL(v, cap_generate, s, P, l, gv, e.dt);
-        if (movesOnly) {
-            PG_VARIANT_CALL(v, cap_leaf_moves, s, P, l, G.leaf, e.dt);
-            return;
-        }
         PG_VARIANT_CALL(v, cap_expand, s, P, l, TTView{}, D - l - 1, (TTCounters *)nullptr, gv, e.dt);
     }
-    const int last = lastExpand + 1 < 0 ? 0 : lastExpand + 1;  // deepest materialized level
-    if (D == 1 || v == SL_BYTE) kd_sum_counts<<<gWork, 256, 0, s>>>(P, last);
-    else PG_VARIANT_CALL(v, cap_leaf_total, s, P, last, G.leaf, e.dt);
+    kd_sum_counts<<<gWork, 256, 0, s>>>(P, D - 1);
 }
 
 // Enqueues the whole search for `depth` on stream s (captured by the caller).
@@ -323,8 +307,8 @@ void slot_forget_tt(Slot &sl, const TTable *tt) {
     }
 }
 
-// perft of one root through a total-only graph on the context's batch slot:
-// no host round trip between levels.  *fits is false (and nothing is
+// perft of one root through a total-only graph on the context's batch slot
+// (the byte-lookup variant): no host round trip between levels.  *fits is false (and nothing is
 // returned) when a level does not fit the arena; the caller then runs the
 // host-driven search, which splits levels.
 int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fits) {
@@ -367,11 +351,7 @@ int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fi
     }
     *fits = true;
     *out = h.acc;
-    e.stats.leaf_items = h.leafItems;
-    e.stats.leaf_launches = depth >= 2 && v != SL_BYTE ? 1 : 0;
     for (u32 l = 1; l < depth && l < 16; l++) e.stats.nodes[l] = h.lv[l].n;
-    if (depth >= 2 && depth - 1 < 16 && v != SL_BYTE) e.stats.nodes[depth - 1] = h.leafItems;
-    if (depth >= 2 && v != SL_BYTE) e.stats.leaf_parents = h.lv[depth - 2].n;
     return PG_OK;
 }
 

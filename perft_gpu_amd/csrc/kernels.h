@@ -31,7 +31,7 @@ __device__ __forceinline__ u64 wave_sum(u64 v) {
 // cannot wrap: it counts at most a few million moves per lane.
 __device__ __forceinline__ void add_checked(u64 *acc, u64 s, u32 *ovf) {
     const u64 old = atomicAdd(acc, s);
-    if (old + s < old) *ovf = 1;
+    if (old + s < old) atomicOr(ovf, 1u);
 }
 
 // sum of v[lo..hi) with a carry check
