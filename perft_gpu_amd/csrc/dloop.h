@@ -445,7 +445,7 @@ static __global__ __launch_bounds__(LIVE_WG) void kd_live(Plan *P, int l) {
 // perft(2) of the boards of level l, fused (see leaf_tiles), per board into
 // the level's perft array
 template <int V>
-__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void kd_leaf(Plan *P, int l, Tables t) {
+__global__ PG_LEAF_BOUNDS void kd_leaf(Plan *P, int l, Tables t) {
     const DLevel L = P->lv[l];
     const bool listed = L.live;
     leaf_tiles<V, true>(L.b, L.cnt, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft, L.state,
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL
 // keys only: the leaf makes each listed child from its parent and move (or,
 // without room for the list, every child, writing the live ones)
 template <int V>
-__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void kd_leaf_keys(
+__global__ PG_LEAF_BOUNDS void kd_leaf_keys(
     Plan *P, int l, Tables t) {
     const DLevel L = P->lv[l];
     const DLevel A = P->lv[l - 1];

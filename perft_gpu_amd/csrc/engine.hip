@@ -55,7 +55,7 @@ u32 Engine::grid(u64 n, int wg) const {
 // they free up, which balances the tail (start perft(8): 51.7 ms with 8
 // work-groups per CU, 47.0 ms with 64).
 u32 Engine::leaf_grid(u64 n) const {
-    u64 want = (n + LEAF_WG - 1) / LEAF_WG;
+    u64 want = (n + LEAF_WG - 1) / LEAF_WG;  // a tile of 64 boards per wave
     const u64 cap = (u64)cus * LEAF_BLOCKS_PER_CU;
     if (want > cap) want = cap;
     return (u32)(want ? want : 1);

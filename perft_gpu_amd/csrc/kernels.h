@@ -120,17 +120,6 @@ __device__ __forceinline__ u32 count_after(Pos p, u16 mv, const Tables &t) {
     make_move<WHITE, false>(p, mv, nullptr, t);
     return count_moves<BLACK, V>(p, t);
 }
-// the same with the moving piece known
-template <int V>
-__device__ __forceinline__ u32 count_after_as(Pos p, u16 mv, int piece, const Tables &t) {
-    if (pos_side(p)) {
-        make_move_as<BLACK, false>(p, mv, piece, nullptr, t);
-        return count_moves<WHITE, V>(p, t);
-    }
-    make_move_as<WHITE, false>(p, mv, piece, nullptr, t);
-    return count_moves<BLACK, V>(p, t);
-}
-
 template <int V>
 __global__ __launch_bounds__(wg_size<V>()) void k_count(const Pos *__restrict__ b, u64 n, u32 *__restrict__ cnt, Tables t) {
     stage_tables<V>(t);
@@ -156,7 +145,7 @@ static __global__ __launch_bounds__(256) void k_sum_u32(const u32 *__restrict__ 
 // Move lists and parent indices of boards [0, n) whose exclusive child
 // offsets are off[0..n].  A work-group takes 256 consecutive boards, whose
 // children form one contiguous output range: the boards generate into an LDS
-// window (move, and owner | piece tag), then the work-group stores the window
+// window (WordSink), then the work-group stores the window
 // one lane per slot, so the HBM writes are coalesced and each byte is written
 // once.  Boards that do not fit the window wait for the next pass.  err is
 // set to 1 if a board generates a different number of moves than it counted
@@ -167,8 +156,7 @@ template <int V>
 __device__ __forceinline__ void generate_tiles(const Pos *__restrict__ b, u64 n, const u64 *__restrict__ off,
                                                u16 *__restrict__ moves, u32 *__restrict__ parent, u32 *err,
                                                const Tables &t) {
-    __shared__ u16 smv[GEN_WINDOW];
-    __shared__ u16 stag[GEN_WINDOW];
+    __shared__ u32 word[GEN_WINDOW];
     __shared__ u32 snext;
     const int tid = threadIdx.x;
     for (u64 tile = blockIdx.x; tile * GEN_WG < n; tile += gridDim.x) {
@@ -186,7 +174,7 @@ __device__ __forceinline__ void generate_tiles(const Pos *__restrict__ b, u64 n,
             if (tid == 0) snext = total;
             __syncthreads();
             if (c && pos >= start && pos + c <= end) {
-                const u32 g = generate_any<V>(b[i], t, smv + (pos - start), c, stag + (pos - start), (u32)tid);
+                const u32 g = generate_words<V>(b[i], t, word + (pos - start), c, (u32)tid);
                 if (g != c) *err = 1;
             } else if (c && pos >= start) {
                 atomicMin(&snext, pos);
@@ -194,8 +182,9 @@ __device__ __forceinline__ void generate_tiles(const Pos *__restrict__ b, u64 n,
             __syncthreads();
             const u32 wend = snext;
             for (u32 j = start + tid; j < wend; j += GEN_WG) {
-                moves[base + j] = smv[j - start];
-                parent[base + j] = (u32)first + (stag[j - start] & 255u);
+                const u32 w = word[j - start];
+                moves[base + j] = (u16)w;
+                parent[base + j] = (u32)first + (w >> 16 & 255u);
             }
             __syncthreads();
             start = wend;
@@ -280,20 +269,143 @@ __device__ __forceinline__ u64 block_excl_scan(u64 v, u64 *total) {
 }
 
 // ---------------------------------------------------------------- fused leaf
-// The last two plies without touching HBM for the (parent, move) items: a
-// work-group takes 256 boards of ply D-2 and their move counts, scans the
-// counts in LDS, generates the moves into an LDS window of leaf_cap slots
-// (boards that do not fit wait for the next window) and counts the legal
-// moves of every child.  PER = also write each board's perft(2).
-// The window is as large as four work-groups per CU allow (160 KB of LDS:
-// at most 40 KB each with the 12 KB of boards, 4 bytes per slot, and 1 KB of
-// per-board sums when PER): 256 boards average about 7000 children, so most
-// tiles then take one pass.
-constexpr int LEAF_WG = 256, LEAF_BLOCKS_PER_CU = 64;
-template <bool PER> constexpr int leaf_cap() { return PER ? 6848 : 7040; }
+// The last two plies without touching HBM for the (parent, move) items.  A
+// wave takes a tile of 64 boards of ply D-2, one per lane, and keeps them as
+// kin in LDS, split by side.  Their moves fall into classes (leaf_eval):
+//   quiet  neither square matters to any reply: all of a board's quiet moves
+//          have the same number of replies, so they are counted, not listed
+//   calm   the king's zone and the pins stay as they are: only the sliders,
+//          pawns and knights that can reply differently are counted again
+//   full   the others: the replies are counted from scratch
+// In games from the start 59 to 74 % of the moves of the first twenty plies
+// are quiet and 6 to 11 % full; later it is a quarter and a half.  Calm and
+// full moves are listed into an LDS window, from its front and from its end,
+// and counted a lane per move; boards that do not fit the window are worked
+// out again for the next one.  Moves that are more than a piece leaving one
+// square for another (castling, promotions, en passant) are put aside by the
+// lanes that meet them and counted afterwards through make_move: as a branch
+// in the main loop they would hold up nearly every wave.
+//
+// Bound by the issue of VALU instructions.  From the start position,
+// perft(8) without merging (119 M boards, 2.4 G listed and counted moves of
+// ply 7) the kernel takes 21.9 ms; as a count of every reply from a board
+// that each lane made itself it took 50.1 ms, the same with the kin in LDS
+// 44.9 and with quiet moves as well 23.7.
+//
+// No work-group barrier: working out the boards (a long chain, no listing)
+// and counting the replies overlap between the waves of a SIMD.  Four waves'
+// tiles of 7.4 KB of boards and 1488 window words are 53.5 KB, so that three
+// work-groups share a CU's 160 KB (which is handed out in pieces of 1280
+// bytes: 54.3 KB each no longer fit, 29.5 ms).  A tile of 64 boards lists 400
+// to 1700 moves: windows of 608 words take 27.5 ms, 1216 words 23.7, 1408
+// words 21.9.  Three waves per SIMD is also what the registers allow; for
+// four the compiler spills, for two (209 registers) it takes 28.3 ms.
+constexpr int LEAF_WG = 256, LEAF_TILE = 64, LEAF_CAP = 1488, LEAF_BLOCKS_PER_CU = 64;
+constexpr u32 LEAF_LATE = 1u << 29;  // window word: a special move that found no room in the aside list
 
 // state of a board after expansion (TT and batch searches)
 enum : u8 { ST_LIVE = 0, ST_HIT = 1, ST_DUP = 2 };
+
+struct LeafTile {
+    Kin k[LEAF_TILE];
+    u32 word[LEAF_CAP];
+    u32 per[LEAF_TILE];  // sum over a board's children
+};
+
+// this wave's number in its work-group, in a scalar register: what is
+// addressed by it, and loops over it, then stay out of the vector registers
+__device__ __forceinline__ u32 wave_number() { return (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// orders a wave's LDS accesses (each wave's are carried out in order; this
+// keeps the compiler from moving them)
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ u32 lanes_below(u64 mask) {
+    return __builtin_amdgcn_mbcnt_hi((u32)(mask >> 32), __builtin_amdgcn_mbcnt_lo((u32)mask, 0));
+}
+__device__ __forceinline__ u32 wave_excl_scan(u32 v, u32 *total) {
+    const int lane = threadIdx.x & 63;
+    u32 x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const u32 y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    *total = __shfl(x, 63, 64);
+    return x - v;
+}
+
+// per[lane] = perft(2) of the wave's boards (lane's board b when live).
+// Returns this lane's number of moves; all lanes of the wave call it.  err is
+// set if a board lists a different number of moves than it counted.
+template <int V>
+__device__ __forceinline__ u32 leaf_expand(LeafTile &s, bool live, const Pos &b, u32 *err, const Tables &t) {
+    const u32 lane = threadIdx.x & 63;
+    if (live) s.k[lane] = kin_any(b, t);
+    u32 moves = 0;
+    for (u64 pending = __ballot(live); pending;) {
+        // the boards still to do (one that did not fit the window is worked
+        // out again: nothing of it is held while the others are counted)
+        wave_sync();
+        LeafEval q{};
+        if (pending >> lane & 1) q = leaf_any(s.k[lane], t);
+        const u32 list = q.calm + q.full;
+        u32 totals;  // calm moves in the low half, the others in the high half
+        const u32 at = wave_excl_scan(q.calm | q.full << 16, &totals), atCalm = at & 0xFFFF, atFull = at >> 16;
+        // calm moves fill the window from its front, the others from its end
+        const bool due = pending >> lane & 1, fits = due && atCalm + atFull + list <= LEAF_CAP;
+        if (fits) {
+            LeafSink o{s.word, LEAF_CAP, lane, atCalm, LEAF_CAP - 1 - atFull};
+            generate_leaf<V>(s.k[lane], q.g, t, o);
+            if (o.calm != atCalm + q.calm || o.full + atFull + q.full != LEAF_CAP - 1) atomicOr(err, 2u);
+            s.per[lane] = q.quiet * q.c0;
+            moves = list + q.quiet;
+        }
+        pending = __ballot(due && !fits);
+        const u32 n = pending ? __shfl(at, __builtin_ctzll(pending), 64) : totals;
+        const u32 nCalm = n & 0xFFFF, nFull = n >> 16;
+        wave_sync();
+        for (u32 j = lane; j < nCalm; j += 64) {
+            const u32 w = s.word[j], o = w >> 16 & 255;
+            atomicAdd(&s.per[o], count_calm_any(s.k[o], w, t));
+        }
+        wave_sync();
+        u32 *const word = s.word + LEAF_CAP - 1;
+        // special moves are put aside: their places, two to a word, in the
+        // part of the window that is free again
+        u16 *const aside = (u16 *)s.word;
+        const u32 room = 2 * (LEAF_CAP - nFull);
+        u32 asides = 0;
+        for (u32 j0 = 0; j0 < nFull; j0 += 64) {
+            const u32 j = j0 + lane;
+            const u32 w = j < nFull ? word[-(int)j] : 0;
+            const u64 special = __ballot(w >> 31);
+            if (special) {
+                if (w >> 31) {
+                    const u32 a = asides + lanes_below(special);
+                    if (a < room) aside[a] = (u16)j;
+                    else word[-(int)j] = w | LEAF_LATE;
+                }
+                asides += (u32)__popcll(special);
+            }
+            if (j < nFull && !(w >> 31)) {
+                const u32 o = w >> 16 & 255;
+                atomicAdd(&s.per[o], count_child_any<V>(s.k[o], w, t));
+            }
+        }
+        wave_sync();
+        // those put aside, then (only if the list was full) the window's late ones
+        const u32 m = asides < room ? asides : room, late = asides > room ? nFull : 0;
+        for (u32 j = lane; j < m + late; j += 64) {
+            const u32 w = word[-(int)(j < m ? aside[j] : j - m)], o = w >> 16 & 255;
+            if (j < m || (w & LEAF_LATE)) atomicAdd(&s.per[o], count_made<V>(s.k[o], w, t));
+        }
+        wave_sync();
+    }
+    return moves;
+}
 
 // The fused leaf over boards [0, n) with move counts cnt[]: PER = false adds
 // every count to *acc; PER = true writes base + perft(2) to per[i] for live
@@ -311,81 +423,56 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
                                            u32 *err, u32 *ovf, const Tables &t, const u32 *__restrict__ idx = nullptr,
                                            const u32 *__restrict__ par = nullptr, const u16 *__restrict__ mv = nullptr) {
     static_assert(V != SL_BYTE, "the byte-lookup tables leave no LDS for the move window");
-    __shared__ Pos sb[LEAF_WG];
-    constexpr int LEAF_CAP = leaf_cap<PER>();
-    __shared__ u16 smv[LEAF_CAP];
-    __shared__ u16 stag[LEAF_CAP];  // owner | moving piece << 8
-    __shared__ u32 sper[PER ? LEAF_WG : 1];
-    __shared__ u32 snext;
-    const int tid = threadIdx.x;
-    const Tables &tl = t;
-    u64 s = 0, itemSum = 0;
-    for (u64 tile = blockIdx.x; tile * LEAF_WG < n; tile += gridDim.x) {
-        const u64 t0 = tile * LEAF_WG + tid;
+    constexpr u32 WAVES = LEAF_WG / 64;
+    __shared__ LeafTile tiles[WAVES];
+    const u32 wave = wave_number();
+    LeafTile &s = tiles[wave];
+    const u32 lane = threadIdx.x & 63;
+    u64 sum = 0, itemSum = 0;
+    for (u64 tile = blockIdx.x * WAVES + wave; tile * LEAF_TILE < n; tile += gridDim.x * WAVES) {
+        const u64 t0 = tile * LEAF_TILE + lane;
         const bool live = t0 < n;
         const u64 i = idx && live ? (u64)idx[t0] : t0;
-        u32 c = 0;
-        if constexpr (MOVES) {
-            if (live) {
-                Pos b = boards[par[i]];
-                make_any(b, mv[i], tl);
-                c = count_any<V>(b, tl);
-                sb[tid] = b;
+        bool valid = false, work = live;
+        Pos b{};
+        if (live) {
+            if constexpr (MOVES) {
+                b = boards[par[i]];
+                make_any(b, mv[i], t);
+            } else {
+                b = boards[i];
+                valid = pos_valid(b);
+                work = cnt[i] != 0;  // a board resolved earlier has count 0
             }
-        } else {
-            c = live ? cnt[i] : 0;
-            if (live) sb[tid] = boards[i];
         }
-        if (PER) sper[tid] = 0;
-        u64 total64;
-        const u32 pos = (u32)block_excl_scan<LEAF_WG>(c, &total64);
-        const u32 total = (u32)total64;
-        itemSum += total64;
-        u32 start = 0;
-        while (start < total) {
-            const u32 end = start + LEAF_CAP;
-            if (tid == 0) snext = total;
-            __syncthreads();
-            const bool here = c && pos >= start && pos + c <= end;
-            if (here) {
-                const u32 g = generate_any<V>(sb[tid], tl, smv + (pos - start), c, stag + (pos - start), (u32)tid);
-                if (g != c) *err = 2;
-            } else if (c && pos >= start) {
-                atomicMin(&snext, pos);
+        itemSum += leaf_expand<V>(s, work, b, err, t);
+        if (live) {
+            const u32 p = work ? s.per[lane] : 0;
+            if constexpr (PER) {
+                if (idx || (state ? state[i] == ST_LIVE : valid)) {
+                    const u64 v = base + p;
+                    if (v < base) *ovf = 1;
+                    per[i] = v;
+                }
+            } else {
+                sum += p;
             }
-            __syncthreads();
-            const u32 wend = snext;
-            for (u32 j = start + tid; j < wend; j += LEAF_WG) {
-                const u32 k = j - start;
-                const u32 tg = stag[k];
-                const int b = tg & 255;
-                const u32 m = count_after_as<V>(sb[b], smv[k], (int)(tg >> 8), tl);
-                if (PER) atomicAdd(&sper[b], m);
-                else s += m;
-            }
-            __syncthreads();
-            start = wend;
         }
-        if (PER && live && (idx || (state ? state[i] == ST_LIVE : pos_valid(sb[tid])))) {
-            const u64 v = base + sper[tid];
-            if (v < base) *ovf = 1;
-            per[i] = v;
-        }
-        __syncthreads();
+        wave_sync();
     }
-    if (tid == 0 && items && itemSum) atomicAdd(items, itemSum);
+    itemSum = wave_sum(itemSum);
+    if ((threadIdx.x & 63) == 0 && items && itemSum) atomicAdd(items, itemSum);
     if (!PER) {
-        s = wave_sum(s);
-        if ((tid & 63) == 0 && s) add_checked(acc, s, ovf);
+        sum = wave_sum(sum);
+        if ((threadIdx.x & 63) == 0 && sum) add_checked(acc, sum, ovf);
     }
 }
 
-// Occupancy targets: four waves per SIMD for Kogge-Stone, five for the magic
-// variants (their table lookups wait on L2, more waves hide it).  Some magic
-// instantiations do not fit five and the compiler says so (-Wpass-failed);
-// they end at four, and asking them for four measured no faster.
+// three waves per SIMD (see above); nothing spills at 168 registers
+#define PG_LEAF_BOUNDS __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(3, 8)))
+
 template <int V, bool PER>
-__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void k_leaf_fused(
+__global__ PG_LEAF_BOUNDS void k_leaf_fused(
     const Pos *__restrict__ boards, const u32 *__restrict__ cnt, u64 n, u64 *acc, u64 *items, u64 *__restrict__ per,
     u32 *err, u32 *ovf, Tables t, const u32 *__restrict__ idx) {
     leaf_tiles<V, PER>(boards, cnt, n, acc, items, per, nullptr, 0, err, ovf, t, idx);
@@ -393,7 +480,7 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL
 
 // the leaf over the children of `gp` listed by par/mv (see leaf_tiles, MOVES)
 template <int V>
-__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void k_leaf_moves(
+__global__ PG_LEAF_BOUNDS void k_leaf_moves(
     const Pos *__restrict__ gp, const u32 *__restrict__ par, const u16 *__restrict__ mv, u64 n, u64 *acc, u64 *items,
     u32 *err, u32 *ovf, Tables t) {
     leaf_tiles<V, false, true>(gp, nullptr, n, acc, items, nullptr, nullptr, 0, err, ovf, t, nullptr, par, mv);
@@ -402,7 +489,7 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL
 // per-child sums over the children of `gp` listed by idx (see leaf_tiles,
 // MOVES with idx): perft(2) of each listed child into per[]
 template <int V>
-__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(V == SL_KOGGE ? 4 : 5, 8))) void k_leaf_moves_per(
+__global__ PG_LEAF_BOUNDS void k_leaf_moves_per(
     const Pos *__restrict__ gp, const u32 *__restrict__ par, const u16 *__restrict__ mv, const u32 *__restrict__ idx,
     u64 n, u64 *items, u64 *__restrict__ per, u32 *err, u32 *ovf, Tables t) {
     leaf_tiles<V, true, true>(gp, nullptr, n, nullptr, items, per, nullptr, 0, err, ovf, t, idx, par, mv);

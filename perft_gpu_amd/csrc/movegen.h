@@ -1,7 +1,9 @@
 // movegen.h -- legal move counting, generation and make-move for gfx950.
 //
 // Written for 64-lane wavefronts: the leaf count is branch-light so that the
-// lanes of a wave (sibling positions) stay converged.
+// lanes of a wave (sibling positions) stay converged.  The leaf itself counts
+// the replies to a board's moves by difference (Kin, leaf_eval, count_child
+// below); what follows holds for the counting of one board by itself.
 //  * One "target" mask folds the reference's separate out-of-check path
 //    (MoveGeneratorBitboard.h:2825-2994) into the normal one: not in check ->
 //    ~own, single check -> checker | squares between, double check -> 0.
@@ -40,6 +42,19 @@ struct FancyEntry {
 };
 static_assert(sizeof(FancyEntry) == 16, "fancy entry is 16 bytes");
 
+// What a king's square determines, one cache line: the squares a rook, bishop
+// or knight there would reach on an empty board, the king's own steps, and
+// the whole file, rank and diagonals through it.
+struct KingRow {
+    u64 rook, bishop, knight, king, file, rank, diag, anti;
+};
+static_assert(sizeof(KingRow) == 64, "a king's row is one line");
+// For a king and a slider on one line: the squares strictly between, and the
+// square next to the king away from the slider (0: off the board).
+struct PinEntry {
+    u64 between, behind;
+};
+
 constexpr int ROOK_BITS = 12, BISHOP_BITS = 9;
 constexpr int FANCY_TABLE_SIZE = 97264, BYTE_ROOK_SIZE = 4900, BYTE_BISHOP_SIZE = 1428;
 constexpr int ZOB_WORDS = 782;
@@ -48,8 +63,8 @@ constexpr int ZOB_WORDS = 782;
 // variant repoints some of them at LDS copies).
 struct Tables {
     const u64 *knight, *king;            // [64] empty-board attacks
-    const u64 *rookEmpty, *bishopEmpty;  // [64]
-    const u64 *between;                  // [64*64] squares strictly between
+    const KingRow *row;                  // [64]
+    const PinEntry *pin;                 // [64*64] king, slider
     const u64 *line;                     // [64*64] full line through two squares
     const u64 *rookMask, *bishopMask;    // [64] relevant occupancy (edges off)
     const u64 *rookMagic, *bishopMagic;  // [64] plain magic factors
@@ -62,6 +77,22 @@ struct Tables {
 };
 
 PG_HD int popc(u64 x) { return __builtin_popcountll(x); }
+// n + popc(x), the two halves through the count instruction's own addend
+// (LLVM sums the halves first and adds with further instructions)
+PG_HD int popc_add(u64 x, int n) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_bcnt_u32_b32 %0, %1, %0" : "+v"(n) : "v"((u32)x));
+    asm("v_bcnt_u32_b32 %0, %1, %0" : "+v"(n) : "v"((u32)(x >> 32)));
+    return n;
+#else
+    return n + __builtin_popcountll(x);
+#endif
+}
+// all ones if c
+PG_HD u64 mask_if(bool c) {
+    const u32 m = c ? ~0u : 0u;
+    return (u64)m << 32 | m;
+}
 PG_HD int ctz(u64 x) { return __builtin_ctzll(x); }
 PG_HD u64 bit(int s) { return 1ULL << s; }
 PG_HD bool several(u64 x) { return (x & (x - 1)) != 0; }
@@ -178,6 +209,10 @@ template <int S> PG_HD u64 shift(u64 x) {
 #endif
     return S > 0 ? x << S : x >> -S;
 }
+PG_HD u64 and_mask(u64 x, u64 m) { return m == ~0ULL ? x : x & m; }
+template <int N> struct Int {
+    static constexpr int value = N;
+};
 struct Prop3 {
     u64 a, b, c;
 };
@@ -310,150 +345,280 @@ template <> struct Sl<SL_BYTE> {
 };
 
 // ---------------------------------------------------------------- context
-struct MoveCtx {
-    u64 occ, mine, enemy, myPawns, myKing, eRooks, pinned, checkers, threatened, target;
-    int k;
+// A board as the side to move sees it.  Bishops and rooks include the queens.
+struct Sides {
+    u64 occ, mine, enemy;
+    u64 myPawns, myKnights, myBishops, myRooks, myKing;
+    u64 ePawns, eKnights, eBishops, eRooks;
+    int k, ek;        // king squares, in range even for a board without a king
+    u32 castle, eCastle;  // castling rights of the side, of the enemy (2 bits each)
+    u32 ep;               // en-passant file + 1
 };
 
-template <int C, int V>
-PG_HD void prologue(const Pos &p, const Tables &t, MoveCtx &x) {
-    const u64 pawns = pos_pawns(p);
-    x.occ = p.kings | pawns | p.knights | p.bishopQueens | p.rookQueens;
-    const u64 black = x.occ & ~p.white;
-    x.mine = C == WHITE ? p.white : black;
-    x.enemy = C == WHITE ? black : p.white;
-    x.myPawns = pawns & x.mine;
-    x.myKing = p.kings & x.mine;
-    x.k = ctz(x.myKing) & 63;  // in range even for a board without a king
-    const u64 eP = pawns & x.enemy, eN = p.knights & x.enemy, eK = p.kings & x.enemy;
-    const u64 eB = p.bishopQueens & x.enemy, eR = p.rookQueens & x.enemy;
-    x.eRooks = eR;
+template <int C> PG_HD Sides sides_of(const Pos &p) {
+    Sides s;
+    const u64 W = p.white, pawns = pos_pawns(p);
+    s.occ = or3(p.kings, pawns, or3(p.knights, p.bishopQueens, p.rookQueens));
+    s.mine = C == WHITE ? W : andn(s.occ, W);
+    s.enemy = C == WHITE ? andn(s.occ, W) : W;
+    s.myPawns = side_of<C>(pawns, W);
+    s.myKnights = side_of<C>(p.knights, W);
+    s.myBishops = side_of<C>(p.bishopQueens, W);
+    s.myRooks = side_of<C>(p.rookQueens, W);
+    s.myKing = side_of<C>(p.kings, W);
+    s.ePawns = side_of<1 - C>(pawns, W);
+    s.eKnights = side_of<1 - C>(p.knights, W);
+    s.eBishops = side_of<1 - C>(p.bishopQueens, W);
+    s.eRooks = side_of<1 - C>(p.rookQueens, W);
+    s.k = ctz(s.myKing) & 63;
+    s.ek = ctz(side_of<1 - C>(p.kings, W)) & 63;
+    s.castle = (u32)(C == WHITE ? pos_wcastle(p) : pos_bcastle(p));
+    s.eCastle = (u32)(C == WHITE ? pos_bcastle(p) : pos_wcastle(p));
+    s.ep = (u32)pos_ep(p);
+    return s;
+}
 
-    // squares the enemy attacks, sliders looking through our king
-    u64 a;
-    {
-        const u64 pw = C == WHITE ? shift<-9>(eP) : shift<7>(eP), pe = C == WHITE ? shift<-7>(eP) : shift<9>(eP);
-        a = or3(t.king[ctz(eK) & 63], andn(pw, FILEH), andn(pe, FILEA));
-        const u64 h1 = or_and(andn(shift<-1>(eN), FILEH), shift<1>(eN), ~FILEA);
-        const u64 h2 = or_and(andn(shift<-2>(eN), FILEG | FILEH), shift<2>(eN), ~(FILEA | FILEB));
-        a = or3(a, shift<16>(h1), shift<-16>(h1));
-        a = or3(a, shift<8>(h2), shift<-8>(h2));
+struct MoveCtx {
+    u64 pinned, checkers, threatened, target;
+};
+
+// squares the enemy attacks with king, pawns and knights
+template <int C> PG_HD u64 leaper_attacks(const Sides &s, const Tables &t) {
+    const u64 pw = C == WHITE ? shift<-9>(s.ePawns) : shift<7>(s.ePawns);
+    const u64 pe = C == WHITE ? shift<-7>(s.ePawns) : shift<9>(s.ePawns);
+    u64 a = or3(t.king[s.ek], andn(pw, FILEH), andn(pe, FILEA));
+    const u64 h1 = or_and(andn(shift<-1>(s.eKnights), FILEH), shift<1>(s.eKnights), ~FILEA);
+    const u64 h2 = or_and(andn(shift<-2>(s.eKnights), FILEG | FILEH), shift<2>(s.eKnights), ~(FILEA | FILEB));
+    a = or3(a, shift<16>(h1), shift<-16>(h1));
+    return or3(a, shift<8>(h2), shift<-8>(h2));
+}
+
+// squares from which an enemy pawn or knight checks, as found
+template <int C> PG_HD u64 leaper_checks(const Sides &s, const Tables &t, u64 chk) {
+    const u64 kw = C == WHITE ? shift<7>(s.myKing) : shift<-9>(s.myKing);
+    const u64 ke = C == WHITE ? shift<9>(s.myKing) : shift<-7>(s.myKing);
+    return or_and(or_and(chk, or_and(andn(kw, FILEH), ke, ~FILEA), s.ePawns), t.row[s.k].knight, s.eKnights);
+}
+
+// Pinned pieces, checkers and the squares a move other than the king's must
+// end on; returns the squares behind the king on a slider's check line.
+// Sliders on a king line: no blocker -> checker, one blocker -> pinned.
+template <int C> PG_HD u64 pins_and_checks(const Sides &s, const Tables &t, MoveCtx &x) {
+    const KingRow &row = t.row[s.k];
+    u64 cand = or_and(row.rook & s.eRooks, row.bishop, s.eBishops);
+    u64 pinned = 0, chk = 0, behind = 0;
+    for (; cand; cand &= cand - 1) {
+        const int q = ctz(cand);
+        const PinEntry e = t.pin[(s.k << 6) | q];
+        const u64 b = e.between & s.occ;
+        // (masks: selects would be runs of v_cndmask on vcc, which issue slowly)
+        const u64 none = mask_if(b == 0);
+        pinned = or_and(pinned, b, mask_if(!several(b)));
+        chk = or_and(chk, bit(q), none);
+        behind = or_and(behind, e.behind, none);
     }
+    chk = leaper_checks<C>(s, t, chk);
+    x.pinned = pinned & s.mine;
+    x.checkers = chk;
+    u64 tgt = ~s.mine;
+    if (chk) tgt &= several(chk) ? 0ULL : (chk | t.pin[(s.k << 6) | ctz(chk)].between);
+    x.target = tgt;
+    return behind;
+}
+
+template <int C, int V>
+PG_HD void prologue(const Sides &s, const Tables &t, MoveCtx &x) {
+    // squares the enemy attacks, sliders looking through our king
+    u64 a = leaper_attacks<C>(s, t);
     if (Sl<V>::kBulk) {
-        a |= ks_attacks(eB, eR, ~x.occ | x.myKing);
+        a |= ks_attacks(s.eBishops, s.eRooks, ~s.occ | s.myKing);
     } else {
-        const u64 o = x.occ ^ x.myKing;
-        for (u64 b = eB; b; b &= b - 1) a |= Sl<V>::bishop(t, ctz(b), o);
-        for (u64 r = eR; r; r &= r - 1) a |= Sl<V>::rook(t, ctz(r), o);
+        const u64 o = s.occ ^ s.myKing;
+        for (u64 b = s.eBishops; b; b &= b - 1) a |= Sl<V>::bishop(t, ctz(b), o);
+        for (u64 r = s.eRooks; r; r &= r - 1) a |= Sl<V>::rook(t, ctz(r), o);
     }
     x.threatened = a;
 
-    // sliders on a king line: no blocker -> checker, one blocker -> pinned
-    u64 cand = (t.rookEmpty[x.k] & eR) | (t.bishopEmpty[x.k] & eB);
-    u64 pinned = 0, chk = 0;
-    for (; cand; cand &= cand - 1) {
-        const int s = ctz(cand);
-        const u64 b = t.between[(x.k << 6) | s] & x.occ;
-        if (b == 0) chk |= bit(s);
-        else if (!several(b)) pinned |= b;
-    }
-    chk |= (t.knight[x.k] & eN) | (pawn_att<C>(x.myKing) & eP);
-    x.pinned = pinned & x.mine;
-    x.checkers = chk;
-    u64 tgt = ~x.mine;
-    if (chk) tgt &= several(chk) ? 0ULL : (chk | t.between[(x.k << 6) | ctz(chk)]);
-    x.target = tgt;
+    (void)pins_and_checks<C>(s, t, x);
 }
 
 enum { P_PAWN = 1, P_KNIGHT, P_BISHOP, P_ROOK, P_QUEEN, P_KING };
+// The piece words that a moving piece belongs to, one bit each; a queen is in
+// both slider words.
+// M_SPECIAL marks a move that is more than a piece leaving one square for
+// another: a promotion, castling, an en-passant capture, or a double push that
+// lets the enemy capture en passant.
+enum : u32 { M_PAWN = 1, M_KNIGHT = 2, M_BISHOP = 4, M_ROOK = 8, M_QUEEN = 12, M_KING = 16, M_SPECIAL = 128 };
+PG_HD int piece_code(u32 m) {
+    constexpr u64 code = (u64)P_PAWN << 3 | (u64)P_KNIGHT << 6 | (u64)P_BISHOP << 12 | (u64)P_ROOK << 24 |
+                         (u64)P_QUEEN << 36 | (u64)P_KING << 48;
+    return (int)(code >> (3 * (m & 31))) & 7;
+}
 
-// Bounded move writer: never stores past `cap`, but keeps counting so a
-// caller can detect a mismatch with the counted size.  With `tag` set it also
-// stores owner | moving piece << 8 per move (the fused leaf's window), so the
-// child can be made without looking the piece up.
+// calls f(square) for every set square of m, low half then high half (a
+// 32-bit find-first-set and clear per square instead of the 64-bit ones)
+template <class F>
+PG_HD void each_square(u64 m, F &&f) {
+    for (u32 lo = (u32)m; lo; lo &= lo - 1) f(__builtin_ctz(lo));
+    for (u32 hi = (u32)(m >> 32); hi; hi &= hi - 1) f(32 + __builtin_ctz(hi));
+}
+// Move writers.  squares(m, full, piece, f): one move f(square) per square of
+// m, those on `full` to be counted in full (see Gen); add(move, piece): one
+// such move; skipped(m): quiet moves.  They are bounded: a writer never
+// stores past its cap, but keeps counting so a caller can detect a mismatch
+// with the counted size.
 struct MoveSink {
     u16 *out;
     u32 cap, n;
-    u16 *tag;
-    u32 owner;
-    PG_HD void add(u16 m, int piece) {
-        if (n < cap) {
-            out[n] = m;
-            if (tag) tag[n] = (u16)(owner | ((u32)piece << 8));
-        }
+    PG_HD void add(u32 m, u32) {
+        if (n < cap) out[n] = (u16)m;
         n++;
     }
+    template <class F> PG_HD void squares(u64 m, u64, u32 piece, F &&f) {
+        each_square(m, [&](int to) { add(f(to), piece); });
+    }
+    PG_HD void skipped(u64) {}
+};
+// A window of words, move | owner << 16 | moving piece and kind of move (M_*)
+// << 24, so that the child can be made without looking the piece up.  Moves
+// past the cap (>= 1) land on its last slot.
+struct WordSink {
+    u32 *out;
+    u32 cap, n, owner;
+    PG_HD void add(u32 m, u32 piece) {
+        out[n < cap ? n : cap - 1] = m | owner << 16 | piece << 24;
+        n++;
+    }
+    template <class F> PG_HD void squares(u64 m, u64, u32 piece, F &&f) {
+        each_square(m, [&](int to) { add(f(to), piece); });
+    }
+    PG_HD void skipped(u64) {}
+};
+// The fused leaf's window of `cap` words: calm moves upwards from place
+// `calm`, the others downwards from place `full`.  A place out of the window
+// (the numbers listed and counted differ) becomes its last.
+struct LeafSink {
+    u32 *word;
+    u32 cap, owner, calm, full;
+    PG_HD void put(u32 m, u32 piece, u32 isFull) {
+        const u32 at = isFull ? full : calm;
+        word[at < cap ? at : cap - 1] = m | owner << 16 | piece << 24;
+        full -= isFull;
+        calm += isFull ^ 1;
+    }
+    PG_HD void add(u32 m, u32 piece) { put(m, piece, 1); }
+    template <class F> PG_HD void squares(u64 m, u64 on, u32 piece, F &&f) {
+        each_square(m, [&](int to) { put(f(to), piece, (u32)(on >> to) & 1); });
+    }
+    PG_HD void skipped(u64) {}
+};
+struct NoSink {
+    PG_HD void add(u32, u32) {}
 };
 
 // en-passant: number of legal captures (MoveGeneratorBitboard.h:3050-3085,
-// and :2891-2902 when in check); writes them when `out` is given.
-template <int C>
-PG_HD int ep_moves(const Pos &p, const Tables &t, const MoveCtx &x, MoveSink *out) {
-    const int f = pos_ep(p);
+// and :2891-2902 when in check), each handed to the sink.
+template <int C, class Sink>
+PG_HD int ep_moves(const Sides &s, const Tables &t, const MoveCtx &x, Sink &out) {
+    const int f = (int)s.ep;
     if (!f) return 0;
     const u64 dst = C == WHITE ? bit(39 + f) : bit(15 + f);
     const u64 cap = C == WHITE ? dst >> 8 : dst << 8;
-    u64 src = (((cap << 1) & ~FILEA) | ((cap >> 1) & ~FILEH)) & x.myPawns;
+    u64 src = (((cap << 1) & ~FILEA) | ((cap >> 1) & ~FILEH)) & s.myPawns;
     int n = 0;
     const int to = ctz(dst);
     if (x.checkers) {
         if (x.checkers != cap) return 0;
         src &= ~x.pinned;
         for (; src; src &= src - 1) {
-            if (out) out->add((u16)(ctz(src) | (to << 6) | (MF_EP_CAPTURE << 12)), P_PAWN);
+            out.add((u32)(ctz(src) | (to << 6) | (MF_EP_CAPTURE << 12)), M_PAWN | M_SPECIAL);
             n++;
         }
         return n;
     }
     for (; src; src &= src - 1) {
-        const int s = ctz(src);
+        const int q = ctz(src);
         bool ok;
-        if (x.pinned & bit(s)) {
-            ok = (dst & t.line[(s << 6) | x.k]) != 0;
+        if (x.pinned & bit(q)) {
+            ok = (dst & t.line[(q << 6) | s.k]) != 0;
         } else {
             // both pawns leave the rank: no rook or queen may then see the king along it
-            const u64 e = ~x.occ | cap | bit(s), eH = andn(e, FILEH), eA = andn(e, FILEA);
-            const u64 ray = (eH ^ east_sum(x.eRooks, eH)) | (eA ^ rev64(east_sum(rev64(x.eRooks), rev64(eA))));
-            ok = (ray & x.myKing) == 0;
+            const u64 e = ~s.occ | cap | bit(q), eH = andn(e, FILEH), eA = andn(e, FILEA);
+            const u64 ray = (eH ^ east_sum(s.eRooks, eH)) | (eA ^ rev64(east_sum(rev64(s.eRooks), rev64(eA))));
+            ok = (ray & s.myKing) == 0;
         }
         if (ok) {
-            if (out) out->add((u16)(s | (to << 6) | (MF_EP_CAPTURE << 12)), P_PAWN);
+            out.add((u32)(q | (to << 6) | (MF_EP_CAPTURE << 12)), M_PAWN | M_SPECIAL);
             n++;
         }
     }
     return n;
 }
 
+// Castling moves: bit 0 king side, bit 1 queen side.  The squares lie in one
+// byte of the back rank; in it, e is bit 4.
 template <int C>
-PG_HD int castle_count(const Pos &p, const MoveCtx &x) {
-    if (x.checkers) return 0;
-    const int r = C == WHITE ? pos_wcastle(p) : pos_bcastle(p);
-    const int sh = C == WHITE ? 0 : 56;
-    int n = 0;
-    if ((r & 1) && !((0x60ULL << sh) & (x.occ | x.threatened))) n++;
-    if ((r & 2) && !((0x0EULL << sh) & x.occ) && !((0x0CULL << sh) & x.threatened)) n++;
-    return n;
+PG_HD u32 castle_bits(u64 occupied, u64 attacked, u32 rights, u64 checkers) {
+    const u32 occ = C == WHITE ? (u32)occupied : (u32)(occupied >> 56);
+    const u32 att = C == WHITE ? (u32)attacked : (u32)(attacked >> 56);
+    const u32 kside = (occ | att) >> 5;                   // f, g neither occupied nor attacked
+    const u32 qside = ((occ & 0x0E) | (att & 0x0C)) >> 1; // b, c, d not occupied, c, d not attacked
+    const u32 stop = ((kside | kside >> 1) & 1) | ((qside | qside >> 1 | qside >> 2) & 1) << 1;
+    return checkers ? 0u : rights & ~stop;
+}
+template <int C>
+PG_HD u32 castle_moves(const Sides &s, const MoveCtx &x) {
+    return castle_bits<C>(s.occ, x.threatened, s.castle, x.checkers);
 }
 
 // ---------------------------------------------------------------- count
-template <int C> PG_HD u32 count_moves_ks(const Pos &p, const Tables &t);
+// Knights per piece (pinned knights never move): one table lookup and
+// popcount each.
+struct KnightLoop {
+    PG_HD int operator()(u64 knights, u64 tgt, const Tables &t) const {
+        int n = 0;
+        for (u64 b = knights; b; b &= b - 1) n += popc(t.knight[ctz(b)] & tgt);
+        return n;
+    }
+};
 
-template <int C, int V>
-PG_HD u32 count_moves(const Pos &p, const Tables &t) {
-    if constexpr (V == SL_KOGGE) return count_moves_ks<C>(p, t);
+// n + the pawns' moves but en passant; pf, pw, pe: those that may push, take
+// westwards, take eastwards
+template <int C>
+PG_HD int pawn_moves(u64 pf, u64 pw, u64 pe, u64 empty, u64 enemy, u64 tgt, int n) {
+    // pushes on the low or high half only where the rank allows
+    const u64 PROMO = C == WHITE ? RANK8 : RANK1;
+    const u64 p1 = fwd<C>(pf) & empty;
+    const u64 p2 = fwd<C>(p1 & (C == WHITE ? RANK3 : RANK6)) & empty & tgt;
+    const u64 t1 = p1 & tgt;
+    n = popc_add(t1, popc_add(p2, n));
+    const u64 et = enemy & tgt;
+    const u64 cw = and3(C == WHITE ? shift<7>(pw) : shift<-9>(pw), ~FILEH, et);
+    const u64 ce = and3(C == WHITE ? shift<9>(pe) : shift<-7>(pe), ~FILEA, et);
+    n = popc_add(cw, popc_add(ce, n));
+    // a move to the last rank is four (one half of each word holds that rank)
+    return n + 3 * (popc(t1 & PROMO) + popc(cw & PROMO) + popc(ce & PROMO));
+}
+
+template <int C, class Knights> PG_HD u32 count_sides_ks(const Sides &s, const Tables &t, const Knights &knights);
+
+template <int C, int V, class Knights>
+PG_HD u32 count_sides(const Sides &s, const Tables &t, const Knights &knights) {
+    if constexpr (V == SL_KOGGE) return count_sides_ks<C>(s, t, knights);
     MoveCtx x;
-    prologue<C, V>(p, t, x);
-    const u64 tgt = x.target, empty = ~x.occ;
-    int n = popc(and_nor(t.king[x.k], x.mine, x.threatened));
+    prologue<C, V>(s, t, x);
+    const u64 tgt = x.target, empty = ~s.occ;
+    int n = popc(and_nor(t.king[s.k], s.mine, x.threatened));
     if (tgt == 0) return n;  // double check: king moves only
 
     // movers; a pinned piece moves only along its pin line
-    u64 pf = x.myPawns, pw = x.myPawns, pe = x.myPawns, myN = p.knights & x.mine;
+    u64 pf = s.myPawns, pw = s.myPawns, pe = s.myPawns, myN = s.myKnights;
     if (x.pinned) {
-        const u64 np = ~x.pinned, dk = diag_of(x.k), ak = anti_of(x.k);
-        pf = and_or(x.myPawns, np, file_of(x.k));
-        pw = and_or(x.myPawns, np, C == WHITE ? ak : dk);
-        pe = and_or(x.myPawns, np, C == WHITE ? dk : ak);
+        const u64 np = ~x.pinned;
+        const KingRow &row = t.row[s.k];
+        pf = and_or(s.myPawns, np, row.file);
+        pw = and_or(s.myPawns, np, C == WHITE ? row.anti : row.diag);
+        pe = and_or(s.myPawns, np, C == WHITE ? row.diag : row.anti);
         myN = andn(myN, x.pinned);
     }
 
@@ -463,29 +628,29 @@ PG_HD u32 count_moves(const Pos &p, const Tables &t) {
     const u64 p2 = fwd<C>(p1 & (C == WHITE ? RANK3 : RANK6)) & empty & tgt;
     const u64 t1 = p1 & tgt;
     n += popc(t1) + 3 * popc(t1 & PROMO) + popc(p2);
-    const u64 et = x.enemy & tgt;
+    const u64 et = s.enemy & tgt;
     const u64 cw = and3(C == WHITE ? shift<7>(pw) : shift<-9>(pw), ~FILEH, et);
     const u64 ce = and3(C == WHITE ? shift<9>(pe) : shift<-7>(pe), ~FILEA, et);
     n += popc(cw) + 3 * popc(cw & PROMO) + popc(ce) + 3 * popc(ce & PROMO);
 
-    // knights (pinned knights never move)
-    for (u64 b = myN; b; b &= b - 1) n += popc(t.knight[ctz(b)] & tgt);
+    n += knights(myN, tgt, t);
 
     // sliders, per piece
-    for (u64 b = p.bishopQueens & x.mine; b; b &= b - 1) {
-        const int s = ctz(b);
-        u64 m = Sl<V>::bishop(t, s, x.occ) & tgt;
-        if (x.pinned & bit(s)) m &= t.line[(s << 6) | x.k];
+    for (u64 b = s.myBishops; b; b &= b - 1) {
+        const int q = ctz(b);
+        u64 m = Sl<V>::bishop(t, q, s.occ) & tgt;
+        if (x.pinned & bit(q)) m &= t.line[(q << 6) | s.k];
         n += popc(m);
     }
-    for (u64 r = p.rookQueens & x.mine; r; r &= r - 1) {
-        const int s = ctz(r);
-        u64 m = Sl<V>::rook(t, s, x.occ) & tgt;
-        if (x.pinned & bit(s)) m &= t.line[(s << 6) | x.k];
+    for (u64 r = s.myRooks; r; r &= r - 1) {
+        const int q = ctz(r);
+        u64 m = Sl<V>::rook(t, q, s.occ) & tgt;
+        if (x.pinned & bit(q)) m &= t.line[(q << 6) | s.k];
         n += popc(m);
     }
-    n += castle_count<C>(p, x);
-    n += ep_moves<C>(p, t, x, nullptr);
+    n += popc((u64)castle_moves<C>(s, x));
+    NoSink none;
+    n += ep_moves<C>(s, t, x, none);
     return (u32)n;
 }
 
@@ -503,214 +668,588 @@ PG_HD u32 count_moves(const Pos &p, const Tables &t) {
 //    to its first blocker are o ^ (o - 2s) = e ^ (e + 2s); west rays the
 //    same on the bit-reversed board;
 //  * pinned pieces need the king-line masks only when something is pinned.
-template <int C>
-PG_HD u32 count_moves_ks(const Pos &p, const Tables &t) {
+template <int C, class Knights>
+PG_HD u32 count_sides_ks(const Sides &s, const Tables &t, const Knights &knights) {
     MoveCtx x;
-    const u64 W = p.white;
-    const u64 pawns = pos_pawns(p);
-    x.occ = or3(p.kings, pawns, or3(p.knights, p.bishopQueens, p.rookQueens));
-    x.mine = C == WHITE ? W : andn(x.occ, W);
-    x.enemy = C == WHITE ? andn(x.occ, W) : W;
-    x.myPawns = side_of<C>(pawns, W);
-    x.myKing = side_of<C>(p.kings, W);
-    x.k = ctz(x.myKing) & 63;
-    const int k = x.k;
-    const u64 eP = side_of<1 - C>(pawns, W), eN = side_of<1 - C>(p.knights, W);
-    const u64 eB = side_of<1 - C>(p.bishopQueens, W), eR = side_of<1 - C>(p.rookQueens, W);
-    x.eRooks = eR;
-
-    // sliders on a king line: no blocker -> checker, one blocker -> pinned
-    u64 cand = or_and(t.rookEmpty[k] & eR, t.bishopEmpty[k], eB);
-    u64 pinned = 0, chk = 0, behind = 0;
-    for (; cand; cand &= cand - 1) {
-        const int s = ctz(cand);
-        const u64 btw = t.between[(k << 6) | s];
-        const u64 b = btw & x.occ;
-        if (b == 0) {
-            chk |= bit(s);
-            behind |= and_nor(t.line[(s << 6) | k] & t.king[k], btw, bit(s));
-        } else if (!several(b)) {
-            pinned |= b;
-        }
-    }
-    {   // pawn and knight checks
-        const u64 kw = C == WHITE ? shift<7>(x.myKing) : shift<-9>(x.myKing);
-        const u64 ke = C == WHITE ? shift<9>(x.myKing) : shift<-7>(x.myKing);
-        chk = or_and(or_and(chk, or_and(andn(kw, FILEH), ke, ~FILEA), eP), t.knight[k], eN);
-    }
-    x.pinned = pinned & x.mine;
-    x.checkers = chk;
-    u64 tgt = ~x.mine;
-    if (chk) tgt &= several(chk) ? 0ULL : (chk | t.between[(k << 6) | ctz(chk)]);
-    x.target = tgt;
+    const KingRow &row = t.row[s.k];
+    const u64 eB = s.eBishops, eR = s.eRooks;
+    const u64 behind = pins_and_checks<C>(s, t, x);
+    const u64 tgt = x.target;
 
     // movers; a pinned piece moves only along its pin line
-    const u64 rq = side_of<C>(p.rookQueens, W), bq = side_of<C>(p.bishopQueens, W);
-    u64 rf = rq, rr = rq, bd = bq, ba = bq, pf = x.myPawns, pw = x.myPawns, pe = x.myPawns;
-    u64 myN = side_of<C>(p.knights, W);
+    const u64 rq = s.myRooks, bq = s.myBishops;
+    u64 rf = rq, rr = rq, bd = bq, ba = bq, pf = s.myPawns, pw = s.myPawns, pe = s.myPawns;
+    u64 myN = s.myKnights;
     if (x.pinned) {
         const u64 np = ~x.pinned;
-        const u64 fk = file_of(k), dk = diag_of(k), ak = anti_of(k);
-        rf = and_or(rq, np, fk);
-        rr = and_or(rq, np, rank_of(k));
-        bd = and_or(bq, np, dk);
-        ba = and_or(bq, np, ak);
-        pf = and_or(x.myPawns, np, fk);
-        pw = and_or(x.myPawns, np, C == WHITE ? ak : dk);
-        pe = and_or(x.myPawns, np, C == WHITE ? dk : ak);
+        rf = and_or(rq, np, row.file);
+        rr = and_or(rq, np, row.rank);
+        bd = and_or(bq, np, row.diag);
+        ba = and_or(bq, np, row.anti);
+        pf = and_or(s.myPawns, np, row.file);
+        pw = and_or(s.myPawns, np, C == WHITE ? row.anti : row.diag);
+        pe = and_or(s.myPawns, np, C == WHITE ? row.diag : row.anti);
         myN = andn(myN, x.pinned);
     }
 
     // enemy attacks without sliders: king, pawns, knights
-    const u64 eK = side_of<1 - C>(p.kings, W);
-    u64 att;
-    {
-        const u64 pw_ = C == WHITE ? shift<-9>(eP) : shift<7>(eP), pe_ = C == WHITE ? shift<-7>(eP) : shift<9>(eP);
-        att = or3(t.king[ctz(eK) & 63], or_and(andn(pw_, FILEH), pe_, ~FILEA), behind);
-        const u64 h1 = or_and(andn(shift<-1>(eN), FILEH), shift<1>(eN), ~FILEA);
-        const u64 h2 = or_and(andn(shift<-2>(eN), FILEG | FILEH), shift<2>(eN), ~(FILEA | FILEB));
-        att = or3(att, shift<16>(h1), shift<-16>(h1));
-        att = or3(att, shift<8>(h2), shift<-8>(h2));
-    }
+    u64 att = leaper_attacks<C>(s, t) | behind;
 
-    const u64 empty = ~x.occ;
+    const u64 empty = ~s.occ;
     int n = 0;
     {   // north and south
         const Prop3 pn = props<8>(empty), ps = props<-8>(empty);
         const u64 an = grow<8>(eR, pn), as = grow<-8>(eR, ps);
         att = or3(att, shift<8>(an), shift<-8>(as));
-        n += popc((grow<8>(rf, pn) << 8) & tgt);
-        n += popc((grow<-8>(rf, ps) >> 8) & tgt);
+        n = popc_add((grow<8>(rf, pn) << 8) & tgt, n);
+        n = popc_add((grow<-8>(rf, ps) >> 8) & tgt, n);
     }
-    const u64 eA = nor2(x.occ, FILEA), eH = nor2(x.occ, FILEH);
+    const u64 eA = nor2(s.occ, FILEA), eH = nor2(s.occ, FILEH);
     {   // east: one add per side
         att = or_xor(att, eH, east_sum(eR, eH));
-        n += popc(xor_and(eH, east_sum(rr, eH), tgt));
+        n = popc_add(xor_and(eH, east_sum(rr, eH), tgt), n);
     }
     {   // west: east on the bit-reversed board
         const u64 eoR = rev64(eA);
         att = or_xor(att, eA, rev64(east_sum(rev64(eR), eoR)));
-        n += popc(xor_and(eA, rev64(east_sum(rev64(rr), eoR)), tgt));
+        n = popc_add(xor_and(eA, rev64(east_sum(rev64(rr), eoR)), tgt), n);
     }
     {   // north-east and south-west
         const Prop3 pa = props<9>(eA), pb = props<-9>(eH);
         att = or_and(att, shift<9>(grow<9>(eB, pa)), ~FILEA);
         att = or_and(att, shift<-9>(grow<-9>(eB, pb)), ~FILEH);
-        n += popc(and3(shift<9>(grow<9>(bd, pa)), ~FILEA, tgt));
-        n += popc(and3(shift<-9>(grow<-9>(bd, pb)), ~FILEH, tgt));
+        n = popc_add(and3(shift<9>(grow<9>(bd, pa)), ~FILEA, tgt), n);
+        n = popc_add(and3(shift<-9>(grow<-9>(bd, pb)), ~FILEH, tgt), n);
     }
     {   // north-west and south-east
         const Prop3 pa = props<7>(eH), pb = props<-7>(eA);
         att = or_and(att, shift<7>(grow<7>(eB, pa)), ~FILEH);
         att = or_and(att, shift<-7>(grow<-7>(eB, pb)), ~FILEA);
-        n += popc(and3(shift<7>(grow<7>(ba, pa)), ~FILEH, tgt));
-        n += popc(and3(shift<-7>(grow<-7>(ba, pb)), ~FILEA, tgt));
+        n = popc_add(and3(shift<7>(grow<7>(ba, pa)), ~FILEH, tgt), n);
+        n = popc_add(and3(shift<-7>(grow<-7>(ba, pb)), ~FILEA, tgt), n);
     }
     x.threatened = att;
-    n += popc(and_nor(t.king[k], x.mine, att));
+    n = popc_add(and_nor(row.king, s.mine, att), n);
 
-    // pawns: pushes on the low or high half only where the rank allows
-    const u64 PROMO = C == WHITE ? RANK8 : RANK1;
-    const u64 p1 = fwd<C>(pf) & empty;
-    const u64 p2 = fwd<C>(p1 & (C == WHITE ? RANK3 : RANK6)) & empty & tgt;
-    const u64 t1 = p1 & tgt;
-    n += popc(t1) + 3 * popc(t1 & PROMO) + popc(p2);
-    const u64 et = x.enemy & tgt;
-    const u64 cw = and3(C == WHITE ? shift<7>(pw) : shift<-9>(pw), ~FILEH, et);
-    const u64 ce = and3(C == WHITE ? shift<9>(pe) : shift<-7>(pe), ~FILEA, et);
-    n += popc(cw) + 3 * popc(cw & PROMO) + popc(ce) + 3 * popc(ce & PROMO);
-    // knights
-    for (u64 b = myN; b; b &= b - 1) n += popc(t.knight[ctz(b)] & tgt);
-    n += castle_count<C>(p, x);
-    n += ep_moves<C>(p, t, x, nullptr);
+    n = pawn_moves<C>(pf, pw, pe, empty, s.enemy, tgt, n);
+    n += knights(myN, tgt, t);
+    n += popc((u64)castle_moves<C>(s, x));
+    NoSink none;
+    n += ep_moves<C>(s, t, x, none);
     return (u32)n;
 }
 
-// ---------------------------------------------------------------- generate
-PG_HD u16 mk_move(int from, int to, int flags) { return (u16)(from | (to << 6) | (flags << 12)); }
-
-// calls f(square) for every set square of m, low half then high half (a
-// 32-bit find-first-set and clear per square instead of the 64-bit ones)
-template <class F>
-PG_HD void each_square(u64 m, F &&f) {
-    for (u32 lo = (u32)m; lo; lo &= lo - 1) f(__builtin_ctz(lo));
-    for (u32 hi = (u32)(m >> 32); hi; hi &= hi - 1) f(32 + __builtin_ctz(hi));
+template <int C, int V>
+PG_HD u32 count_moves(const Pos &p, const Tables &t) {
+    return count_sides<C, V>(sides_of<C>(p), t, KnightLoop());
 }
 
-// Writes the legal moves of p to out (at most cap of them); returns the
-// number of legal moves (at most 218).
+// ---------------------------------------------------------------- generate
+PG_HD u32 mk_move(int from, int to, int flags) { return (u32)(from | (to << 6) | (flags << 12)); }
+
+// What the moves of a side follow from.  A move between two squares of the
+// quiet set of its piece (qP, qN, qB, qR; a queen's is qB & qR) is left out;
+// one between two squares of its calm set (zP, ...) is calm (see quiet
+// moves).  king, kingFull: the king's moves that are not quiet, not calm.
+struct Gen {
+    u64 pinned, checkers, target, king, kingFull;
+    u64 qP, qN, qB, qR, zP, zN, zB, zR;
+    u32 castle;
+};
+
+template <int C, int V>
+PG_HD Gen gen_all(const Sides &s, const Tables &t) {
+    MoveCtx x;
+    prologue<C, V>(s, t, x);
+    return Gen{x.pinned, x.checkers, x.target, and_nor(t.row[s.k].king, s.mine, x.threatened), 0, 0, 0, 0, 0, 0, 0, 0, 0,
+               castle_moves<C>(s, x)};
+}
+
+// Hands the legal moves of s that are not left out (at most 218) to the sink.
 // Pawn captures carry the capture flag; other captures do not, as on the
 // reference's device path (MoveGeneratorBitboard.h:2525-2529).
-template <int C, int V>
-PG_HD u32 generate_moves(const Pos &p, const Tables &t, u16 *out, u32 cap, u16 *tag = nullptr, u32 owner = 0) {
-    MoveCtx x;
-    prologue<C, V>(p, t, x);
-    const u64 tgt = x.target, empty = ~x.occ;
-    MoveSink o{out, cap, 0, tag, owner};
-    each_square(and_nor(t.king[x.k], x.mine, x.threatened),
-                [&](int to) { o.add(mk_move(x.k, to, MF_QUIET), P_KING); });
-    if (tgt == 0) return o.n;
+template <int C, int V, class Sink>
+PG_HD void generate_sides(const Sides &s, const Gen &g, const Tables &t, Sink &o) {
+    const u64 tgt = g.target, empty = ~s.occ;
+    o.squares(g.king, g.kingFull, M_KING, [&](int to) { return mk_move(s.k, to, MF_QUIET); });
+    if (tgt == 0) return;
 
     // a pinned pawn moves only along its pin line
-    u64 pf = x.myPawns, pw = x.myPawns, pe = x.myPawns;
-    if (x.pinned) {
-        const u64 np = ~x.pinned, dk = diag_of(x.k), ak = anti_of(x.k);
-        pf = and_or(x.myPawns, np, file_of(x.k));
-        pw = and_or(x.myPawns, np, C == WHITE ? ak : dk);
-        pe = and_or(x.myPawns, np, C == WHITE ? dk : ak);
+    u64 pf = s.myPawns, pw = s.myPawns, pe = s.myPawns;
+    if (g.pinned) {
+        const u64 np = ~g.pinned;
+        const KingRow &row = t.row[s.k];
+        pf = and_or(s.myPawns, np, row.file);
+        pw = and_or(s.myPawns, np, C == WHITE ? row.anti : row.diag);
+        pe = and_or(s.myPawns, np, C == WHITE ? row.diag : row.anti);
     }
     const int up = C == WHITE ? 8 : -8;
     const u64 PROMO = C == WHITE ? RANK8 : RANK1;
-    auto promos = [&](int from, int to, int cap) {
-        o.add(mk_move(from, to, MF_PROMO | cap | 0), P_PAWN);
-        o.add(mk_move(from, to, MF_PROMO | cap | 1), P_PAWN);
-        o.add(mk_move(from, to, MF_PROMO | cap | 3), P_PAWN);
-        o.add(mk_move(from, to, MF_PROMO | cap | 2), P_PAWN);
+    auto promos = [&](u64 m, int back, int cap) {
+        each_square(m, [&](int to) {
+            o.add(mk_move(to - back, to, MF_PROMO | cap | 0), M_PAWN | M_SPECIAL);
+            o.add(mk_move(to - back, to, MF_PROMO | cap | 1), M_PAWN | M_SPECIAL);
+            o.add(mk_move(to - back, to, MF_PROMO | cap | 3), M_PAWN | M_SPECIAL);
+            o.add(mk_move(to - back, to, MF_PROMO | cap | 2), M_PAWN | M_SPECIAL);
+        });
     };
     // pushes
     const u64 p1 = fwd<C>(pf) & empty;
     const u64 p2 = fwd<C>(p1 & (C == WHITE ? RANK3 : RANK6)) & empty & tgt;
-    each_square(andn(p1 & tgt, PROMO), [&](int to) { o.add(mk_move(to - up, to, MF_QUIET), P_PAWN); });
-    each_square(p1 & tgt & PROMO, [&](int to) { promos(to - up, to, 0); });
-    each_square(p2, [&](int to) { o.add(mk_move(to - 2 * up, to, MF_DOUBLE_PUSH), P_PAWN); });
+    const u64 t1 = p1 & tgt;
+    const u64 beside = (andn(s.ePawns, FILEH) << 1) | (andn(s.ePawns, FILEA) >> 1);
+    const u64 q1 = and3(andn(t1, PROMO), g.qP, fwd<C>(g.qP)), q2 = andn(and3(p2, g.qP, fwd<C>(fwd<C>(g.qP))), beside);
+    o.skipped(q1);
+    o.skipped(q2);
+    o.squares(and_nor(t1, PROMO, q1), ~(g.zP & fwd<C>(g.zP)), M_PAWN, [&](int to) { return mk_move(to - up, to, MF_QUIET); });
+    promos(t1 & PROMO, up, 0);
+    o.squares(and_nor(p2, q2, beside), ~(g.zP & fwd<C>(fwd<C>(g.zP))), M_PAWN,
+              [&](int to) { return mk_move(to - 2 * up, to, MF_DOUBLE_PUSH); });
+    o.squares(p2 & beside, ~0ULL, M_PAWN | M_SPECIAL, [&](int to) { return mk_move(to - 2 * up, to, MF_DOUBLE_PUSH); });
     // captures
-    const u64 et = x.enemy & tgt;
+    const u64 et = s.enemy & tgt;
     const u64 cw = and3(C == WHITE ? shift<7>(pw) : shift<-9>(pw), ~FILEH, et);
     const u64 ce = and3(C == WHITE ? shift<9>(pe) : shift<-7>(pe), ~FILEA, et);
     constexpr int dw = C == WHITE ? 7 : -9, de = C == WHITE ? 9 : -7;
-    each_square(andn(cw, PROMO), [&](int to) { o.add(mk_move(to - dw, to, MF_CAPTURE), P_PAWN); });
-    each_square(andn(ce, PROMO), [&](int to) { o.add(mk_move(to - de, to, MF_CAPTURE), P_PAWN); });
-    each_square(cw & PROMO, [&](int to) { promos(to - dw, to, MF_CAPTURE); });
-    each_square(ce & PROMO, [&](int to) { promos(to - de, to, MF_CAPTURE); });
-    ep_moves<C>(p, t, x, &o);
+    o.squares(andn(cw, PROMO), ~(g.zP & shift<dw>(g.zP)), M_PAWN, [&](int to) { return mk_move(to - dw, to, MF_CAPTURE); });
+    o.squares(andn(ce, PROMO), ~(g.zP & shift<de>(g.zP)), M_PAWN, [&](int to) { return mk_move(to - de, to, MF_CAPTURE); });
+    promos(cw & PROMO, dw, MF_CAPTURE);
+    promos(ce & PROMO, de, MF_CAPTURE);
+    MoveCtx x;
+    x.pinned = g.pinned;
+    x.checkers = g.checkers;
+    ep_moves<C>(s, t, x, o);
     // castling
-    if (!x.checkers) {
-        const int r = C == WHITE ? pos_wcastle(p) : pos_bcastle(p);
-        const int sh = C == WHITE ? 0 : 56;
-        if ((r & 1) && !((0x60ULL << sh) & (x.occ | x.threatened))) o.add(mk_move(4 + sh, 6 + sh, MF_KING_CASTLE), P_KING);
-        if ((r & 2) && !((0x0EULL << sh) & x.occ) && !((0x0CULL << sh) & x.threatened)) o.add(mk_move(4 + sh, 2 + sh, MF_QUEEN_CASTLE), P_KING);
-    }
+    constexpr int e = C == WHITE ? 4 : 60;
+    if (g.castle & 1) o.add(mk_move(e, e + 2, MF_KING_CASTLE), M_KING | M_SPECIAL);
+    if (g.castle & 2) o.add(mk_move(e, e - 2, MF_QUEEN_CASTLE), M_KING | M_SPECIAL);
+    // a piece on q with moves m, its quiet and calm sets
+    auto moves = [&](int q, u64 m, u64 quiet, u64 calm, u32 piece) {
+        const u64 left = and3(m, quiet, mask_if((quiet >> q) & 1));
+        o.skipped(left);
+        o.squares(andn(m, left), ~(calm & mask_if((calm >> q) & 1)), piece, [&](int to) { return mk_move(q, to, MF_QUIET); });
+    };
     // knights (pinned knights never move)
-    for (u64 b = andn(p.knights & x.mine, x.pinned); b; b &= b - 1) {
-        const int s = ctz(b);
-        each_square(t.knight[s] & tgt, [&](int to) { o.add(mk_move(s, to, MF_QUIET), P_KNIGHT); });
+    for (u64 b = andn(s.myKnights, g.pinned); b; b &= b - 1) {
+        const int q = ctz(b);
+        moves(q, t.knight[q] & tgt, g.qN, g.zN, M_KNIGHT);
     }
     // sliders
-    for (u64 b = p.bishopQueens & x.mine; b; b &= b - 1) {
-        const int s = ctz(b);
-        u64 m = Sl<V>::bishop(t, s, x.occ) & tgt;
-        if (x.pinned & bit(s)) m &= t.line[(s << 6) | x.k];
-        const int pc = (p.rookQueens & bit(s)) ? P_QUEEN : P_BISHOP;
-        each_square(m, [&](int to) { o.add(mk_move(s, to, MF_QUIET), pc); });
+    for (u64 b = s.myBishops; b; b &= b - 1) {
+        const int q = ctz(b);
+        u64 m = Sl<V>::bishop(t, q, s.occ) & tgt;
+        if (g.pinned & bit(q)) m &= t.line[(q << 6) | s.k];
+        const bool queen = s.myRooks & bit(q);
+        moves(q, m, queen ? g.qB & g.qR : g.qB, queen ? g.zB & g.zR : g.zB, queen ? M_QUEEN : M_BISHOP);
     }
-    for (u64 r = p.rookQueens & x.mine; r; r &= r - 1) {
-        const int s = ctz(r);
-        u64 m = Sl<V>::rook(t, s, x.occ) & tgt;
-        if (x.pinned & bit(s)) m &= t.line[(s << 6) | x.k];
-        const int pc = (p.bishopQueens & bit(s)) ? P_QUEEN : P_ROOK;
-        each_square(m, [&](int to) { o.add(mk_move(s, to, MF_QUIET), pc); });
+    for (u64 r = s.myRooks; r; r &= r - 1) {
+        const int q = ctz(r);
+        u64 m = Sl<V>::rook(t, q, s.occ) & tgt;
+        if (g.pinned & bit(q)) m &= t.line[(q << 6) | s.k];
+        const bool queen = s.myBishops & bit(q);
+        moves(q, m, queen ? g.qB & g.qR : g.qR, queen ? g.zB & g.zR : g.zR, queen ? M_QUEEN : M_ROOK);
     }
+}
+
+// Writes the legal moves of p to out (at most cap of them); returns the
+// number of legal moves.
+template <int C, int V>
+PG_HD u32 generate_moves(const Pos &p, const Tables &t, u16 *out, u32 cap) {
+    MoveSink o{out, cap, 0};
+    const Sides s = sides_of<C>(p);
+    generate_sides<C, V>(s, gen_all<C, V>(s, t), t, o);
     return o.n;
+}
+
+// ---------------------------------------------------------------- kin
+// A board as its children see it: the fused leaf keeps its boards in this
+// form in LDS.  Most of a child is its parent unchanged, so what would be
+// worked out for every child is worked out once: the piece words by side, the
+// kings' squares, and the attack sets of the first two knights of the side
+// that will reply.  A child then takes one xor or and-not per word instead of
+// a make-move on the combined words and the split by side after it.
+struct Kin {
+    u64 bP, bN, bB, bR;  // the replying side
+    u64 aP, aN, aB, aR;  // the side to move
+    u64 occ, mine;       // all men, the replying side's
+    u64 n0, n1;          // attacks of the first two of bN
+    u64 pinned;          // the replying side's pinned men if the other passes
+    u32 info;            // see KIN_*
+    u32 knights;         // squares of the first two of bN: 6 bits each; KIN_MORE: there are others; king and
+                         // castling moves if the other side passes << KIN_STAY
+};
+static_assert(sizeof(Kin) == 104 + 8, "a tile of 64 boards is 7 KB of its wave's LDS");
+// info: king squares (replying side, side to move), castling rights (replying
+// side, side to move), en-passant file + 1, side to move
+enum { KIN_EK = 6, KIN_CASTLE = 12, KIN_MYCASTLE = 14, KIN_EP = 16, KIN_SIDE = 20 };
+constexpr u32 KIN_MORE = 1u << 12;
+constexpr int KIN_STAY = 13;
+
+template <int A> PG_HD Kin kin_of(const Sides &s, const Tables &t) {
+    Kin k;
+    k.bP = s.ePawns;
+    k.bN = s.eKnights;
+    k.bB = s.eBishops;
+    k.bR = s.eRooks;
+    k.aP = s.myPawns;
+    k.aN = s.myKnights;
+    k.aB = s.myBishops;
+    k.aR = s.myRooks;
+    k.occ = s.occ;
+    k.mine = s.enemy;
+    k.n0 = k.n1 = k.pinned = 0;
+    k.knights = 0;
+    u64 n = k.bN;
+    if (n) {
+        const int q = ctz(n);
+        k.n0 = t.knight[q];
+        k.knights = (u32)q;
+        n &= n - 1;
+        if (n) {
+            const int r = ctz(n);
+            k.n1 = t.knight[r];
+            k.knights |= (u32)r << 6 | (several(n) ? KIN_MORE : 0u);
+        }
+    }
+    k.info = (u32)s.ek | (u32)s.k << KIN_EK | s.eCastle << KIN_CASTLE | s.castle << KIN_MYCASTLE | s.ep << KIN_EP |
+             (u32)A << KIN_SIDE;
+    return k;
+}
+
+// the board itself again, as the side to move sees it
+PG_HD Sides sides_of_kin(const Kin &k) {
+    Sides s;
+    s.occ = k.occ;
+    s.mine = andn(k.occ, k.mine);
+    s.enemy = k.mine;
+    s.myPawns = k.aP;
+    s.myKnights = k.aN;
+    s.myBishops = k.aB;
+    s.myRooks = k.aR;
+    s.ePawns = k.bP;
+    s.eKnights = k.bN;
+    s.eBishops = k.bB;
+    s.eRooks = k.bR;
+    s.ek = (int)(k.info & 63);
+    s.k = (int)(k.info >> KIN_EK & 63);
+    s.myKing = bit(s.k);
+    s.castle = k.info >> KIN_MYCASTLE & 3;
+    s.eCastle = k.info >> KIN_CASTLE & 3;
+    s.ep = k.info >> KIN_EP & 15;
+    return s;
+}
+
+// popcount of the knights' moves with the parent's attack sets of the first
+// two: a knight that was captured or is pinned is not in `knights`
+struct KinKnights {
+    const Kin &k;
+    PG_HD int operator()(u64 knights, u64 tgt, const Tables &t) const {
+        const int q = (int)(k.knights & 63), r = (int)(k.knights >> 6 & 63);
+        const u32 m0 = (u32)((int)((u32)(knights >> q) << 31) >> 31), m1 = (u32)((int)((u32)(knights >> r) << 31) >> 31);
+        int n = popc_add(and3(k.n0, tgt, (u64)m0 << 32 | m0), popc_add(and3(k.n1, tgt, (u64)m1 << 32 | m1), 0));
+        if (k.knights & KIN_MORE) n += KnightLoop()(and_nor(knights, bit(q), bit(r)), tgt, t);
+        return n;
+    }
+};
+
+// Number of legal replies (by side B) after the move of window word `w`, not
+// a special one, from the board k.
+template <int B, int V>
+PG_HD u32 count_child(const Kin &k, u32 w, const Tables &t) {
+    const int to = (int)(w >> 6 & 63);
+    const u64 src = bit((int)(w & 63)), dst = bit(to), both = src | dst;
+    // the moving piece's words change on both squares, its enemy's lose the target
+    const auto moved = [&](u64 x, int i) {
+        const u32 m = (u32)((int)(w << (7 - i)) >> 31);
+        return bop3<0x78>(x, both, (u64)m << 32 | m);  // x ^ (both & m)
+    };
+    Sides s;
+    s.ePawns = moved(k.aP, 0);
+    s.eKnights = moved(k.aN, 1);
+    s.eBishops = moved(k.aB, 2);
+    s.eRooks = moved(k.aR, 3);
+    s.myPawns = andn(k.bP, dst);
+    s.myKnights = andn(k.bN, dst);
+    s.myBishops = andn(k.bB, dst);
+    s.myRooks = andn(k.bR, dst);
+    s.occ = bop3<0xBA>(k.occ, src, dst);  // (occ & ~src) | dst
+    s.mine = andn(k.mine, dst);
+    s.enemy = andn(s.occ, s.mine);
+    s.k = (int)(k.info & 63);
+    s.myKing = bit(s.k);
+    s.ek = w >> 28 & 1 ? to : (int)(k.info >> KIN_EK & 63);
+    // a move to a corner takes that side's right, as make_move
+    const u32 edge = B == WHITE ? (u32)dst : (u32)(dst >> 56);
+    s.castle = k.info >> KIN_CASTLE & 3 & ~((edge >> 7 & 1) | (edge & 1) << 1);
+    s.eCastle = 0;
+    s.ep = 0;
+    return count_sides<B, V>(s, t, KinKnights{k});
+}
+
+// the board itself again (clock 0)
+PG_HD Pos pos_of_kin(const Kin &k) {
+    const u32 side = k.info >> KIN_SIDE & 1, mine = k.info >> KIN_MYCASTLE & 3, theirs = k.info >> KIN_CASTLE & 3;
+    Pos p;
+    p.white = side ? k.mine : andn(k.occ, k.mine);
+    p.pawns = k.aP | k.bP | (u64)(side ? theirs | mine << 2 : mine | theirs << 2) | (u64)side << 63;
+    p.knights = k.aN | k.bN;
+    p.bishopQueens = k.aB | k.bB;
+    p.rookQueens = k.aR | k.bR;
+    p.kings = bit((int)(k.info & 63)) | bit((int)(k.info >> KIN_EK & 63));
+    return p;
+}
+
+// ---------------------------------------------------------------- quiet moves
+// Most moves change little of what the other side could do.  Let side A be to
+// move, B not in check, and let the zone be B's king, the squares it could step
+// to, and those it would cross castling.
+//
+// A move of A from s to t that is not special (M_SPECIAL) is calm when neither
+// s nor t is
+//  * on an open line between a slider of A and a zone square, first blockers
+//    included, or on a line between a slider of A and B's king, whatever
+//    stands on it: then no other slider's view of the zone changes, nor a pin
+//    on a man of B;
+//  * one from which the moved piece itself reaches the zone: a pawn's, knight's
+//    or king's step from it; for a slider an open line, or the line of B's
+//    king (a pin);
+//  * between king and rook where B may still castle, or that rook's corner, or
+//    a man of B next to its king.
+// After it B is not in check, its pins are those it would have if A passed,
+// and so are its king's and castling moves: only its sliders, pawns and
+// knights need counting (count_calm).
+//
+// A calm move to an empty square is quiet when moreover neither s nor t is on
+// a ray of a slider of B (up to and including its first blocker), in front of
+// a pawn of B within its push, or on a square it attacks: then every man of B
+// has the moves it would have if A passed (a knight's do not depend on s and
+// t), so the replies to the quiet moves are their number times that count, and
+// the moves are not even listed.
+//
+// Of the moves of all positions four plies into the game 74% are quiet and 21%
+// calm; in random games 59 and 29% up to ply 19, 38 and 36% to ply 39, 30 and
+// 35% to ply 59, 25 to 30 and 15 to 31% later.
+struct LeafEval {
+    Gen g;
+    u32 calm, full, quiet;  // numbers of moves
+    u32 c0;                 // replies to each quiet move
+};
+
+// keeps the compiler from carrying what it loaded from LDS in registers past
+// this point (it is loaded again)
+PG_HD void reload() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#endif
+}
+
+// k: the board (kin_of); its pins and staying moves are filled in.
+template <int A>
+PG_HD LeafEval leaf_eval(Kin &k, const Tables &t) {
+    constexpr int B = 1 - A, sh = B == WHITE ? 0 : 56;
+    Sides s = sides_of_kin(k);
+    const KingRow &ra = t.row[s.k], &rb = t.row[s.ek];
+    const u64 e = ~s.occ, kb = bit(s.ek), aB = s.myBishops, aR = s.myRooks, bB = s.eBishops, bR = s.eRooks;
+    LeafEval r;
+    Gen &g = r.g;
+    MoveCtx x;
+    const u64 behind = pins_and_checks<A>(s, t, x);
+    const u64 tgtA = x.target, tgtB = ~s.enemy;
+
+    // B's pins and checks, the zone, and the squares that are not calm for any
+    // piece: on lines between B's king and sliders of A, ...
+    u64 zone = andn(rb.king, s.enemy) | kb, tied = rb.king & s.enemy, pinB = 0, chkB = 0;
+    if (s.eCastle & 1) {
+        zone |= 0x60ULL << sh;
+        tied |= 0xE0ULL << sh;
+    }
+    if (s.eCastle & 2) {
+        zone |= 0x0CULL << sh;
+        tied |= 0x0FULL << sh;
+    }
+    for (u64 c = or_and(rb.rook & aR, rb.bishop, aB); c; c &= c - 1) {
+        const int q = ctz(c);
+        const u64 btw = t.pin[(s.ek << 6) | q].between, on = btw & s.occ;
+        pinB = or_and(pinB, on, mask_if(!several(on)));
+        tied = or3(tied, btw, bit(q));
+        chkB = or_and(chkB, bit(q), mask_if(on == 0));
+    }
+    pinB &= s.enemy;
+    chkB = or_and(or_and(chkB, rb.knight, s.myKnights), pawn_att<B>(kb), s.myPawns);
+
+    // one pass over the directions, B's sliders, A's and the zone's view
+    // through the same propagators: the two sides' slider moves, the squares
+    // each attacks, the open lines between A and the zone, and where a slider
+    // of A would reach the zone from
+    const u64 pB = pawn_att<B>(s.ePawns);
+    u64 attA = or3(t.king[s.k], pawn_att<A>(s.myPawns), knight_att(s.myKnights));
+    u64 raysB = 0, zR = rb.rook, zB = rb.bishop;
+    int nA = 0, nB = 0;
+    const auto pair = [&](auto dir, const Prop3 &pu, const Prop3 &pd, u64 mu, u64 md, u64 a, u64 b, u64 &z) {
+        constexpr int S = decltype(dir)::value;
+        const u64 au = and_mask(shift<S>(grow<S>(a, pu)), mu), ad = and_mask(shift<-S>(grow<-S>(a, pd)), md);
+        const u64 zu = and_mask(shift<S>(grow<S>(zone, pu)), mu), zd = and_mask(shift<-S>(grow<-S>(zone, pd)), md);
+        const u64 bu = and_mask(shift<S>(grow<S>(b, pu)), mu), bd = and_mask(shift<-S>(grow<-S>(b, pd)), md);
+        nA = popc_add(au & tgtA, popc_add(ad & tgtA, nA));
+        nB = popc_add(bu & tgtB, popc_add(bd & tgtB, nB));
+        tied = or_and(or_and(tied, au, zd), ad, zu);
+        attA = or3(attA, au, ad);
+        raysB = or3(raysB, bu, bd);
+        z = or3(z, zu, zd);
+    };
+    const u64 eA = andn(e, FILEA), eH = andn(e, FILEH);
+    pair(Int<8>(), props<8>(e), props<-8>(e), ~0ULL, ~0ULL, aR, bR, zR);
+    pair(Int<1>(), props<1>(eA), props<-1>(eH), ~FILEA, ~FILEH, aR, bR, zR);
+    pair(Int<9>(), props<9>(eA), props<-9>(eH), ~FILEA, ~FILEH, aB, bB, zB);
+    pair(Int<7>(), props<7>(eH), props<-7>(eA), ~FILEH, ~FILEA, aB, bB, zB);
+    // pinned sliders were counted as if they could leave their line
+    const auto bound = [&](u64 pins, u64 bishops, u64 rooks, u64 tgt, int king) {
+        int n = 0;
+        for (u64 c = and_or(pins, bishops, rooks); c; c &= c - 1) {
+            const int q = ctz(c);
+            const u64 off = andn(tgt, t.line[(q << 6) | king]);
+            n = popc_add(and3(Sl<SL_KOGGE>::bishop(t, q, s.occ), off, mask_if((bishops >> q) & 1)), n);
+            n = popc_add(and3(Sl<SL_KOGGE>::rook(t, q, s.occ), off, mask_if((rooks >> q) & 1)), n);
+        }
+        return n;
+    };
+    if (x.pinned) nA -= bound(x.pinned, aB, aR, tgtA, s.k);
+    if (pinB) nB -= bound(pinB, bB, bR, tgtB, s.ek);
+
+    // B's moves if A passed
+    const u32 stay = (u32)popc(and_nor(rb.king, s.enemy, attA)) +
+                     (u32)popc((u64)castle_bits<B>(s.occ, attA, s.eCastle, 0));
+    {
+        u64 pf = s.ePawns, pw = pf, pe = pf;
+        if (pinB) {
+            const u64 np = ~pinB;
+            pf = and_or(pf, np, rb.file);
+            pw = and_or(pw, np, B == WHITE ? rb.anti : rb.diag);
+            pe = and_or(pe, np, B == WHITE ? rb.diag : rb.anti);
+        }
+        nB = pawn_moves<B>(pf, pw, pe, e, s.mine, tgtB, nB);
+    }
+    nB += KinKnights{k}(andn(s.eKnights, pinB), tgtB, t);
+    r.c0 = (u32)nB + stay;
+    k.pinned = pinB;
+    k.knights = (k.knights & (2 * KIN_MORE - 1)) | stay << KIN_STAY;
+    reload();
+    s = sides_of_kin(k);
+
+    // the calm and quiet sets
+    const u64 calm = andn(mask_if(chkB == 0), tied);
+    const u64 pawnHome = B == WHITE ? RANK1 << 8 : RANK8 >> 8;
+    const u64 push = fwd<B>(s.ePawns) | fwd<B>(fwd<B>(s.ePawns & pawnHome));
+    const u64 still = andn(~or3(raysB, push, pB), s.enemy);
+    g.zP = andn(calm, pawn_att<B>(zone));
+    g.zN = andn(calm, knight_att(zone));
+    g.zB = andn(calm, zB);
+    g.zR = andn(calm, zR);
+    g.qP = g.zP & still;
+    g.qN = g.zN & still;
+    g.qB = g.zB & still;
+    g.qR = g.zR & still;
+    const u64 zK = andn(calm, king_att(zone)), zKm = zK & mask_if((zK >> s.k) & 1);
+
+    // A's moves by kind
+    g.pinned = x.pinned;
+    g.checkers = x.checkers;
+    g.target = tgtA;
+    const u64 attB = or3(t.king[s.ek], pB, or3(knight_att(s.eKnights), behind, raysB));
+    const u64 kings = and_nor(ra.king, s.mine, attB);
+    const u64 kq = and3(kings, zKm, still & mask_if((still >> s.k) & 1));
+    g.king = andn(kings, kq);
+    g.kingFull = andn(kings, zKm);
+    g.castle = castle_bits<A>(s.occ, attB, s.castle, x.checkers);
+    int all = nA + popc(kings) + popc((u64)g.castle), quiet = popc(kq), notFull = popc(kings & zKm);  // notFull: calm or quiet
+    if (tgtA) {
+        u64 pf = s.myPawns, pw = pf, pe = pf;
+        if (x.pinned) {
+            const u64 np = ~x.pinned;
+            pf = and_or(pf, np, ra.file);
+            pw = and_or(pw, np, A == WHITE ? ra.anti : ra.diag);
+            pe = and_or(pe, np, A == WHITE ? ra.diag : ra.anti);
+        }
+        const u64 PROMO = A == WHITE ? RANK8 : RANK1;
+        const u64 beside = (andn(s.ePawns, FILEH) << 1) | (andn(s.ePawns, FILEA) >> 1);
+        const u64 p1 = fwd<A>(pf) & e, p2 = fwd<A>(p1 & (A == WHITE ? RANK3 : RANK6)) & e & tgtA;
+        const u64 t1 = p1 & tgtA, s1 = andn(t1, PROMO), s2 = andn(p2, beside);
+        const u64 et = s.enemy & tgtA;
+        constexpr int dw = A == WHITE ? 7 : -9, de = A == WHITE ? 9 : -7;
+        const u64 cw = and3(shift<dw>(pw), ~FILEH, et), ce = and3(shift<de>(pe), ~FILEA, et);
+        all = popc_add(t1, popc_add(p2, popc_add(cw, popc_add(ce, all))));
+        all += 3 * (popc(t1 & PROMO) + popc(cw & PROMO) + popc(ce & PROMO));
+        const u64 z1 = fwd<A>(g.zP), z2 = fwd<A>(z1), q1 = fwd<A>(g.qP), q2 = fwd<A>(q1);
+        notFull = popc_add(and3(s1, g.zP, z1), popc_add(and3(s2, g.zP, z2), notFull));
+        quiet = popc_add(and3(s1, g.qP, q1), popc_add(and3(s2, g.qP, q2), quiet));
+        notFull = popc_add(and3(andn(cw, PROMO), g.zP, shift<dw>(g.zP)), notFull);
+        notFull = popc_add(and3(andn(ce, PROMO), g.zP, shift<de>(g.zP)), notFull);
+        NoSink none;
+        all += ep_moves<A>(s, t, x, none);
+        const auto kinds = [&](int q, u64 m, u64 zs, u64 qs) {
+            notFull = popc_add(and3(m, zs, mask_if((zs >> q) & 1)), notFull);
+            quiet = popc_add(and3(m, qs, mask_if((qs >> q) & 1)), quiet);
+        };
+        for (u64 b = andn(s.myKnights, x.pinned); b; b &= b - 1) {
+            const int q = ctz(b);
+            const u64 m = t.knight[q] & tgtA;
+            all = popc_add(m, all);
+            kinds(q, m, g.zN, g.qN);
+        }
+        const u64 queens = aB & aR;
+        for (u64 b = and_or(aB & g.zB, ~queens, g.zR); b; b &= b - 1) {
+            const int q = ctz(b);
+            const u64 nq = mask_if(!((queens >> q) & 1));
+            u64 m = Sl<SL_KOGGE>::bishop(t, q, s.occ) & tgtA;
+            if (x.pinned & bit(q)) m &= t.line[(q << 6) | s.k];
+            kinds(q, m, and_or(g.zB, nq, g.zR), and_or(g.qB, nq, g.qR));
+        }
+        for (u64 b = and_or(aR & g.zR, ~queens, g.zB); b; b &= b - 1) {
+            const int q = ctz(b);
+            const u64 nq = mask_if(!((queens >> q) & 1));
+            u64 m = Sl<SL_KOGGE>::rook(t, q, s.occ) & tgtA;
+            if (x.pinned & bit(q)) m &= t.line[(q << 6) | s.k];
+            kinds(q, m, and_or(g.zR, nq, g.zB), and_or(g.qR, nq, g.qB));
+        }
+    }
+    r.quiet = (u32)quiet;
+    r.calm = (u32)(notFull - quiet);
+    r.full = (u32)(all - notFull);
+    return r;
+}
+
+// Number of replies (by side B) after the calm move of window word `w`.
+template <int B>
+PG_HD u32 count_calm(const Kin &k, u32 w, const Tables &t) {
+    const u64 src = bit((int)(w & 63)), dst = bit((int)(w >> 6 & 63));
+    const u64 occ = bop3<0xBA>(k.occ, src, dst), mine = andn(k.mine, dst);  // (occ & ~src) | dst
+    const u64 tgt = ~mine, empty = ~occ;
+    const u64 bq = andn(k.bB, dst), rq = andn(k.bR, dst);
+    u64 rf = rq, rr = rq, bd = bq, ba = bq, pf = andn(k.bP, dst), pw = pf, pe = pf, kn = andn(k.bN, dst);
+    if (k.pinned) {
+        const KingRow &row = t.row[k.info & 63];
+        const u64 np = ~k.pinned;
+        rf = and_or(rq, np, row.file);
+        rr = and_or(rq, np, row.rank);
+        bd = and_or(bq, np, row.diag);
+        ba = and_or(bq, np, row.anti);
+        pw = and_or(pf, np, B == WHITE ? row.anti : row.diag);
+        pe = and_or(pf, np, B == WHITE ? row.diag : row.anti);
+        pf = and_or(pf, np, row.file);
+        kn &= np;
+    }
+    int n = (int)(k.knights >> KIN_STAY);
+    n = popc_add((grow<8>(rf, props<8>(empty)) << 8) & tgt, n);
+    n = popc_add((grow<-8>(rf, props<-8>(empty)) >> 8) & tgt, n);
+    const u64 eA = nor2(occ, FILEA), eH = nor2(occ, FILEH);
+    n = popc_add(xor_and(eH, east_sum(rr, eH), tgt), n);
+    n = popc_add(xor_and(eA, rev64(east_sum(rev64(rr), rev64(eA))), tgt), n);
+    n = popc_add(and3(shift<9>(grow<9>(bd, props<9>(eA))), ~FILEA, tgt), n);
+    n = popc_add(and3(shift<-9>(grow<-9>(bd, props<-9>(eH))), ~FILEH, tgt), n);
+    n = popc_add(and3(shift<7>(grow<7>(ba, props<7>(eH))), ~FILEH, tgt), n);
+    n = popc_add(and3(shift<-7>(grow<-7>(ba, props<-7>(eA))), ~FILEA, tgt), n);
+    n = pawn_moves<B>(pf, pw, pe, empty, andn(occ, mine), tgt, n);
+    return (u32)(n + KinKnights{k}(kn, tgt, t));
 }
 
 // ---------------------------------------------------------------- make move
@@ -852,9 +1391,53 @@ PG_HD u32 count_any(const Pos &p, const Tables &t) {
     return pos_side(p) ? count_moves<BLACK, V>(p, t) : count_moves<WHITE, V>(p, t);
 }
 template <int V>
-PG_HD u32 generate_any(const Pos &p, const Tables &t, u16 *out, u32 cap = 256, u16 *tag = nullptr, u32 owner = 0) {
-    return pos_side(p) ? generate_moves<BLACK, V>(p, t, out, cap, tag, owner)
-                       : generate_moves<WHITE, V>(p, t, out, cap, tag, owner);
+PG_HD u32 generate_any(const Pos &p, const Tables &t, u16 *out, u32 cap = 256) {
+    return pos_side(p) ? generate_moves<BLACK, V>(p, t, out, cap) : generate_moves<WHITE, V>(p, t, out, cap);
+}
+// the same into window words (WordSink)
+template <int V>
+PG_HD u32 generate_words(const Pos &p, const Tables &t, u32 *out, u32 cap, u32 owner) {
+    WordSink o{out, cap, 0, owner};
+    if (pos_side(p)) {
+        const Sides s = sides_of<BLACK>(p);
+        generate_sides<BLACK, V>(s, gen_all<BLACK, V>(s, t), t, o);
+    } else {
+        const Sides s = sides_of<WHITE>(p);
+        generate_sides<WHITE, V>(s, gen_all<WHITE, V>(s, t), t, o);
+    }
+    return o.n;
+}
+// the moves of k that are not quiet
+template <int V>
+PG_HD void generate_leaf(const Kin &k, const Gen &g, const Tables &t, LeafSink &o) {
+    const Sides s = sides_of_kin(k);
+    if (k.info >> KIN_SIDE & 1) generate_sides<BLACK, V>(s, g, t, o);
+    else generate_sides<WHITE, V>(s, g, t, o);
+}
+template <int V>
+PG_HD u32 count_child_any(const Kin &k, u32 w, const Tables &t) {
+    return k.info >> KIN_SIDE & 1 ? count_child<WHITE, V>(k, w, t) : count_child<BLACK, V>(k, w, t);
+}
+// the same for any move, by making it
+template <int V>
+PG_HD u32 count_made(const Kin &k, u32 w, const Tables &t) {
+    Pos p = pos_of_kin(k);
+    const int piece = piece_code(w >> 24);
+    if (pos_side(p)) {
+        make_move_as<BLACK, false>(p, (u16)w, piece, nullptr, t);
+        return count_moves<WHITE, V>(p, t);
+    }
+    make_move_as<WHITE, false>(p, (u16)w, piece, nullptr, t);
+    return count_moves<BLACK, V>(p, t);
+}
+PG_HD u32 count_calm_any(const Kin &k, u32 w, const Tables &t) {
+    return k.info >> KIN_SIDE & 1 ? count_calm<WHITE>(k, w, t) : count_calm<BLACK>(k, w, t);
+}
+PG_HD Kin kin_any(const Pos &p, const Tables &t) {
+    return pos_side(p) ? kin_of<BLACK>(sides_of<BLACK>(p), t) : kin_of<WHITE>(sides_of<WHITE>(p), t);
+}
+PG_HD LeafEval leaf_any(Kin &k, const Tables &t) {
+    return k.info >> KIN_SIDE & 1 ? leaf_eval<BLACK>(k, t) : leaf_eval<WHITE>(k, t);
 }
 PG_HD void make_any(Pos &p, u16 mv, const Tables &t) {
     if (pos_side(p)) make_move<BLACK, false>(p, mv, nullptr, t);

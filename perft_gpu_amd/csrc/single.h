@@ -125,27 +125,17 @@ PG_HD u64 s_node_cap(const SRegion &r) {
 }
 
 // ---------------------------------------------------------------- tiles
-// A work-group's boards and the moves they generate (the fused leaf's window;
-// 40 KB, so that four work-groups share a CU's LDS).
-constexpr int S_CAP = 6800;
-struct STile {
-    Pos b[LEAF_WG];
-    u16 mv[S_CAP];
-    u16 tag[S_CAP];  // owner | moving piece << 8
-    u32 per[LEAF_WG];
-    u32 next;
-    u64 base;
-};
-
-// Boards per tile.  Whole waves of boards keep the lanes of the tile's
-// expansion full; a level of too few boards for that on every CU is dealt out
-// 8 boards or more at a time, for the time of its longest tile.  (The fused
-// leaf of a depth-5 search, 2e4 boards: 84 us in tiles of 256, 47 us so.)
-constexpr u32 S_RESIDENT = 1024;  // work-groups the chip holds (four per CU)
-__device__ __forceinline__ u32 s_tile_boards(u64 n) {
-    if (n < 64 * S_RESIDENT) return n < 8 * S_RESIDENT ? 8u : (u32)((n + S_RESIDENT - 1) / S_RESIDENT);
-    const u64 t = n / (8 * S_RESIDENT) / 64 * 64;
-    return t < 64 ? 64u : t > LEAF_WG ? (u32)LEAF_WG : (u32)t;
+// a value that all lanes hold, in scalar registers
+__device__ __forceinline__ u64 uniform64(u64 v) {
+    return (u64)(u32)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (u32)__builtin_amdgcn_readfirstlane((int)v);
+}
+// Boards per tile of the leaf (a wave each) and of the level kernel (a
+// work-group each): a level of too few boards for whole tiles on every CU is
+// dealt out a few at a time, for the time of its longest tile.
+constexpr u32 S_RESIDENT = 1024;  // work-groups of the level kernel the chip holds (four per CU)
+__device__ __forceinline__ u32 s_tile_boards(u64 n, u32 tiles, u32 least, u32 most) {
+    const u64 t = (n + tiles - 1) / tiles;
+    return t < least ? least : t > most ? most : (u32)t;
 }
 
 // *acc += the work-group's sum of s, one atomic; sums may need all 64 bits,
@@ -177,99 +167,96 @@ __device__ __forceinline__ void s_mad(u64 *s, u64 w, u64 c, bool *carry) {
     *carry |= __umul64hi(w, c) != 0 || *s < v;
 }
 
-// The moves of the tile's boards (lane tid: s.b[tid] with c legal moves, 0 for
-// an idle lane), a window at a time: f(first, last, start) handles the listed
-// moves first..last, of which slot j - start holds number j.
-template <int V, class F>
-__device__ __forceinline__ u32 s_windows(STile &s, u32 c, u32 *err, const Tables &t, F &&f, u32 pos, u32 total) {
-    const int tid = threadIdx.x;
-    u32 start = 0;
-    while (start < total) {
-        const u32 end = start + S_CAP;
-        if (tid == 0) s.next = total;
-        __syncthreads();
-        if (c && pos >= start && pos + c <= end) {
-            const u32 g = generate_any<V>(s.b[tid], t, s.mv + (pos - start), c, s.tag + (pos - start), (u32)tid);
-            if (g != c) atomicOr(err, 2u);
-        } else if (c && pos >= start) {
-            atomicMin(&s.next, pos);
-        }
-        __syncthreads();
-        const u32 wend = s.next;
-        f(start, wend);
-        __syncthreads();
-        start = wend;
-    }
-    return total;
-}
-
 struct SSum {
     u64 total = 0, items = 0, paths = 0;
     bool carry = false, wide = false;
 };
 
-// perft(2) of the tile's boards times their weights
+// perft(2) of the wave's boards, each counted once
 template <int V>
-__device__ __forceinline__ void s_leaf_tile(STile &s, bool live, const Pos &b, u64 w, SSum &sum, u32 *err,
-                                            const Tables &t) {
-    const int tid = threadIdx.x;
-    u32 c = 0;
+__device__ __forceinline__ void s_leaf_tile(LeafTile &s, bool live, const Pos &b, SSum &sum, u32 *err, const Tables &t) {
+    const u32 c = leaf_expand<V>(s, live, b, err, t);
     if (live) {
-        c = count_any<V>(b, t);
-        s.b[tid] = b;
-    }
-    s.per[tid] = 0;
-    u64 total;
-    const u32 pos = (u32)block_excl_scan<LEAF_WG>(c, &total);
-    s_windows<V>(
-        s, c, err, t,
-        [&](u32 start, u32 wend) {
-            for (u32 j = start + tid; j < wend; j += LEAF_WG) {
-                const u32 tg = s.tag[j - start];
-                const u32 o = tg & 255;
-                atomicAdd(&s.per[o], count_after_as<V>(s.b[o], s.mv[j - start], (int)(tg >> 8), t));
-            }
-        },
-        pos, (u32)total);
-    if (live) {
-        s_mad(&sum.total, w, s.per[tid], &sum.carry);
-        s_mad(&sum.paths, w, c, &sum.wide);
+        sum.total += s.per[threadIdx.x & 63];
+        sum.paths += c;
         sum.items += c;
     }
-    __syncthreads();
 }
 
-// the tile's moves into the list of the next ply; node = the first board's
-// place.  False when the list is full.
+// the wave's sum of v, in scalar registers
+__device__ __forceinline__ u32 wave_sum32(u32 v) {
+    u32 x = v;
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);  // row_shr 1, 2, 4, 8
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);
+    return (u32)(__builtin_amdgcn_readlane((int)x, 15) + __builtin_amdgcn_readlane((int)x, 31) +
+                 __builtin_amdgcn_readlane((int)x, 47) + __builtin_amdgcn_readlane((int)x, 63));
+}
+// *s += the wave's sum of w * c, all in scalar registers: the leaf leaves no
+// vector register for a lane's sums.  *wide: the sum passed 64 bits.
+__device__ __forceinline__ void s_wave_mad(u64 *s, u64 w, u32 c, bool *wide) {
+    const u64 v = w * c;
+    u64 lo, hi = 0;
+    if (__ballot(v >> 26) == 0 && __ballot(w >> 32) == 0) {
+        lo = wave_sum32((u32)v);
+    } else {
+        lo = uniform64(wave_sum((w & 0xFFFFFFFFULL) * c));
+        hi = uniform64(wave_sum((w >> 32) * c));
+        hi += lo >> 32;
+        lo = hi << 32 | (lo & 0xFFFFFFFFULL);
+    }
+    *s += lo;
+    *wide |= hi >> 32 != 0 || *s < lo;
+}
+
+// The moves of a work-group's boards (this lane: board b when live, of weight
+// w) into the list of the next ply; node = the first board's place.  They are
+// staged in LDS so that the list is written by consecutive lanes, a window at
+// a time; a list that is full raises overflow.
+constexpr int S_CAP = 6912;
+struct ListTile {
+    Pos b[LEAF_WG];
+    u32 word[S_CAP];
+    u32 next;
+    u64 base;
+};
 template <int V>
-__device__ __forceinline__ void s_list_tile(STile &s, bool live, const Pos &b, u64 w, u32 node, u64 *counter,
+__device__ __forceinline__ void s_list_tile(ListTile &s, bool live, const Pos &b, u64 w, u32 node, u64 *counter,
                                             const SLevel &L, SPlan *P, SSum &sum, const Tables &t) {
-    const int tid = threadIdx.x;
     u32 c = 0;
     if (live) {
+        s.b[threadIdx.x] = b;
         c = count_any<V>(b, t);
-        s.b[tid] = b;
         s_mad(&sum.paths, w, c, &sum.wide);
     }
     u64 total64;
     const u32 pos = (u32)block_excl_scan<LEAF_WG>(c, &total64);
-    if (tid == 0) {
+    const u32 total = (u32)total64;
+    if (threadIdx.x == 0) {
         s.base = atomicAdd(counter, total64);
-        if (s.base + total64 > L.cap) P->overflow = 1;
+        if (s.base + total > L.cap) P->overflow = 1;
     }
     __syncthreads();
     const u64 base = s.base;
-    if (base + total64 <= L.cap)
-        s_windows<V>(
-            s, c, &P->err, t,
-            [&](u32 start, u32 wend) {
-                for (u32 j = start + tid; j < wend; j += LEAF_WG) {
-                    const u32 tg = s.tag[j - start];
-                    L.mv[base + j] = s.mv[j - start];
-                    L.par[base + j] = (node + (tg & 255)) | (tg >> 8) << S_NODE_BITS;
-                }
-            },
-            pos, (u32)total64);
+    for (u32 start = 0; base + total <= L.cap && start < total;) {
+        if (threadIdx.x == 0) s.next = total;
+        __syncthreads();
+        if (c && pos >= start && pos + c <= start + S_CAP) {
+            if (generate_words<V>(s.b[threadIdx.x], t, s.word + (pos - start), c, threadIdx.x) != c) P->err = 2;
+        } else if (c && pos >= start) {
+            atomicMin(&s.next, pos);
+        }
+        __syncthreads();
+        const u32 end = s.next;
+        for (u32 j = start + threadIdx.x; j < end; j += LEAF_WG) {
+            const u32 m = s.word[j - start];
+            L.mv[base + j] = (u16)m;
+            L.par[base + j] = (node + (m >> 16 & 255)) | (u32)piece_code(m >> 24) << S_NODE_BITS;
+        }
+        __syncthreads();
+        start = end;
+    }
     __syncthreads();
 }
 
@@ -331,8 +318,6 @@ __device__ __forceinline__ void s_finish(SPlan *P, const SSum &sum, int depth, u
     __hip_atomic_store(&out->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-#define S_LEAF_BOUNDS(V) __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu((V) == SL_KOGGE ? 4 : 5, 8)))
-
 // ---------------------------------------------------------------- kernels
 // perft(1) and perft(2): one work-group
 template <int V>
@@ -342,80 +327,90 @@ __global__ __launch_bounds__(LEAF_WG) void ks_one(SRoot r, SPlan *P, int depth, 
     if (depth == 1) {
         if (tid == 0) sum.total = sum.paths = count_any<V>(r.b, t);
     } else if (tid < r.n) {
-        sum.total = count_after_as<V>(r.b, r.mv[tid], r.piece[tid], t);
+        sum.total = count_any<V>(s_made(r.b, r.mv[tid], r.piece[tid], t), t);
         sum.items = sum.paths = 1;
     }
     s_finish(P, sum, depth, bias, out, seq);
 }
 
-// perft(3): the fused leaf over the root's children, 8 per work-group, so
-// that each work-group's children's moves are one pass of its lanes
-constexpr int S_SMALL_TILE = 8;
+// perft(3): the fused leaf over the root's children, S_SMALL_TILE per wave,
+// so that the replies to their moves are about one pass of its lanes
+constexpr u32 S_WAVES = LEAF_WG / 64, S_SMALL_TILE = 4;
 template <int V>
-__global__ S_LEAF_BOUNDS(V) void ks_three(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ STile s;
+__global__ PG_LEAF_BOUNDS void ks_three(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
+    __shared__ LeafTile s[S_WAVES];
     SSum sum;
-    const u32 i = blockIdx.x * S_SMALL_TILE + threadIdx.x;
-    const bool live = threadIdx.x < S_SMALL_TILE && i < r.n;
+    const u32 wave = wave_number(), lane = threadIdx.x & 63, i = (blockIdx.x * S_WAVES + wave) * S_SMALL_TILE + lane;
+    const bool live = lane < S_SMALL_TILE && i < r.n;
     Pos b{};
     if (live) b = s_made(r.b, r.mv[i], r.piece[i], t);
-    s_leaf_tile<V>(s, live, b, 1, sum, &P->err, t);
+    s_leaf_tile<V>(s[wave], live, b, sum, &P->err, t);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
     s_finish(P, sum, 3, bias, out, seq);
 }
 
-// The children of the root's move number blockIdx / PARTS, part blockIdx %
-// PARTS of them: every work-group lists the moves of its child of the root
-// itself (one lane), which spares the kernel and the round through memory
-// that a list of ply 2 would take.
-template <int V, int PARTS>
-__device__ __forceinline__ bool s_grandchild(STile &s, const SRoot &r, SPlan *P, u32 *n2, Pos *b, const Tables &t) {
-    const u32 i = blockIdx.x / PARTS, part = blockIdx.x % PARTS;
+// The moves of the child of the root by its move number blockIdx / parts:
+// every work-group lists them itself (one lane), which spares the kernel and
+// the round through memory that a list of ply 2 would take.  The work-group's
+// share is number blockIdx % parts of them, *lo to *hi.
+template <int V>
+__device__ __forceinline__ Pos s_child_moves(u32 *word, const SRoot &r, SPlan *P, u32 parts, u32 *lo, u32 *hi,
+                                             const Tables &t) {
+    __shared__ u32 count;
+    const u32 i = blockIdx.x / parts, part = blockIdx.x % parts;
     const Pos c = s_made(r.b, r.mv[i], r.piece[i], t);
-    if (threadIdx.x == 0) s.next = generate_any<V>(c, t, s.mv, 256, s.tag, 0);
+    if (threadIdx.x == 0) {
+        count = generate_words<V>(c, t, word, 256, 0);
+        if (blockIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
+        if (part == 0) atomicAdd(&P->paths[2], (u64)count);
+    }
     __syncthreads();
-    const u32 n = s.next < 256 ? s.next : 256;
-    const u32 lo = n * part / PARTS, hi = n * (part + 1) / PARTS;
-    const u32 j = lo + threadIdx.x;
-    const bool live = j < hi;
-    if (live) *b = s_made(c, s.mv[j], s.tag[j] >> 8, t);
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
-    if (part == 0 && threadIdx.x == 0) atomicAdd(&P->paths[2], (u64)n);
-    *n2 = hi - lo;
-    __syncthreads();
-    return live;
+    const u32 n = count < 256 ? count : 256;
+    *lo = n * part / parts;
+    *hi = n * (part + 1) / parts;
+    return c;
 }
 
-// perft(4): the fused leaf over the root's grandchildren
-constexpr int S_FOUR_PARTS = 4, S_TOP_PARTS = 2;
+// perft(4): the fused leaf over the root's grandchildren, dealt to the waves
+constexpr u32 S_FOUR_PARTS = 4, S_TOP_PARTS = 2;
 template <int V>
-__global__ S_LEAF_BOUNDS(V) void ks_four(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ STile s;
+__global__ PG_LEAF_BOUNDS void ks_four(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
+    __shared__ LeafTile s[S_WAVES];
+    __shared__ u32 word[256];
     SSum sum;
+    u32 lo, hi;
+    const Pos c = s_child_moves<V>(word, r, P, S_FOUR_PARTS, &lo, &hi, t);
+    const u32 wave = wave_number(), j = lo + (threadIdx.x & 63) * S_WAVES + wave;
+    const bool live = j < hi;
     Pos b{};
-    u32 n;
-    const bool live = s_grandchild<V, S_FOUR_PARTS>(s, r, P, &n, &b, t);
-    s_leaf_tile<V>(s, live, b, 1, sum, &P->err, t);
+    if (live) b = s_made(c, (u16)word[j], piece_code(word[j] >> 24), t);
+    s_leaf_tile<V>(s[wave], live, b, sum, &P->err, t);
     s_finish(P, sum, 4, bias, out, seq);
 }
 
 // plies 1 to 3 of a deeper search: the nodes of ply 2 and the list of ply 3
 template <int V>
-__global__ S_LEAF_BOUNDS(V) void ks_top(SRoot r, SPlan *P, SRegion rg, Tables t) {
-    __shared__ STile s;
+__global__ __launch_bounds__(LEAF_WG) void ks_top(SRoot r, SPlan *P, SRegion rg, Tables t) {
+    __shared__ ListTile s;
+    __shared__ u32 word[256];
     __shared__ u32 first;
     SSum sum;
-    Pos b{};
-    u32 n;
-    const bool live = s_grandchild<V, S_TOP_PARTS>(s, r, P, &n, &b, t);
+    u32 lo, hi;
+    const Pos c = s_child_moves<V>(word, r, P, S_TOP_PARTS, &lo, &hi, t);
     const SLevel L = s_level(rg, 2, 0);
+    const u32 n = hi - lo, j = lo + threadIdx.x;
+    const bool live = j < hi;
     if (threadIdx.x == 0) first = (u32)atomicAdd(&P->nNode[2], (u64)n);
     __syncthreads();
     if (first + n > rg.node2) {  // cannot happen: node2 is the root's moves times the most a position has
         if (threadIdx.x == 0) P->overflow = 1;
         return;
     }
-    if (live) L.node[first + threadIdx.x] = SNode{b, 1, S_NO_SLOT, 0};
+    Pos b{};
+    if (live) {
+        b = s_made(c, (u16)word[j], piece_code(word[j] >> 24), t);
+        L.node[first + threadIdx.x] = SNode{b, 1, S_NO_SLOT, 0};
+    }
     s_list_tile<V>(s, live, b, 1, first, &P->nList[3], L, P, sum, t);
     s_add(&P->paths[3], sum.paths, &P->overflow);
 }
@@ -505,6 +500,12 @@ static __global__ __launch_bounds__(S_COLLAPSE_WG) void ks_collapse(SPlan *P, SR
 // Board number i of ply l and its weight: a node of the collapse (its weight
 // completed here), or (LIST) the listed move i made from its parent, kept as
 // node i for the next ply when KEEP.
+template <bool LIST>
+__device__ __forceinline__ u64 s_weight(const SLevel &A, const SNode *node, u64 i) {
+    if constexpr (LIST) return A.node[A.par[i] & S_NODE_MAX].w;
+    const SNode &nd = node[i];
+    return nd.slot != S_NO_SLOT ? nd.w + A.set[nd.slot].w : nd.w;
+}
 template <bool LIST, bool KEEP>
 __device__ __forceinline__ Pos s_board(const SRegion &rg, const SLevel &A, SNode *node, u64 i, u64 *w, const Tables &t) {
     if constexpr (LIST) {
@@ -527,8 +528,8 @@ __device__ __forceinline__ Pos s_board(const SRegion &rg, const SLevel &A, SNode
 
 // ply l's boards to the list of ply l + 1
 template <int V, bool LIST>
-__global__ S_LEAF_BOUNDS(V) void ks_level(SPlan *P, SRegion rg, int l, Tables t) {
-    __shared__ STile s;
+__global__ __launch_bounds__(LEAF_WG) void ks_level(SPlan *P, SRegion rg, int l, Tables t) {
+    __shared__ ListTile s;
     if (s_stopped(P)) return;
     const SLevel A = s_level(rg, l - 1, P->nNode[l - 1]);
     const u64 n = LIST ? P->nList[l] : P->nNode[l];
@@ -538,7 +539,7 @@ __global__ S_LEAF_BOUNDS(V) void ks_level(SPlan *P, SRegion rg, int l, Tables t)
     }
     const SLevel L = s_level(rg, l, n);
     if (LIST && blockIdx.x == 0 && threadIdx.x == 0) P->nNode[l] = n;
-    const u32 T = s_tile_boards(n);
+    const u32 T = s_tile_boards(n, S_RESIDENT, 8, LEAF_WG);
     SSum sum;
     for (u64 tile = blockIdx.x; tile * T < n; tile += gridDim.x) {
         const u64 i = tile * T + threadIdx.x;
@@ -554,29 +555,40 @@ __global__ S_LEAF_BOUNDS(V) void ks_level(SPlan *P, SRegion rg, int l, Tables t)
 
 // the last plies: perft(2) of ply depth - 2's boards
 template <int V, bool LIST>
-__global__ S_LEAF_BOUNDS(V) void ks_leaf(SPlan *P, SRegion rg, int depth, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ STile s;
-    __shared__ u32 next;
-    SSum sum;
+__global__ PG_LEAF_BOUNDS void ks_leaf(SPlan *P, SRegion rg, int depth, u64 bias, SResult *out, u64 seq, Tables t) {
+    __shared__ LeafTile tiles[S_WAVES];
+    u64 total = 0, paths = 0, items = 0;  // the wave's
+    bool carry = false, wide = false;
     const int l = depth - 2;
     if (!s_stopped(P)) {
-        const SLevel A = s_level(rg, l - 1, P->nNode[l - 1]);
-        const u64 n = LIST ? P->nList[l] : P->nNode[l];
+        const u32 wave = wave_number();
+        LeafTile &s = tiles[wave];
+        const u32 lane = threadIdx.x & 63, waves = gridDim.x * S_WAVES;
+        const SLevel A = s_level(rg, l - 1, uniform64(P->nNode[l - 1]));
+        const u64 n = uniform64(LIST ? P->nList[l] : P->nNode[l]);
         SNode *node = (SNode *)rg.half[l & 1];
-        const u32 T = s_tile_boards(n);
-        // the first tiles are dealt out, the others taken as work-groups get done
-        for (u64 tile = blockIdx.x; tile * T < n;) {
-            if (threadIdx.x == 0) next = atomicAdd(&P->tile, 1u) + gridDim.x;
-            const u64 i = tile * T + threadIdx.x;
-            const bool live = threadIdx.x < T && i < n;
+        const u32 T = s_tile_boards(n, waves, 4, LEAF_TILE);
+        // the first tiles are dealt out, the others taken as waves get done
+        for (u64 tile = blockIdx.x * S_WAVES + wave; tile * T < n;) {
+            u32 next = 0;
+            if (lane == 0) next = atomicAdd(&P->tile, 1u) + waves;
+            const u64 i = tile * T + lane;
+            const bool live = lane < T && i < n;
             Pos b{};
-            u64 w = 0;
+            u64 w;
             if (live) b = s_board<LIST, false>(rg, A, node, i, &w, t);
-            s_leaf_tile<V>(s, live, b, w, sum, &P->err, t);
-            tile = next;
-            __syncthreads();
+            tile = (u32)__builtin_amdgcn_readfirstlane((int)next);
+            const u32 c = leaf_expand<V>(s, live, b, &P->err, t);
+            w = 0;
+            if (live) w = s_weight<LIST>(A, node, i);  // again: there is no register to keep it in
+            s_wave_mad(&total, w, live ? s.per[lane] : 0, &carry);
+            s_wave_mad(&paths, w, c, &wide);
+            items += wave_sum32(c);
+            wave_sync();
         }
     }
+    SSum sum;
+    if ((threadIdx.x & 63) == 0) sum = SSum{total, items, paths, carry, wide};
     s_finish(P, sum, depth, bias, out, seq);
 }
 

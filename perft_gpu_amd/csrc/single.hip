@@ -53,7 +53,7 @@ static void launch(Engine &e, const Single &s, const SRoot &r, const SRegion &rg
     if (depth <= 2) {
         ks_one<V><<<1, LEAF_WG, 0, st>>>(r, s.plan, depth, bias, s.res, s.seq, e.dt);
     } else if (depth == 3 || r.n == 0) {
-        const int g = r.n ? (r.n + S_SMALL_TILE - 1) / S_SMALL_TILE : 1;
+        const int g = r.n ? (r.n + S_SMALL_TILE * S_WAVES - 1) / (S_SMALL_TILE * S_WAVES) : 1;
         ks_three<V><<<g, LEAF_WG, 0, st>>>(r, s.plan, bias, s.res, s.seq, e.dt);
     } else if (depth == 4) {
         ks_four<V><<<r.n * S_FOUR_PARTS, LEAF_WG, 0, st>>>(r, s.plan, bias, s.res, s.seq, e.dt);
@@ -66,7 +66,7 @@ static void launch(Engine &e, const Single &s, const SRoot &r, const SRegion &rg
                 ks_collapse<<<l <= 3 ? 256 : e.cus * 8, S_COLLAPSE_WG, 0, st>>>(s.plan, rg, l, e.dt);
             }
             if (l == depth - 2) {
-                const int g = e.cus * 4;
+                const int g = e.cus * 3;  // as many as are resident
                 if (set) ks_leaf<V, false><<<g, LEAF_WG, 0, st>>>(s.plan, rg, depth, bias, s.res, s.seq, e.dt);
                 else ks_leaf<V, true><<<g, LEAF_WG, 0, st>>>(s.plan, rg, depth, bias, s.res, s.seq, e.dt);
             } else {
@@ -92,15 +92,15 @@ int perft_single(Engine &e, const Pos &root, u32 depth, int v, bool collapse, u6
     if (!ht) return PG_ETABLE;
     SRoot r{};
     r.b = root;
-    u16 mv[256], tag[256];
-    r.n = generate_any<SL_KOGGE>(root, ht->view(), mv, 256, tag, 0);
+    u32 word[256];
+    r.n = generate_words<SL_KOGGE>(root, ht->view(), word, 256, 0);
     if (r.n > S_MOVES) {
         set_error("the position has %u moves", r.n);
         return PG_EINVAL;
     }
     for (u32 i = 0; i < r.n; i++) {
-        r.mv[i] = mv[i];
-        r.piece[i] = (u8)(tag[i] >> 8);
+        r.mv[i] = (u16)word[i];
+        r.piece[i] = (u8)piece_code(word[i] >> 24);
     }
     SRegion rg{};
     rg.bytes = (e.arenaBytes / 2) & ~(size_t)255;

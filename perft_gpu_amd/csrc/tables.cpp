@@ -2,7 +2,7 @@
 //
 // Same tables as MoveGeneratorBitboard::init (MoveGeneratorBitboard.h:982-
 // 1080) and Magics.cpp, constructed by this code:
-//  * empty-board attacks, squares-between and full-line tables;
+//  * empty-board attacks, king rows, pin entries and full lines;
 //  * relevant-occupancy masks (edges removed, :1026-1047);
 //  * plain magics: 12-bit rook / 9-bit bishop tables found by a seeded search
 //    (the reference seeds from the clock, :1025; a fixed seed keeps builds
@@ -94,9 +94,15 @@ int HostTables::build(u64 seed, char *err, int errlen) {
     }
     for (int a = 0; a < 64; a++)
         for (int b = 0; b < 64; b++) {
-            between[a * 64 + b] = between_sq(a, b);
             line[a * 64 + b] = a == b ? file_of(a) : line_sq(a, b);
+            // a: the king, b: the slider
+            PinEntry &e = pin[a * 64 + b];
+            e.between = between_sq(a, b);
+            e.behind = 0;
+            if (a != b && (line_sq(a, b) & bit(b))) e.behind = line_sq(a, b) & king[a] & ~e.between & ~bit(b);
         }
+    for (int s = 0; s < 64; s++)
+        row[s] = KingRow{rookEmpty[s], bishopEmpty[s], knight[s], king[s], file_of(s), rank_of(s), diag_of(s), anti_of(s)};
     for (int s = 0; s < 64; s++) {
         u64 sq = bit(s), m = rookEmpty[s] & ~sq;
         if (!(sq & RANK1)) m &= ~RANK1;
@@ -179,8 +185,8 @@ int HostTables::build(u64 seed, char *err, int errlen) {
 
 Tables HostTables::view() const {
     Tables t;
-    t.knight = knight; t.king = king; t.rookEmpty = rookEmpty; t.bishopEmpty = bishopEmpty;
-    t.between = between; t.line = line; t.rookMask = rookMask; t.bishopMask = bishopMask;
+    t.knight = knight; t.king = king; t.row = row; t.pin = pin;
+    t.line = line; t.rookMask = rookMask; t.bishopMask = bishopMask;
     t.rookMagic = rookMagic; t.bishopMagic = bishopMagic;
     t.rookPlain = rookPlain.data(); t.bishopPlain = bishopPlain.data();
     t.rookFancy = rookFancy; t.bishopFancy = bishopFancy; t.fancy = fancy.data();
@@ -189,9 +195,8 @@ Tables HostTables::view() const {
     return t;
 }
 
-static const size_t kSizes[19] = {
-    64 * 8, 64 * 8, 64 * 8, 64 * 8,              // knight king rookEmpty bishopEmpty
-    4096 * 8, 4096 * 8,                          // between line
+static const size_t kSizes[TABLE_COUNT] = {
+    64 * 8, 64 * 8, sizeof(KingRow) * 64, sizeof(PinEntry) * 4096, 4096 * 8,  // knight king row pin line
     64 * 8, 64 * 8, 64 * 8, 64 * 8,              // masks, plain factors
     (64u << ROOK_BITS) * 8, (64u << BISHOP_BITS) * 8,
     64 * 16, 64 * 16,                            // fancy entries
@@ -203,7 +208,7 @@ static const size_t kSizes[19] = {
 TableLayout table_layout() {
     TableLayout L;
     size_t o = 0;
-    for (int i = 0; i < 19; i++) {
+    for (int i = 0; i < TABLE_COUNT; i++) {
         L.off[i] = o;
         o += (kSizes[i] + 255) & ~(size_t)255;
     }
@@ -214,13 +219,13 @@ TableLayout table_layout() {
 void pack_tables(const HostTables &h, std::vector<u8> &blob) {
     TableLayout L = table_layout();
     blob.assign(L.total, 0);
-    const void *src[19] = {h.knight, h.king, h.rookEmpty, h.bishopEmpty, h.between, h.line, h.rookMask,
-                           h.bishopMask, h.rookMagic, h.bishopMagic, h.rookPlain.data(), h.bishopPlain.data(),
-                           h.rookFancy, h.bishopFancy, h.fancy.data(), h.byteIdx.data(), h.byteRook.data(),
-                           h.byteBishop.data(), nullptr};
-    for (int i = 0; i < 18; i++) memcpy(&blob[L.off[i]], src[i], kSizes[i]);
-    memcpy(&blob[L.off[18]], h.zobLo, ZOB_WORDS * 8);
-    memcpy(&blob[L.off[18] + ZOB_WORDS * 8], h.zobHi, ZOB_WORDS * 8);
+    const void *src[TABLE_COUNT - 1] = {h.knight, h.king, h.row, h.pin, h.line, h.rookMask, h.bishopMask, h.rookMagic,
+                                        h.bishopMagic, h.rookPlain.data(), h.bishopPlain.data(), h.rookFancy,
+                                        h.bishopFancy, h.fancy.data(), h.byteIdx.data(), h.byteRook.data(),
+                                        h.byteBishop.data()};
+    for (int i = 0; i < TABLE_COUNT - 1; i++) memcpy(&blob[L.off[i]], src[i], kSizes[i]);
+    memcpy(&blob[L.off[TABLE_COUNT - 1]], h.zobLo, ZOB_WORDS * 8);
+    memcpy(&blob[L.off[TABLE_COUNT - 1] + ZOB_WORDS * 8], h.zobHi, ZOB_WORDS * 8);
 }
 
 Tables tables_at(const u8 *b) {
@@ -228,24 +233,23 @@ Tables tables_at(const u8 *b) {
     Tables t;
     t.knight = (const u64 *)(b + L.off[0]);
     t.king = (const u64 *)(b + L.off[1]);
-    t.rookEmpty = (const u64 *)(b + L.off[2]);
-    t.bishopEmpty = (const u64 *)(b + L.off[3]);
-    t.between = (const u64 *)(b + L.off[4]);
-    t.line = (const u64 *)(b + L.off[5]);
-    t.rookMask = (const u64 *)(b + L.off[6]);
-    t.bishopMask = (const u64 *)(b + L.off[7]);
-    t.rookMagic = (const u64 *)(b + L.off[8]);
-    t.bishopMagic = (const u64 *)(b + L.off[9]);
-    t.rookPlain = (const u64 *)(b + L.off[10]);
-    t.bishopPlain = (const u64 *)(b + L.off[11]);
-    t.rookFancy = (const FancyEntry *)(b + L.off[12]);
-    t.bishopFancy = (const FancyEntry *)(b + L.off[13]);
-    t.fancy = (const u64 *)(b + L.off[14]);
-    t.byteIdx = (const u8 *)(b + L.off[15]);
-    t.byteRook = (const u64 *)(b + L.off[16]);
-    t.byteBishop = (const u64 *)(b + L.off[17]);
-    t.zobLo = (const u64 *)(b + L.off[18]);
-    t.zobHi = (const u64 *)(b + L.off[18] + ZOB_WORDS * 8);
+    t.row = (const KingRow *)(b + L.off[2]);
+    t.pin = (const PinEntry *)(b + L.off[3]);
+    t.line = (const u64 *)(b + L.off[4]);
+    t.rookMask = (const u64 *)(b + L.off[5]);
+    t.bishopMask = (const u64 *)(b + L.off[6]);
+    t.rookMagic = (const u64 *)(b + L.off[7]);
+    t.bishopMagic = (const u64 *)(b + L.off[8]);
+    t.rookPlain = (const u64 *)(b + L.off[9]);
+    t.bishopPlain = (const u64 *)(b + L.off[10]);
+    t.rookFancy = (const FancyEntry *)(b + L.off[11]);
+    t.bishopFancy = (const FancyEntry *)(b + L.off[12]);
+    t.fancy = (const u64 *)(b + L.off[13]);
+    t.byteIdx = (const u8 *)(b + L.off[14]);
+    t.byteRook = (const u64 *)(b + L.off[15]);
+    t.byteBishop = (const u64 *)(b + L.off[16]);
+    t.zobLo = (const u64 *)(b + L.off[17]);
+    t.zobHi = (const u64 *)(b + L.off[17] + ZOB_WORDS * 8);
     return t;
 }
 

@@ -10,7 +10,9 @@ namespace pg {
 
 struct HostTables {
     u64 knight[64], king[64], rookEmpty[64], bishopEmpty[64];
-    u64 between[64 * 64], line[64 * 64];
+    KingRow row[64];
+    PinEntry pin[64 * 64];
+    u64 line[64 * 64];
     u64 rookMask[64], bishopMask[64];
     u64 rookMagic[64], bishopMagic[64];
     std::vector<u64> rookPlain, bishopPlain;      // 64*4096, 64*512
@@ -30,9 +32,11 @@ struct HostTables {
 // Returns null, with a message in *err, if construction failed.
 const HostTables *host_tables(const char **err = nullptr);
 
+constexpr int TABLE_COUNT = 18;
+
 // Serialized byte layout used for the single device allocation.
 struct TableLayout {
-    size_t off[20];
+    size_t off[TABLE_COUNT];
     size_t total;
 };
 TableLayout table_layout();
