@@ -303,6 +303,148 @@ __device__ __forceinline__ u64 block_excl_scan(u64 v, u64 *total) {
 constexpr int LEAF_WG = 256, LEAF_TILE = 64, LEAF_CAP = 1488, LEAF_BLOCKS_PER_CU = 64;
 constexpr u32 LEAF_LATE = 1u << 29;  // window word: a special move that found no room in the aside list
 
+// a value that all lanes hold, in scalar registers
+__device__ __forceinline__ u64 uniform64(u64 v) {
+    return (u64)(u32)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (u32)__builtin_amdgcn_readfirstlane((int)v);
+}
+// the wave's sum of v, in scalar registers
+__device__ __forceinline__ u32 wave_sum32(u32 v) {
+    u32 x = v;
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);  // row_shr 1, 2, 4, 8
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);
+    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);
+    return (u32)(__builtin_amdgcn_readlane((int)x, 15) + __builtin_amdgcn_readlane((int)x, 31) +
+                 __builtin_amdgcn_readlane((int)x, 47) + __builtin_amdgcn_readlane((int)x, 63));
+}
+// p after the move mv of its piece of code `piece`
+__device__ __forceinline__ Pos made(Pos p, u16 mv, int piece, const Tables &t) {
+    if (pos_side(p)) make_move_as<BLACK, false>(p, mv, piece, nullptr, t);
+    else make_move_as<WHITE, false>(p, mv, piece, nullptr, t);
+    return p;
+}
+__device__ __forceinline__ u32 lanes_below(u64 mask) {
+    return __builtin_amdgcn_mbcnt_hi((u32)(mask >> 32), __builtin_amdgcn_mbcnt_lo((u32)mask, 0));
+}
+// orders a wave's LDS accesses (each wave's are carried out in order; this
+// keeps the compiler from moving them)
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// a board that all lanes hold, in scalar registers
+__device__ __forceinline__ Pos uniform_pos(Pos p) {
+    u64 w[sizeof(Pos) / 8];
+    memcpy(w, &p, sizeof(Pos));
+#pragma unroll
+    for (u32 i = 0; i < sizeof(Pos) / 8; i++) w[i] = uniform64(w[i]);
+    memcpy(&p, w, sizeof(Pos));
+    return p;
+}
+
+// the same, kept apart from earlier uses: nothing worked out from it stays in
+// registers from one use to the next
+__device__ __forceinline__ Pos opaque_pos(Pos p) {
+    u64 w[sizeof(Pos) / 8];
+    memcpy(w, &p, sizeof(Pos));
+#pragma unroll
+    for (u32 i = 0; i < sizeof(Pos) / 8; i++) asm volatile("" : "+s"(w[i]));
+    memcpy(&p, w, sizeof(Pos));
+    return p;
+}
+
+// The moves of one board listed by a whole wave.  The board is the same in
+// all lanes: what concerns all of it is worked out by the scalar unit, and a
+// lane works out the piece on its own square, an enemy slider's attacks or
+// one's own moves.  One lane that lists a board by itself (generate_words)
+// takes about four times as long, for it does one piece after the other.
+struct WaveSink {
+    u32 *word;
+    u32 n, lane;
+    __device__ void add(u32 m, u32 piece) {
+        if (lane == 0) word[n] = m | piece << 24;
+        n++;
+    }
+    template <class F> __device__ void squares(u64 m, u64, u32 piece, F &&f) {
+        if (m >> lane & 1) word[n + lanes_below(m)] = f((int)lane) | piece << 24;
+        n += (u32)popc(m);
+    }
+    __device__ void skipped(u64) {}
+};
+__device__ __forceinline__ u32 wave_or32(u32 x) {
+    x |= (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);  // row_shr 1, 2, 4, 8
+    x |= (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);
+    x |= (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);
+    x |= (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);
+    return (u32)(__builtin_amdgcn_readlane((int)x, 15) | __builtin_amdgcn_readlane((int)x, 31) |
+                 __builtin_amdgcn_readlane((int)x, 47) | __builtin_amdgcn_readlane((int)x, 63));
+}
+__device__ __forceinline__ u64 wave_or64(u64 x) { return (u64)wave_or32((u32)(x >> 32)) << 32 | wave_or32((u32)x); }
+
+template <int C, int V>
+__device__ __forceinline__ void wave_side_words(const Pos &p, const Tables &t, WaveSink &o) {
+    const Sides s = sides_of<C>(p);
+    const u32 sq = o.lane;
+    const u64 here = bit((int)sq);
+    const bool rook = (s.myRooks | s.eRooks) & here, bishop = (s.myBishops | s.eBishops) & here, enemy = s.enemy & here;
+    const u64 occ = enemy ? s.occ ^ s.myKing : s.occ;  // enemy sliders look through the king
+    u64 att = 0;
+    if (rook) att = Sl<V>::rook(t, (int)sq, occ);
+    if (bishop) att |= Sl<V>::bishop(t, (int)sq, occ);
+    MoveCtx x;
+    x.threatened = leaper_attacks<C>(s, t) | wave_or64(enemy ? att : 0);
+    const KingRow &row = t.row[s.k];
+    const bool line = or_and(row.rook & s.eRooks, row.bishop, s.eBishops) & here;
+    u64 b = ~0ULL;  // what stands between an enemy slider and the king
+    if (line) b = t.pin[s.k << 6 | (int)sq].between & s.occ;
+    x.checkers = leaper_checks<C>(s, t, __ballot(b == 0));
+    x.pinned = wave_or64(several(b) ? 0 : b) & s.mine;
+    x.target = ~s.mine;
+    if (x.checkers) x.target &= several(x.checkers) ? 0ULL : x.checkers | t.pin[s.k << 6 | ctz(x.checkers)].between;
+    const Gen g{x.pinned, x.checkers, x.target, and_nor(row.king, s.mine, x.threatened), 0, 0, 0, 0, 0, 0, 0, 0, 0,
+                castle_moves<C>(s, x)};
+    if (!king_pawn_moves<C>(s, g, t, o)) return;
+    const bool knight = s.myKnights & here;
+    u64 m = (knight ? t.knight[sq] : enemy ? 0 : att) & x.target;
+    if (m && x.pinned & here) m &= knight ? 0 : t.line[sq << 6 | (u32)s.k];
+    const u32 piece = knight ? M_KNIGHT : (bishop ? M_BISHOP : 0u) | (rook ? M_ROOK : 0u);
+    for (u64 left = __ballot(m != 0); left; left = __ballot(m != 0)) {
+        if (m) {
+            o.word[o.n + lanes_below(left)] = mk_move((int)sq, ctz(m), MF_QUIET) | piece << 24;
+            m &= m - 1;
+        }
+        o.n += (u32)popc(left);
+    }
+}
+// out: room for the moves of any position
+template <int V>
+__device__ __forceinline__ u32 wave_words(const Pos &p, const Tables &t, u32 *out) {
+    WaveSink o{out, 0, threadIdx.x & 63};
+    if (pos_side(p)) wave_side_words<BLACK, V>(p, t, o);
+    else wave_side_words<WHITE, V>(p, t, o);
+    return (u32)__builtin_amdgcn_readfirstlane((int)o.n);
+}
+
+// perft(2) of one board by a whole wave: its moves are listed, then counted a
+// lane each.  Returns the lane's part; *moves: the board's moves.  About 5 us
+// for a wave alone, where a tile of the fused leaf takes 25 and more, but
+// about ten times the instructions per board of a full tile.
+template <int V>
+__device__ __forceinline__ u32 wave_perft2(const Pos &b, u32 *list, u32 *moves, const Tables &t) {
+    const u32 m = wave_words<V>(b, t, list), lane = threadIdx.x & 63;
+    wave_sync();
+    u32 sum = 0;
+    for (u32 k = lane; k < m; k += 64) sum += count_any<V>(made(b, (u16)list[k], piece_code(list[k] >> 24), t), t);
+    wave_sync();
+    *moves = m;
+    return sum;
+}
+// the board after the move in list[i], in scalar registers
+__device__ __forceinline__ Pos wave_made(const Pos &b, const u32 *list, u32 i, const Tables &t) {
+    const u32 w = (u32)__builtin_amdgcn_readfirstlane((int)list[i]);
+    return uniform_pos(made(b, (u16)w, piece_code(w >> 24), t));
+}
+
 // state of a board after expansion (TT and batch searches)
 enum : u8 { ST_LIVE = 0, ST_HIT = 1, ST_DUP = 2 };
 
@@ -316,15 +458,6 @@ struct LeafTile {
 // addressed by it, and loops over it, then stay out of the vector registers
 __device__ __forceinline__ u32 wave_number() { return (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
-// orders a wave's LDS accesses (each wave's are carried out in order; this
-// keeps the compiler from moving them)
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-__device__ __forceinline__ u32 lanes_below(u64 mask) {
-    return __builtin_amdgcn_mbcnt_hi((u32)(mask >> 32), __builtin_amdgcn_mbcnt_lo((u32)mask, 0));
-}
 __device__ __forceinline__ u32 wave_excl_scan(u32 v, u32 *total) {
     const int lane = threadIdx.x & 63;
     u32 x = v;
@@ -407,6 +540,16 @@ __device__ __forceinline__ u32 leaf_expand(LeafTile &s, bool live, const Pos &b,
     return moves;
 }
 
+// Boards per tile: too few boards for whole tiles on every CU are dealt out a
+// few at a time, for the time of the longest tile (a wave alone takes about
+// 15 us for one).
+constexpr u32 LEAF_RESIDENT = 3072;  // waves the chip holds
+__device__ __forceinline__ u32 leaf_tile_boards(u64 n, u32 waves) {
+    if (waves > LEAF_RESIDENT) waves = LEAF_RESIDENT;
+    const u64 t = (n + waves - 1) / waves;
+    return t < 4 ? 4 : t > LEAF_TILE ? LEAF_TILE : (u32)t;
+}
+
 // The fused leaf over boards [0, n) with move counts cnt[]: PER = false adds
 // every count to *acc; PER = true writes base + perft(2) to per[i] for live
 // boards (state[i] == ST_LIVE when state is given, else a valid board).
@@ -429,9 +572,11 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
     LeafTile &s = tiles[wave];
     const u32 lane = threadIdx.x & 63;
     u64 sum = 0, itemSum = 0;
-    for (u64 tile = blockIdx.x * WAVES + wave; tile * LEAF_TILE < n; tile += gridDim.x * WAVES) {
-        const u64 t0 = tile * LEAF_TILE + lane;
-        const bool live = t0 < n;
+    n = uniform64(n);
+    const u32 T = leaf_tile_boards(n, gridDim.x * WAVES);
+    for (u64 tile = blockIdx.x * WAVES + wave; tile * T < n; tile += gridDim.x * WAVES) {
+        const u64 t0 = tile * T + lane;
+        const bool live = lane < T && t0 < n;
         const u64 i = idx && live ? (u64)idx[t0] : t0;
         bool valid = false, work = live;
         Pos b{};
@@ -445,7 +590,7 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
                 work = cnt[i] != 0;  // a board resolved earlier has count 0
             }
         }
-        itemSum += leaf_expand<V>(s, work, b, err, t);
+        itemSum += wave_sum32(leaf_expand<V>(s, work, b, err, t));
         if (live) {
             const u32 p = work ? s.per[lane] : 0;
             if constexpr (PER) {
@@ -460,7 +605,6 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
         }
         wave_sync();
     }
-    itemSum = wave_sum(itemSum);
     if ((threadIdx.x & 63) == 0 && items && itemSum) atomicAdd(items, itemSum);
     if (!PER) {
         sum = wave_sum(sum);

@@ -768,11 +768,13 @@ PG_HD Gen gen_all(const Sides &s, const Tables &t) {
 // Hands the legal moves of s that are not left out (at most 218) to the sink.
 // Pawn captures carry the capture flag; other captures do not, as on the
 // reference's device path (MoveGeneratorBitboard.h:2525-2529).
-template <int C, int V, class Sink>
-PG_HD void generate_sides(const Sides &s, const Gen &g, const Tables &t, Sink &o) {
+// First the king's and the pawns' moves and castling; false if the king alone
+// may move.
+template <int C, class Sink>
+PG_HD bool king_pawn_moves(const Sides &s, const Gen &g, const Tables &t, Sink &o) {
     const u64 tgt = g.target, empty = ~s.occ;
     o.squares(g.king, g.kingFull, M_KING, [&](int to) { return mk_move(s.k, to, MF_QUIET); });
-    if (tgt == 0) return;
+    if (tgt == 0) return false;
 
     // a pinned pawn moves only along its pin line
     u64 pf = s.myPawns, pw = s.myPawns, pe = s.myPawns;
@@ -823,6 +825,13 @@ PG_HD void generate_sides(const Sides &s, const Gen &g, const Tables &t, Sink &o
     constexpr int e = C == WHITE ? 4 : 60;
     if (g.castle & 1) o.add(mk_move(e, e + 2, MF_KING_CASTLE), M_KING | M_SPECIAL);
     if (g.castle & 2) o.add(mk_move(e, e - 2, MF_QUEEN_CASTLE), M_KING | M_SPECIAL);
+    return true;
+}
+
+template <int C, int V, class Sink>
+PG_HD void generate_sides(const Sides &s, const Gen &g, const Tables &t, Sink &o) {
+    if (!king_pawn_moves<C>(s, g, t, o)) return;
+    const u64 tgt = g.target;
     // a piece on q with moves m, its quiet and calm sets
     auto moves = [&](int q, u64 m, u64 quiet, u64 calm, u32 piece) {
         const u64 left = and3(m, quiet, mask_if((quiet >> q) & 1));

@@ -50,16 +50,19 @@ constexpr u64 S_ITEM_MAX = 3400000000ULL;  // s_slots of as many items: slot num
 
 // Device state of a search.  All counters are zero between calls: the last
 // work-group of a search publishes them to the host and clears them.  Every
-// work-group of the last kernel adds into acc, items, paths and done, which
-// therefore lie in lines of their own (atomics on one address take about 6 ns
-// each, one after the other).
+// work-group of the last kernel adds into acc, paths, items and done.  Atomics
+// on one line take about 6 ns each, one after the other, so each of these is
+// spread over banks (work-group i adds to bank i % S_BANKS).
+constexpr u32 S_BANKS = 32;
 struct SPlan {
     alignas(128) u64 nNode[S_MAX_PLY];  // boards kept per ply
     alignas(128) u64 nList[S_MAX_PLY];  // moves listed per ply (the boards of that ply before the collapse)
     alignas(128) u64 paths[S_MAX_PLY];  // perft(ply): the listed moves, each with its parent's weight
-    alignas(128) u64 acc;
-    alignas(128) u64 items;
-    alignas(128) u32 done;
+    struct alignas(128) Bank {
+        u64 acc, paths, items;          // of the last kernel; paths: of its ply
+        u32 done;
+    } bank[S_BANKS];
+    alignas(128) u32 done;              // banks that are complete
     alignas(128) u32 tile;              // next tile of the last kernel
     alignas(128) u32 overflow, err, ovf;
 };
@@ -125,10 +128,6 @@ PG_HD u64 s_node_cap(const SRegion &r) {
 }
 
 // ---------------------------------------------------------------- tiles
-// a value that all lanes hold, in scalar registers
-__device__ __forceinline__ u64 uniform64(u64 v) {
-    return (u64)(u32)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (u32)__builtin_amdgcn_readfirstlane((int)v);
-}
 // Boards per tile of the leaf (a wave each) and of the level kernel (a
 // work-group each): a level of too few boards for whole tiles on every CU is
 // dealt out a few at a time, for the time of its longest tile.
@@ -138,6 +137,12 @@ __device__ __forceinline__ u32 s_tile_boards(u64 n, u32 tiles, u32 least, u32 mo
     return t < least ? least : t > most ? most : (u32)t;
 }
 
+// the wave's sum of v; *wide: it passed 64 bits
+__device__ __forceinline__ u64 s_wave_total(u64 v, bool *wide) {
+    const u64 lo = wave_sum(v & 0xFFFFFFFFULL), hi = wave_sum(v >> 32) + (lo >> 32);
+    *wide |= hi >> 32 != 0;
+    return hi << 32 | (lo & 0xFFFFFFFFULL);
+}
 // *acc += the work-group's sum of s, one atomic; sums may need all 64 bits,
 // and *ovf is raised when a total passes them
 __device__ __forceinline__ void s_add(u64 *acc, u64 s, u32 *ovf) {
@@ -172,27 +177,6 @@ struct SSum {
     bool carry = false, wide = false;
 };
 
-// perft(2) of the wave's boards, each counted once
-template <int V>
-__device__ __forceinline__ void s_leaf_tile(LeafTile &s, bool live, const Pos &b, SSum &sum, u32 *err, const Tables &t) {
-    const u32 c = leaf_expand<V>(s, live, b, err, t);
-    if (live) {
-        sum.total += s.per[threadIdx.x & 63];
-        sum.paths += c;
-        sum.items += c;
-    }
-}
-
-// the wave's sum of v, in scalar registers
-__device__ __forceinline__ u32 wave_sum32(u32 v) {
-    u32 x = v;
-    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true);  // row_shr 1, 2, 4, 8
-    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true);
-    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true);
-    x += (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true);
-    return (u32)(__builtin_amdgcn_readlane((int)x, 15) + __builtin_amdgcn_readlane((int)x, 31) +
-                 __builtin_amdgcn_readlane((int)x, 47) + __builtin_amdgcn_readlane((int)x, 63));
-}
 // *s += the wave's sum of w * c, all in scalar registers: the leaf leaves no
 // vector register for a lane's sums.  *wide: the sum passed 64 bits.
 __device__ __forceinline__ void s_wave_mad(u64 *s, u64 w, u32 c, bool *wide) {
@@ -260,13 +244,8 @@ __device__ __forceinline__ void s_list_tile(ListTile &s, bool live, const Pos &b
     __syncthreads();
 }
 
-__device__ __forceinline__ Pos s_made(Pos p, u16 mv, int piece, const Tables &t) {
-    if (pos_side(p)) make_move_as<BLACK, false>(p, mv, piece, nullptr, t);
-    else make_move_as<WHITE, false>(p, mv, piece, nullptr, t);
-    return p;
-}
 __device__ __forceinline__ Pos s_child(const SNode *nodes, u32 par, u16 mv, const Tables &t) {
-    return s_made(nodes[par & S_NODE_MAX].b, mv, (int)(par >> S_NODE_BITS), t);
+    return made(nodes[par & S_NODE_MAX].b, mv, (int)(par >> S_NODE_BITS), t);
 }
 
 __device__ __forceinline__ u64 s_load(const u64 *p) {
@@ -291,29 +270,51 @@ __device__ __forceinline__ bool s_stopped(const SPlan *P) {
 // writer arrived, so waiting for one's own is enough (a release fence would
 // write the L2 back once per work-group).
 __device__ __forceinline__ void s_finish(SPlan *P, const SSum &sum, int depth, u64 bias, SResult *out, u64 seq) {
-    s_add(&P->acc, sum.total, &P->ovf);
-    s_add(&P->paths[depth - 1], sum.paths, &P->overflow);
-    s_add(&P->items, sum.items, &P->overflow);
+    const u32 bank = blockIdx.x % S_BANKS, banks = gridDim.x < S_BANKS ? gridDim.x : S_BANKS;
+    SPlan::Bank &B = P->bank[bank];
+    s_add(&B.acc, sum.total, &P->ovf);
+    s_add(&B.paths, sum.paths, &P->overflow);
+    s_add(&B.items, sum.items, &P->overflow);
     if (sum.carry) atomicOr(&P->ovf, 1u);
     if (sum.wide) atomicOr(&P->overflow, 1u);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x) return;
-    if (atomicAdd(&P->done, 1u) + 1 != gridDim.x) return;
-    const u64 acc = s_load(&P->acc);
+    __shared__ u32 last;
+    if (threadIdx.x == 0) {
+        last = 0;
+        const u32 members = (gridDim.x - bank + S_BANKS - 1) / S_BANKS;
+        if (atomicAdd(&B.done, 1u) + 1 == members) last = atomicAdd(&P->done, 1u) + 1 == banks;
+    }
+    __syncthreads();
+    if (!last || threadIdx.x >= 64) return;
+    // the last work-group's first wave: the banks' sums, with carries
+    const u32 lane = threadIdx.x;
+    u64 acc = 0, paths = 0, items = 0;
+    if (lane < banks) {
+        SPlan::Bank &L = P->bank[lane];
+        acc = s_load(&L.acc);
+        paths = s_load(&L.paths);
+        items = s_load(&L.items);
+        L.acc = L.paths = L.items = 0;
+        L.done = 0;
+    }
+    bool accWide = false, pathsWide = false;
+    acc = s_wave_total(acc, &accWide);
+    paths = s_wave_total(paths, &pathsWide);
+    items = wave_sum(items);
+    if (lane) return;
     out->acc = acc + bias;
-    out->ovf = s_load(&P->ovf) | (acc + bias < bias);
-    out->overflow = s_load(&P->overflow);
+    out->ovf = s_load(&P->ovf) | accWide | (acc + bias < bias);
+    out->overflow = s_load(&P->overflow) | pathsWide;
     out->err = s_load(&P->err);
-    out->items = s_load(&P->items);
-    const int last = depth >= 2 ? depth - 2 : 0;
-    const u64 kept = s_load(&P->nNode[last]);
-    out->boards = kept ? kept : s_load(&P->nList[last]);
+    out->items = items;
+    const int l2 = depth >= 2 ? depth - 2 : 0;
+    const u64 kept = s_load(&P->nNode[l2]);
+    out->boards = kept ? kept : s_load(&P->nList[l2]);
     for (int l = 0; l < S_MAX_PLY; l++) {
-        out->paths[l] = s_load(&P->paths[l]);
+        out->paths[l] = s_load(&P->paths[l]) + (l == depth - 1 ? paths : 0);
         P->nNode[l] = P->nList[l] = P->paths[l] = 0;
     }
-    P->acc = P->items = 0;
     P->overflow = P->err = P->ovf = P->done = P->tile = 0;
     __hip_atomic_store(&out->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -327,92 +328,117 @@ __global__ __launch_bounds__(LEAF_WG) void ks_one(SRoot r, SPlan *P, int depth, 
     if (depth == 1) {
         if (tid == 0) sum.total = sum.paths = count_any<V>(r.b, t);
     } else if (tid < r.n) {
-        sum.total = count_any<V>(s_made(r.b, r.mv[tid], r.piece[tid], t), t);
+        sum.total = count_any<V>(made(r.b, r.mv[tid], r.piece[tid], t), t);
         sum.items = sum.paths = 1;
     }
     s_finish(P, sum, depth, bias, out, seq);
 }
 
-// perft(3): the fused leaf over the root's children, S_SMALL_TILE per wave,
-// so that the replies to their moves are about one pass of its lanes
-constexpr u32 S_WAVES = LEAF_WG / 64, S_SMALL_TILE = 4;
+// perft(3): a wave per child of the root
+constexpr u32 S_WAVES = LEAF_WG / 64;
 template <int V>
-__global__ PG_LEAF_BOUNDS void ks_three(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ LeafTile s[S_WAVES];
+__global__ __launch_bounds__(LEAF_WG) void ks_three(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
+    __shared__ u32 list[S_WAVES][256];
     SSum sum;
-    const u32 wave = wave_number(), lane = threadIdx.x & 63, i = (blockIdx.x * S_WAVES + wave) * S_SMALL_TILE + lane;
-    const bool live = lane < S_SMALL_TILE && i < r.n;
-    Pos b{};
-    if (live) b = s_made(r.b, r.mv[i], r.piece[i], t);
-    s_leaf_tile<V>(s[wave], live, b, sum, &P->err, t);
+    const u32 wave = wave_number(), i = blockIdx.x * S_WAVES + wave;
+    if (i < r.n) {
+        u32 moves;
+        sum.total = wave_perft2<V>(uniform_pos(made(r.b, r.mv[i], r.piece[i], t)), list[wave], &moves, t);
+        if ((threadIdx.x & 63) == 0) sum.items = sum.paths = moves;
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
     s_finish(P, sum, 3, bias, out, seq);
 }
 
-// The moves of the child of the root by its move number blockIdx / parts:
-// every work-group lists them itself (one lane), which spares the kernel and
-// the round through memory that a list of ply 2 would take.  The work-group's
-// share is number blockIdx % parts of them, *lo to *hi.
+// Plies 1 and 2 of a deeper search: the waves of work-group blockIdx list the
+// moves of the child of the root by its move number blockIdx / parts, each by
+// itself, which spares the kernel and the round through memory that a list of
+// ply 2 would take.  The work-group's share is number blockIdx % parts of
+// them, *lo to *hi.
 template <int V>
-__device__ __forceinline__ Pos s_child_moves(u32 *word, const SRoot &r, SPlan *P, u32 parts, u32 *lo, u32 *hi,
+__device__ __forceinline__ Pos s_child_moves(u32 *list, const SRoot &r, SPlan *P, u32 parts, u32 *lo, u32 *hi,
                                              const Tables &t) {
-    __shared__ u32 count;
     const u32 i = blockIdx.x / parts, part = blockIdx.x % parts;
-    const Pos c = s_made(r.b, r.mv[i], r.piece[i], t);
+    const Pos c = uniform_pos(made(r.b, r.mv[i], r.piece[i], t));
+    const u32 n = wave_words<V>(c, t, list);
+    wave_sync();
     if (threadIdx.x == 0) {
-        count = generate_words<V>(c, t, word, 256, 0);
         if (blockIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
-        if (part == 0) atomicAdd(&P->paths[2], (u64)count);
+        if (part == 0) atomicAdd(&P->paths[2], (u64)n);
     }
-    __syncthreads();
-    const u32 n = count < 256 ? count : 256;
     *lo = n * part / parts;
     *hi = n * (part + 1) / parts;
     return c;
 }
 
-// perft(4): the fused leaf over the root's grandchildren, dealt to the waves
-constexpr u32 S_FOUR_PARTS = 4, S_TOP_PARTS = 2;
+// perft(4): a wave per board of ply 2 (a few where a child has many moves)
+constexpr u32 S_FOUR_PARTS = 8, S_TOP_PARTS = 8;
 template <int V>
-__global__ PG_LEAF_BOUNDS void ks_four(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ LeafTile s[S_WAVES];
-    __shared__ u32 word[256];
+__global__ __launch_bounds__(LEAF_WG) void ks_four(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
+    __shared__ u32 child[S_WAVES][256], list[S_WAVES][256];
     SSum sum;
+    const u32 wave = wave_number();
     u32 lo, hi;
-    const Pos c = s_child_moves<V>(word, r, P, S_FOUR_PARTS, &lo, &hi, t);
-    const u32 wave = wave_number(), j = lo + (threadIdx.x & 63) * S_WAVES + wave;
-    const bool live = j < hi;
-    Pos b{};
-    if (live) b = s_made(c, (u16)word[j], piece_code(word[j] >> 24), t);
-    s_leaf_tile<V>(s[wave], live, b, sum, &P->err, t);
+    const Pos c = s_child_moves<V>(child[wave], r, P, S_FOUR_PARTS, &lo, &hi, t);
+    for (u32 j = lo + wave; j < hi; j += S_WAVES) {
+        u32 moves;
+        sum.total += wave_perft2<V>(wave_made(c, child[wave], j, t), list[wave], &moves, t);
+        if ((threadIdx.x & 63) == 0) {
+            sum.items += moves;
+            sum.paths += moves;
+        }
+    }
     s_finish(P, sum, 4, bias, out, seq);
 }
 
-// plies 1 to 3 of a deeper search: the nodes of ply 2 and the list of ply 3
+// plies 1 to 3 of a deeper search: the nodes of ply 2 and the list of ply 3,
+// a wave per board of ply 2
 template <int V>
 __global__ __launch_bounds__(LEAF_WG) void ks_top(SRoot r, SPlan *P, SRegion rg, Tables t) {
-    __shared__ ListTile s;
-    __shared__ u32 word[256];
-    __shared__ u32 first;
-    SSum sum;
+    __shared__ u32 child[S_WAVES][256], list[S_WAVES][256];
+    __shared__ u32 first, count[S_WAVES];
+    __shared__ u64 base;
+    const u32 wave = wave_number(), lane = threadIdx.x & 63;
     u32 lo, hi;
-    const Pos c = s_child_moves<V>(word, r, P, S_TOP_PARTS, &lo, &hi, t);
+    const Pos c = s_child_moves<V>(child[wave], r, P, S_TOP_PARTS, &lo, &hi, t);
     const SLevel L = s_level(rg, 2, 0);
-    const u32 n = hi - lo, j = lo + threadIdx.x;
-    const bool live = j < hi;
-    if (threadIdx.x == 0) first = (u32)atomicAdd(&P->nNode[2], (u64)n);
+    u64 paths = 0;
+    if (threadIdx.x == 0) first = lo < hi ? (u32)atomicAdd(&P->nNode[2], (u64)(hi - lo)) : 0;
     __syncthreads();
-    if (first + n > rg.node2) {  // cannot happen: node2 is the root's moves times the most a position has
+    if (first + (hi - lo) > rg.node2) {  // cannot happen: node2 is the root's moves times the most a position has
         if (threadIdx.x == 0) P->overflow = 1;
         return;
     }
-    Pos b{};
-    if (live) {
-        b = s_made(c, (u16)word[j], piece_code(word[j] >> 24), t);
-        L.node[first + threadIdx.x] = SNode{b, 1, S_NO_SLOT, 0};
+    for (u32 j0 = lo; j0 < hi; j0 += S_WAVES) {
+        const u32 j = j0 + wave, node = first + j - lo;
+        u32 m = 0;
+        if (j < hi) {
+            const Pos b = wave_made(c, child[wave], j, t);
+            m = wave_words<V>(b, t, list[wave]);
+            if (lane == 0) L.node[node] = SNode{b, 1, S_NO_SLOT, 0};
+        }
+        if (lane == 0) count[wave] = m;
+        __syncthreads();
+        u32 before = 0, total = 0;
+        for (u32 w = 0; w < S_WAVES; w++) {
+            if (w < wave) before += count[w];
+            total += count[w];
+        }
+        if (threadIdx.x == 0) {
+            base = atomicAdd(&P->nList[3], (u64)total);
+            if (base + total > L.cap) P->overflow = 1;
+        }
+        __syncthreads();
+        if (base + total <= L.cap)
+            for (u32 k = lane; k < m; k += 64) {
+                const u32 w = list[wave][k];
+                L.mv[base + before + k] = (u16)w;
+                L.par[base + before + k] = node | (u32)piece_code(w >> 24) << S_NODE_BITS;
+            }
+        paths += total;
+        __syncthreads();
     }
-    s_list_tile<V>(s, live, b, 1, first, &P->nList[3], L, P, sum, t);
-    s_add(&P->paths[3], sum.paths, &P->overflow);
+    if (threadIdx.x == 0 && paths) atomicAdd(&P->paths[3], paths);
 }
 
 // empties the set of ply l (whose size follows from its list)
@@ -463,7 +489,7 @@ static __global__ __launch_bounds__(S_COLLAPSE_WG) void ks_collapse(SPlan *P, SR
             const u16 mv = L.mv[i];
             const SNode &p = L.node[par & S_NODE_MAX];
             nd.w = p.w;
-            nd.b = s_made(p.b, mv, (int)(par >> S_NODE_BITS), t);
+            nd.b = made(p.b, mv, (int)(par >> S_NODE_BITS), t);
             const u64 h = s_hash(nd.b);
             const u64 id = (h << 48) | (u64)mv << 32 | par;
             at = __umul64hi(h, slots);
@@ -567,17 +593,19 @@ __global__ PG_LEAF_BOUNDS void ks_leaf(SPlan *P, SRegion rg, int depth, u64 bias
         const SLevel A = s_level(rg, l - 1, uniform64(P->nNode[l - 1]));
         const u64 n = uniform64(LIST ? P->nList[l] : P->nNode[l]);
         SNode *node = (SNode *)rg.half[l & 1];
-        const u32 T = s_tile_boards(n, waves, 4, LEAF_TILE);
-        // the first tiles are dealt out, the others taken as waves get done
+        const u32 T = leaf_tile_boards(n, waves);
+        // the first tiles are dealt out, the others (if any) taken as waves
+        // get done: 3072 waves that ask for one at once wait 18 us
+        const bool more = (u64)waves * T < n;
         for (u64 tile = blockIdx.x * S_WAVES + wave; tile * T < n;) {
             u32 next = 0;
-            if (lane == 0) next = atomicAdd(&P->tile, 1u) + waves;
+            if (more && lane == 0) next = atomicAdd(&P->tile, 1u) + waves;
             const u64 i = tile * T + lane;
             const bool live = lane < T && i < n;
             Pos b{};
             u64 w;
             if (live) b = s_board<LIST, false>(rg, A, node, i, &w, t);
-            tile = (u32)__builtin_amdgcn_readfirstlane((int)next);
+            tile = more ? (u32)__builtin_amdgcn_readfirstlane((int)next) : n;
             const u32 c = leaf_expand<V>(s, live, b, &P->err, t);
             w = 0;
             if (live) w = s_weight<LIST>(A, node, i);  // again: there is no register to keep it in

@@ -53,7 +53,7 @@ static void launch(Engine &e, const Single &s, const SRoot &r, const SRegion &rg
     if (depth <= 2) {
         ks_one<V><<<1, LEAF_WG, 0, st>>>(r, s.plan, depth, bias, s.res, s.seq, e.dt);
     } else if (depth == 3 || r.n == 0) {
-        const int g = r.n ? (r.n + S_SMALL_TILE * S_WAVES - 1) / (S_SMALL_TILE * S_WAVES) : 1;
+        const int g = r.n ? (r.n + S_WAVES - 1) / S_WAVES : 1;
         ks_three<V><<<g, LEAF_WG, 0, st>>>(r, s.plan, bias, s.res, s.seq, e.dt);
     } else if (depth == 4) {
         ks_four<V><<<r.n * S_FOUR_PARTS, LEAF_WG, 0, st>>>(r, s.plan, bias, s.res, s.seq, e.dt);
