@@ -45,7 +45,20 @@ struct Plan {
     u32 ovf;            // a 64-bit total wrapped
     u64 peak;           // highest bump top reached (bytes of the region used)
     u64 liveN;          // entries of the leaf level's live list
+    u64 began;          // device clock at the search's start
     DLevel lv[TT_MAX_DEPTH];
+};
+
+// A search's inputs and results in pinned host memory, which its first and
+// last kernels read and write themselves: copies on the stream cost 8 to 10 us
+// each, of which a search would need five.
+struct Link {
+    Plan plan;          // as the search begins; the last kernel updates the counters
+    const Pos *b;       // roots and keys (null: already on the device)
+    const Key128 *k;
+    u64 *out;           // the roots' perfts (null: left on the device)
+    u64 ticks;          // device clock ticks from the first kernel to the last
+    u64 want, seq;      // seq = want is written last
 };
 
 __device__ __forceinline__ void *plan_alloc(Plan *P, u64 bytes) {
@@ -70,18 +83,33 @@ __device__ __forceinline__ void *plan_try_alloc(Plan *P, u64 bytes) {
 
 #define PG_GRID_LOOP_N(i, n) PG_GRID_LOOP(i, n)
 
-// level-0 move counts (deeper levels get them from expansion)
+// The first kernel: the plan and the roots come from the host, the roots are
+// counted (deeper levels get their counts from the expansion) and the table
+// of depth D is probed: hits are resolved before the expansion.
 template <int V>
-__global__ __launch_bounds__(wg_size<V>()) void kd_count(Plan *P, Tables t) {
+__global__ __launch_bounds__(wg_size<V>()) void kd_begin(Plan *P, const Link *H, TTView tt, int D, TTCounters *ctr,
+                                                         int small, Tables t) {
     stage_tables<V>(t);
-    const DLevel L = P->lv[0];
-    PG_GRID_LOOP(i, L.n) L.cnt[i] = count_any<V>(L.b[i], t);
-}
-
-// roots: probe the table of depth D; hits are resolved before expansion
-static __global__ __launch_bounds__(256) void kd_root_probe(Plan *P, TTView tt, int D, TTCounters *ctr) {
-    const DLevel L = P->lv[0];
+    if (blockIdx.x == 0) {
+        const u64 *from = (const u64 *)&H->plan;
+        for (u32 i = threadIdx.x; i < sizeof(Plan) / 8; i += blockDim.x) ((u64 *)P)[i] = from[i];
+        __syncthreads();
+        if (threadIdx.x == 0) P->began = wall_clock64();
+    }
+    const DLevel L = H->plan.lv[0];
+    const u64 bias = H->plan.bias;
+    const Pos *const hb = H->b;
+    const Key128 *const hk = H->k;
     PG_GRID_LOOP(i, L.n) {
+        const Pos b = hb ? hb[i] : L.b[i];
+        if (hb) {
+            L.b[i] = b;
+            if (L.k) L.k[i] = hk[i];
+        }
+        if (small) {
+            L.perft[i] = bias;
+            continue;
+        }
         u64 v = 0;
         const bool probe = D >= 2 && tt.base[D] && L.k;
         const bool hit = probe && tt_probe(tt, D, L.k[i], &v);
@@ -93,8 +121,36 @@ static __global__ __launch_bounds__(256) void kd_root_probe(Plan *P, TTView tt, 
         // the same input; a hit is recorded in state/perft and expands to nothing
         L.state[i] = hit ? ST_HIT : ST_LIVE;
         L.perft[i] = v;
-        if (hit) L.cnt[i] = 0;
+        L.cnt[i] = hit ? 0 : count_any<V>(b, t);
     }
+}
+
+// The last kernel, one work-group: results and counters to the host.
+static __global__ __launch_bounds__(1024) void kd_end(const Plan *P, Link *H) {
+    const DLevel L = P->lv[0];
+    u64 *const out = H->out;
+    if (out)
+        for (u64 i = threadIdx.x; i < L.n; i += blockDim.x) out[i] = L.perft[i];
+    if (threadIdx.x == 0) {
+        Plan &h = H->plan;
+        h.overflow = P->overflow;
+        h.err = P->err;
+        h.ovf = P->ovf;
+        h.leafItems = P->leafItems;
+        h.peak = P->peak;
+        H->ticks = wall_clock64() - P->began;
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(&H->seq, H->want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// level-0 move counts of a total-only search
+template <int V>
+__global__ __launch_bounds__(wg_size<V>()) void kd_count(Plan *P, Tables t) {
+    stage_tables<V>(t);
+    const DLevel L = P->lv[0];
+    PG_GRID_LOOP(i, L.n) L.cnt[i] = count_any<V>(L.b[i], t);
 }
 
 static __global__ __launch_bounds__(256) void kd_root_store(Plan *P, TTView tt, int D, TTCounters *ctr) {
@@ -464,6 +520,129 @@ __global__ PG_LEAF_BOUNDS void kd_leaf_keys(
     leaf_tiles<V, true, true>(A.b, nullptr, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft,
                               listed ? nullptr : L.state, 0, &P->err, &P->ovf, t, listed ? L.live : nullptr, A.par,
                               A.mv);
+}
+
+// Small searches without a table (depth 3 or 4): no levels in memory.  A wave
+// takes a part of a root's moves, lists the boards of ply D-2 below them, a
+// tile at a time (wave_words lists one board's moves), and hands the tile to
+// the fused leaf; kd_begin has set the results to the bias.  What the level
+// loop spends on such a search is mostly its kernels of 3 to 5 us each, ten
+// per level.
+// The same for so few roots that every board of ply D-2 can have a wave of its
+// own (wave_perft2).
+template <int V, int D>
+__global__ __launch_bounds__(LEAF_WG) void kd_tiny(Plan *P, Tables t) {
+    constexpr u32 WAVES = LEAF_WG / 64, PARTS = 32;
+    __shared__ u32 list[WAVES][3][256];
+    __shared__ u32 items;
+    const u32 wave = wave_number(), lane = threadIdx.x & 63;
+    u32(&ls)[3][256] = list[wave];
+    if (threadIdx.x == 0) items = 0;
+    __syncthreads();
+    const DLevel L = P->lv[0];
+    const u64 units = uniform64(L.n) * (D == 3 ? PARTS : PARTS * PARTS);
+    u32 listed = 0;
+    for (u64 u = blockIdx.x * WAVES + wave; u < units; u += gridDim.x * WAVES) {
+        const u64 ri = u / (units / L.n);
+        const u32 part = (u32)(u % PARTS), part2 = (u32)(u / PARTS % PARTS);
+        const Pos root = uniform_pos(L.b[ri]);
+        const u32 n = wave_words<V>(root, t, ls[0]);
+        wave_sync();
+        u32 sum = 0, moves;
+        for (u32 i = part; i < n; i += PARTS) {
+            const Pos c = wave_made(root, ls[0], i, t);
+            if constexpr (D == 3) {
+                sum += wave_perft2<V>(c, ls[1], &moves, t);
+                listed += moves;
+            } else {
+                const u32 m = wave_words<V>(c, t, ls[1]);
+                wave_sync();
+                for (u32 j = part2; j < m; j += PARTS) {
+                    sum += wave_perft2<V>(wave_made(c, ls[1], j, t), ls[2], &moves, t);
+                    listed += moves;
+                }
+            }
+        }
+        sum = wave_sum32(sum);
+        if (lane == 0 && sum) add_checked(&P->lv[0].perft[ri], sum, &P->ovf);
+        wave_sync();
+    }
+    if (lane == 0) atomicAdd(&items, listed);
+    __syncthreads();
+    if (threadIdx.x == 0 && items) atomicAdd(&P->leafItems, (u64)items);
+}
+
+template <int V, int D>
+__global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(2, 8))) void kd_small(Plan *P, Tables t) {
+    static_assert(D == 3 || D == 4, "two plies end in the leaf");
+    constexpr u32 WAVES = LEAF_WG / 64, MOST = D == 3 ? 8 : 32;
+    __shared__ LeafTile tiles[WAVES];
+    const u32 wave = wave_number(), lane = threadIdx.x & 63;
+    LeafTile &s = tiles[wave];
+    const u64 n = uniform64(P->lv[0].n);
+    const u32 waves = gridDim.x * WAVES < LEAF_RESIDENT ? gridDim.x * WAVES : LEAF_RESIDENT;
+    u32 parts = 1;
+    while (parts < MOST && n * parts * 2 <= waves) parts *= 2;
+    u64 items = 0;
+    for (u64 u = blockIdx.x * WAVES + wave; u < n * parts; u += gridDim.x * WAVES) {
+        const u64 ri = u / parts;
+        const u32 part = (u32)(u % parts);
+        // read again for each listing: no registers to keep it in
+        const Pos *const rp = P->lv[0].b + ri;
+        u32 lo = 0, hi = 1, mine = 0, at = 0;
+        u32 chunk = 0, rootMoves = 0;  // D == 4: the part's moves, 64 at a time, one in each lane
+        do {
+            if (D == 4) {
+                rootMoves = wave_words<V>(opaque_pos(uniform_pos(*rp)), t, s.word);
+                wave_sync();
+                lo = rootMoves * part / parts + chunk;
+                hi = rootMoves * (part + 1) / parts;
+                if (lo + lane < hi) mine = s.word[lo + lane];
+                wave_sync();
+                if (hi > lo + 64) hi = lo + 64;
+                hi = hi > lo ? hi - lo : 0;
+                lo = 0;
+            }
+            // lo: the next board to list, at: its next move
+            for (;;) {
+                u32 fill = 0;
+                Pos b{};
+                while (fill < 64 && lo < hi) {
+                    Pos p = opaque_pos(uniform_pos(*rp));
+                    if (D == 4) {
+                        const u32 w = (u32)__builtin_amdgcn_readlane((int)mine, (int)lo);
+                        p = made(p, (u16)w, piece_code(w >> 24), t);
+                    }
+                    u32 m = wave_words<V>(p, t, s.word);
+                    wave_sync();
+                    if (D == 3) {
+                        if (at == 0) at = m * part / parts;
+                        m = m * (part + 1) / parts;
+                    }
+                    const u32 take = m - at < 64 - fill ? m - at : 64 - fill;
+                    if (lane >= fill && lane < fill + take) {
+                        const u32 w = s.word[at + lane - fill];
+                        b = made(p, (u16)w, piece_code(w >> 24), t);
+                    }
+                    wave_sync();
+                    fill += take;
+                    at += take;
+                    if (at >= m) {
+                        lo++;
+                        at = 0;
+                    }
+                }
+                if (!fill) break;
+                const u32 c = leaf_expand<V>(s, lane < fill, b, &P->err, t);
+                items += wave_sum32(c);
+                const u32 sum = wave_sum32(lane < fill ? s.per[lane] : 0);
+                if (lane == 0) add_checked(&P->lv[0].perft[ri], sum, &P->ovf);
+                wave_sync();
+            }
+            chunk += 64;
+        } while (D == 4 && rootMoves * part / parts + chunk < rootMoves * (part + 1) / parts);
+    }
+    if (lane == 0 && items) atomicAdd(&P->leafItems, items);
 }
 
 // the plan's total += the move counts of level l (perft(1) of a total-only search)

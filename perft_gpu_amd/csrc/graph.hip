@@ -26,11 +26,25 @@ struct GraphShape {
     int total;  // 1: one root, only the sum is wanted (no per-board perft arrays)
     int cap;    // > 0: at most this many work-groups per CU in every kernel (leaves CUs to other streams)
     int gmax;   // > 0: at most this many work-groups in any kernel (a small search's whole need)
+    int leafMax;  // the same for the leaf, whose waves take a few boards each
+    int small;  // searched without levels in memory: 1 kd_small, 2 kd_tiny
     bool operator==(const GraphShape &o) const {
         return depth == o.depth && v == o.v && keys == o.keys && dedup == o.dedup && bpc == o.bpc && tt == o.tt &&
-               total == o.total && cap == o.cap && gmax == o.gmax;
+               total == o.total && cap == o.cap && gmax == o.gmax && leafMax == o.leafMax && small == o.small;
     }
 };
+
+// Whether n roots to `depth` are searched without levels in memory.  Measured
+// time of the graph in us, level loop / kd_small / kd_tiny: depth 3, 1 root
+// 79 / 34 / 21, 16 roots 98 / 39 / 25, 61 roots 111 / 38 / 28, 250 roots 127 /
+// 40 / -, 1000 roots 152 / 57 / -, 4096 roots 205 / 235 / -; depth 4, 1 root
+// 122 / 83 / 38, 4 roots 151 / 124 / 76, 61 roots 231 / 149 / -, 250 roots
+// 357 / 405 / -.
+static int small_search(u64 n, int depth, int v, const TTable *tt) {
+    if (tt || v == SL_BYTE || (depth != 3 && depth != 4)) return 0;
+    if (n <= (depth == 3 ? 128 : 6)) return 2;
+    return n <= (depth == 3 ? 1536 : 96);
+}
 
 // The most work-groups any kernel of a search of n roots to `depth` can use:
 // its largest materialized level holds at most about n * 48^(depth-2)
@@ -65,7 +79,7 @@ static Grids grids_for(const Engine &e, const GraphShape &sh) {
         g.work = std::min(g.work, sh.gmax);
         g.scan = std::min(g.scan, sh.gmax);
         g.byteV = std::min(g.byteV, sh.gmax);
-        g.leaf = std::min(g.leaf, sh.gmax);
+        g.leaf = std::min(g.leaf, sh.leafMax);
     }
     g.v = sh.v == SL_BYTE ? g.byteV : g.work;
     return g;
@@ -76,19 +90,38 @@ struct BatchGraph {
     hipGraphExec_t exec = nullptr;
 };
 
+// the leaf's work-groups for a search that does not fill the chip: a wave
+// takes 4 boards and more, or (kd_tiny) one
+static int leaf_need(const GraphShape &sh) { return sh.gmax * (sh.small == 2 ? 16 : 4); }
+
+// the graph of a served batch
+static GraphShape server_shape(const Engine &e, const TTable *tt, u64 n, int depth, int v, int dedup, int wgCap) {
+    const int g = grid_limit(e, n, depth);
+    GraphShape sh{depth, v, 1, dedup ? 1 : 0, e.bpc, tt, 0, wgCap, g, 0, small_search(n, depth, v, tt)};
+    sh.leafMax = leaf_need(sh);
+    return sh;
+}
+
 // One batch slot: a plan in device memory and the arena region it carves.
 struct Slot {
     Plan *dPlan = nullptr;
-    Plan *hPlan = nullptr;  // pinned staging copy
+    Link *link = nullptr;   // pinned: the plan's staging copy, inputs and results
+    u64 seq = 0;
+    u8 *stage = nullptr;    // pinned: roots, keys and results of a batch
+    size_t stageBytes = 0;
+    double tickMs = 0;      // length of a device clock tick
     u8 *region = nullptr;
     size_t regionBytes = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<BatchGraph> graphs;
 };
 
 template <int V> static void cap_count(hipStream_t s, Plan *P, int g, const Tables &t) {
     kd_count<V><<<g, wg_size<V>(), 0, s>>>(P, t);
+}
+template <int V> static void cap_begin(hipStream_t s, Plan *P, const Link *H, const TTView &tt, int D, TTCounters *ctr,
+                                       int small, int g, const Tables &t) {
+    kd_begin<V><<<g, wg_size<V>(), 0, s>>>(P, H, tt, D, ctr, small, t);
 }
 template <int V> static void cap_generate(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
     kd_generate<V><<<g, wg_size<V>(), 0, s>>>(P, l, t);
@@ -106,6 +139,15 @@ template <int V> static void cap_expand_keys(hipStream_t s, Plan *P, int l, cons
 }
 template <int V> static void cap_leaf_keys(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
     if constexpr (V != SL_BYTE) kd_leaf_keys<V><<<g, LEAF_WG, 0, s>>>(P, l, t);
+}
+
+template <int V> static void cap_small(hipStream_t s, Plan *P, int depth, int tiny, int g, const Tables &t) {
+    if constexpr (V != SL_BYTE) {
+        if (tiny && depth == 3) kd_tiny<V, 3><<<g, LEAF_WG, 0, s>>>(P, t);
+        else if (tiny) kd_tiny<V, 4><<<g, LEAF_WG, 0, s>>>(P, t);
+        else if (depth == 3) kd_small<V, 3><<<g, LEAF_WG, 0, s>>>(P, t);
+        else kd_small<V, 4><<<g, LEAF_WG, 0, s>>>(P, t);
+    }
 }
 
 // The search of one root when only its perft is wanted, for the byte-lookup
@@ -128,7 +170,7 @@ static void enqueue_total(const Engine &e, hipStream_t s, Plan *P, const GraphSh
 }
 
 // Enqueues the whole search for `depth` on stream s (captured by the caller).
-static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, const GraphShape &sh) {
+static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, Link *H, const GraphShape &sh) {
     const int D = sh.depth, v = sh.v;
     const Grids G = grids_for(e, sh);
     const int gWork = G.work, gScan = G.scan, gLeaf = G.leaf, gv = G.v;
@@ -138,8 +180,12 @@ static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, const GraphS
         tt = sh.tt->view;
         ctr = sh.tt->dCtr;
     }
-    PG_VARIANT_CALL(v, cap_count, s, P, gv, e.dt);
-    kd_root_probe<<<gWork, 256, 0, s>>>(P, tt, D, ctr);
+    PG_VARIANT_CALL(v, cap_begin, s, P, H, tt, D, ctr, sh.small, gv, e.dt);
+    if (sh.small) {
+        PG_VARIANT_CALL(v, cap_small, s, P, D, sh.small == 2, gLeaf, e.dt);
+        kd_end<<<1, 1024, 0, s>>>(P, H);
+        return;
+    }
     // levels expanded into children: remaining depth r = D - l >= 3, or >= 2
     // for the byte-lookup variant (no fused leaf, LDS is taken by its tables)
     const int lastExpand = v == SL_BYTE ? D - 2 : D - 3;
@@ -184,7 +230,8 @@ static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, const GraphS
         kd_resolve<<<gWork, 256, 0, s>>>(P, l, tt, D - l - 1, ctr);
         kd_segsum<<<gWork, 256, 0, s>>>(P, l);
     }
-    kd_root_store<<<gWork, 256, 0, s>>>(P, tt, D, ctr);
+    if (sh.tt) kd_root_store<<<gWork, 256, 0, s>>>(P, tt, D, ctr);
+    kd_end<<<1, 1024, 0, s>>>(P, H);
 }
 
 static int get_graph(Engine &e, Slot &sl, const GraphShape &sh, hipGraphExec_t *out) {
@@ -196,7 +243,7 @@ static int get_graph(Engine &e, Slot &sl, const GraphShape &sh, hipGraphExec_t *
     hipGraph_t graph;
     HIP_TRY(hipStreamBeginCapture(sl.stream, hipStreamCaptureModeThreadLocal));
     if (sh.total) enqueue_total(e, sl.stream, sl.dPlan, sh);
-    else enqueue_search(e, sl.stream, sl.dPlan, sh);
+    else enqueue_search(e, sl.stream, sl.dPlan, sl.link, sh);
     HIP_TRY(hipStreamEndCapture(sl.stream, &graph));
     hipGraphExec_t exec;
     HIP_TRY(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
@@ -206,11 +253,29 @@ static int get_graph(Engine &e, Slot &sl, const GraphShape &sh, hipGraphExec_t *
     return PG_OK;
 }
 
-// Runs one batch (sub-range of the level-0 arrays already on the device);
-// sets *overflow if it did not fit.
-static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n, const DLevel &L0, size_t top0,
-                     bool *overflow, u64 *leafItems, double *ms, u64 *peak) {
-    Plan &h = *sl.hPlan;
+// Waits until the search launched last on the slot has handed its results
+// over: the host sees them sooner than the stream's end; a long search is
+// waited for by the stream.
+static int wait_slot(Slot &sl) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (u32 spin = 0;; spin++) {
+        if (__atomic_load_n(&sl.link->seq, __ATOMIC_ACQUIRE) == sl.seq) return PG_OK;
+        if (spin % 64 == 63 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(500)) break;
+    }
+    HIP_TRY(hipStreamSynchronize(sl.stream));
+    if (__atomic_load_n(&sl.link->seq, __ATOMIC_ACQUIRE) == sl.seq) return PG_OK;
+    set_error("batch: the search ended without a result");
+    return PG_EHIP;
+}
+
+// Fills the slot's link for n roots at L0 and launches the search.
+static int launch_search(Engine &e, Slot &sl, const GraphShape &sh, u64 n, const DLevel &L0, size_t top0, const Pos *b,
+                         const Key128 *k, u64 *out) {
+    hipGraphExec_t exec;
+    const int rc = get_graph(e, sl, sh, &exec);
+    if (rc) return rc;
+    Link &H = *sl.link;
+    Plan &h = H.plan;
     memset(&h, 0, sizeof(Plan));
     h.base = sl.region;
     h.cap = sl.regionBytes;
@@ -218,24 +283,39 @@ static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
     h.bias = e.bias;
     h.lv[0] = L0;
     h.lv[0].n = n;
-    h.lv[0].b += first;
-    if (h.lv[0].k) h.lv[0].k += first;
-    h.lv[0].cnt += first;
-    h.lv[0].perft += first;
-    h.lv[0].state += first;
-    h.lv[0].dup += first;
-    hipGraphExec_t exec;
-    int rc = get_graph(e, sl, sh, &exec);
-    if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(sl.dPlan, &h, sizeof(Plan), hipMemcpyHostToDevice, sl.stream));
-    HIP_TRY(hipEventRecord(sl.ev0, sl.stream));
+    H.b = b;
+    H.k = k;
+    H.out = out;
+    H.want = ++sl.seq;
     HIP_TRY(hipGraphLaunch(exec, sl.stream));
-    HIP_TRY(hipEventRecord(sl.ev1, sl.stream));
-    HIP_TRY(hipMemcpyAsync(&h, sl.dPlan, sizeof(Plan), hipMemcpyDeviceToHost, sl.stream));
-    HIP_TRY(hipStreamSynchronize(sl.stream));
-    float t = 0;
-    (void)hipEventElapsedTime(&t, sl.ev0, sl.ev1);
-    *ms += t;
+    return PG_OK;
+}
+
+// A batch's inputs and results on the host, in the order of the level-0
+// arrays (null: copied over already, results left there).
+struct Staged {
+    const Pos *b = nullptr;
+    const Key128 *k = nullptr;
+    u64 *out = nullptr;
+};
+
+// Runs one batch (sub-range of the level-0 arrays; in.b: to be filled from
+// there); sets *overflow if it did not fit.
+static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n, const DLevel &L0, size_t top0,
+                     const Staged &in, bool *overflow, u64 *leafItems, double *ms, u64 *peak) {
+    DLevel L = L0;
+    L.b += first;
+    if (L.k) L.k += first;
+    L.cnt += first;
+    L.perft += first;
+    L.state += first;
+    L.dup += first;
+    int rc = launch_search(e, sl, sh, n, L, top0, in.b ? in.b + first : nullptr, in.k ? in.k + first : nullptr,
+                           in.out ? in.out + first : nullptr);
+    if (!rc) rc = wait_slot(sl);
+    if (rc) return rc;
+    const Plan &h = sl.link->plan;
+    *ms += (double)sl.link->ticks * sl.tickMs;
     *overflow = h.overflow != 0;
     *leafItems += h.leafItems;
     if (h.peak > *peak) *peak = h.peak;
@@ -251,10 +331,10 @@ static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
 }
 
 static int run_split(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n, const DLevel &L0, size_t top0,
-                     u64 *leafItems, double *ms, u64 *launches, u64 *splits, u64 *peak) {
+                     const Staged &in, u64 *leafItems, double *ms, u64 *launches, u64 *splits, u64 *peak) {
     bool over = false;
     (*launches)++;
-    int rc = run_range(e, sl, sh, first, n, L0, top0, &over, leafItems, ms, peak);
+    int rc = run_range(e, sl, sh, first, n, L0, top0, in, &over, leafItems, ms, peak);
     if (rc) return rc;
     if (!over) return PG_OK;
     if (n == 1) {
@@ -263,9 +343,10 @@ static int run_split(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
     }
     (*splits)++;
     const u64 h = n / 2;
-    rc = run_split(e, sl, sh, first, h, L0, top0, leafItems, ms, launches, splits, peak);
+    const Staged rest{nullptr, nullptr, in.out};  // the roots are on the device now
+    rc = run_split(e, sl, sh, first, h, L0, top0, rest, leafItems, ms, launches, splits, peak);
     if (rc) return rc;
-    return run_split(e, sl, sh, first + h, n - h, L0, top0, leafItems, ms, launches, splits, peak);
+    return run_split(e, sl, sh, first + h, n - h, L0, top0, rest, leafItems, ms, launches, splits, peak);
 }
 
 int slot_init(Engine &e, Slot &sl, u8 *region, size_t bytes, hipStream_t stream) {
@@ -273,10 +354,11 @@ int slot_init(Engine &e, Slot &sl, u8 *region, size_t bytes, hipStream_t stream)
     sl.regionBytes = bytes;
     sl.stream = stream;
     HIP_TRY(hipMalloc(&sl.dPlan, sizeof(Plan)));
-    HIP_TRY(hipHostMalloc(&sl.hPlan, sizeof(Plan)));
-    HIP_TRY(hipEventCreate(&sl.ev0));
-    HIP_TRY(hipEventCreate(&sl.ev1));
-    (void)e;
+    HIP_TRY(hipHostMalloc(&sl.link, sizeof(Link)));
+    memset(sl.link, 0, sizeof(Link));
+    int khz = 0;
+    HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e.device));
+    sl.tickMs = khz > 0 ? 1.0 / khz : 0;
     return PG_OK;
 }
 
@@ -284,9 +366,8 @@ void slot_free(Slot &sl) {
     for (auto &g : sl.graphs) (void)hipGraphExecDestroy(g.exec);
     sl.graphs.clear();
     if (sl.dPlan) (void)hipFree(sl.dPlan);
-    if (sl.hPlan) (void)hipHostFree(sl.hPlan);
-    if (sl.ev0) (void)hipEventDestroy(sl.ev0);
-    if (sl.ev1) (void)hipEventDestroy(sl.ev1);
+    if (sl.link) (void)hipHostFree(sl.link);
+    if (sl.stage) (void)hipHostFree(sl.stage);
     sl = Slot();
 }
 
@@ -319,7 +400,7 @@ int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fi
         if (rc) return rc;
     }
     Slot &sl = *e.batchSlot;
-    Plan &h = *sl.hPlan;
+    Plan &h = sl.link->plan;
     memset(&h, 0, sizeof(Plan));
     h.base = sl.region;
     h.cap = sl.regionBytes;
@@ -329,7 +410,8 @@ int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fi
     h.lv[0].cnt = (u32 *)(sl.region + 256);
     h.top = 512;
     h.acc = e.bias;
-    GraphShape sh{(int)depth, v, 0, 0, e.bpc, nullptr, 1, 0, grid_limit(e, 1, (int)depth)};
+    const int g = grid_limit(e, 1, (int)depth);
+    GraphShape sh{(int)depth, v, 0, 0, e.bpc, nullptr, 1, 0, g, g, 0};
     hipGraphExec_t exec;
     int rc = get_graph(e, sl, sh, &exec);
     if (rc) return rc;
@@ -355,6 +437,8 @@ int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fi
     return PG_OK;
 }
 
+constexpr u64 STAGE_ROOTS = 1 << 18;  // most roots staged in kept memory (18 MiB)
+
 // Batched perft of n roots on slot sl.  Results in out[] (host), in the
 // caller's order.
 int batch_perft(Engine &e, Slot &sl, TTable *tt, const Pos *roots, u64 n, u32 depth, int v, int dedup, int bpc,
@@ -373,8 +457,26 @@ int batch_perft(Engine &e, Slot &sl, TTable *tt, const Pos *roots, u64 n, u32 de
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](u64 a, u64 b) { return pos_side(roots[a]) < pos_side(roots[b]); });
     const bool keys = tt != nullptr || dedup;
-    std::vector<Pos> hb(n);
-    std::vector<Key128> hk(keys ? n : 0);
+    // roots, keys and results are staged in pinned memory, kept for later
+    // batches; a batch of very many roots brings its own
+    const size_t bytes = n * (sizeof(Pos) + sizeof(Key128) + 8);
+    std::vector<u8> own;
+    u8 *stage = sl.stage;
+    if (n > STAGE_ROOTS) {
+        own.resize(bytes);
+        stage = own.data();
+    } else if (bytes > sl.stageBytes) {
+        if (sl.stage) (void)hipHostFree(sl.stage);
+        sl.stage = nullptr;
+        sl.stageBytes = 0;
+        const size_t want = std::max<size_t>(2 * bytes, 64 << 10);
+        HIP_TRY(hipHostMalloc(&sl.stage, want));
+        sl.stageBytes = want;
+        stage = sl.stage;
+    }
+    Pos *const hb = reinterpret_cast<Pos *>(stage);
+    Key128 *const hk = reinterpret_cast<Key128 *>(stage + n * sizeof(Pos));
+    u64 *const res = reinterpret_cast<u64 *>(stage + n * (sizeof(Pos) + sizeof(Key128)));
     for (u64 i = 0; i < n; i++) {
         hb[i] = roots[order[i]];
         if (keys) hk[i] = zobrist128(hb[i], hv);
@@ -399,17 +501,26 @@ int batch_perft(Engine &e, Slot &sl, TTable *tt, const Pos *roots, u64 n, u32 de
         set_error("batch of %llu roots does not fit the region", (unsigned long long)n);
         return PG_ENOMEM;
     }
-    HIP_TRY(hipMemcpyAsync(L0.b, hb.data(), n * sizeof(Pos), hipMemcpyHostToDevice, sl.stream));
-    if (keys) HIP_TRY(hipMemcpyAsync(L0.k, hk.data(), n * sizeof(Key128), hipMemcpyHostToDevice, sl.stream));
+    Staged in;
+    if (own.empty()) {
+        in = Staged{hb, hk, res};
+    } else {
+        HIP_TRY(hipMemcpyAsync(L0.b, hb, n * sizeof(Pos), hipMemcpyHostToDevice, sl.stream));
+        if (keys) HIP_TRY(hipMemcpyAsync(L0.k, hk, n * sizeof(Key128), hipMemcpyHostToDevice, sl.stream));
+    }
+    // the default grid is the search's whole need; a set one holds for every kernel
+    const int gmax = e.batchGrid >= 0 ? e.batchGrid : grid_limit(e, n, (int)depth);
     GraphShape sh{(int)depth, v, keys ? 1 : 0, dedup ? 1 : 0, bpc > 0 ? bpc : e.bpc, tt, 0, 0,
-                  e.batchGrid >= 0 ? e.batchGrid : grid_limit(e, n, (int)depth)};
+                  gmax, 0, small_search(n, (int)depth, v, tt)};
+    sh.leafMax = e.batchGrid >= 0 ? gmax : leaf_need(sh);
     u64 leafItems = 0, launches = 0, splits = 0, peak = 0;
     double ms = 0;
-    int rc = run_split(e, sl, sh, 0, n, L0, top, &leafItems, &ms, &launches, &splits, &peak);
+    int rc = run_split(e, sl, sh, 0, n, L0, top, in, &leafItems, &ms, &launches, &splits, &peak);
     if (rc) return rc;
-    std::vector<u64> res(n);
-    HIP_TRY(hipMemcpyAsync(res.data(), L0.perft, n * 8, hipMemcpyDeviceToHost, sl.stream));
-    HIP_TRY(hipStreamSynchronize(sl.stream));
+    if (!own.empty()) {
+        HIP_TRY(hipMemcpyAsync(res, L0.perft, n * 8, hipMemcpyDeviceToHost, sl.stream));
+        HIP_TRY(hipStreamSynchronize(sl.stream));
+    }
     for (u64 i = 0; i < n; i++) out[order[i]] = res[i];
     if (bs) {
         bs->graph_ms = ms;
@@ -688,25 +799,8 @@ int pg::server_submit(Server &srv, uint32_t slot, const pg_pos48 *pos, uint32_t 
     L0.state = (u8 *)take(n);
     L0.dup = (u32 *)take(n * 4);
     if (!L0.dup) return PG_ENOMEM;
-    HIP_TRY(hipMemcpyAsync(L0.b, hb, n * sizeof(Pos), hipMemcpyHostToDevice, sl.stream));
-    HIP_TRY(hipMemcpyAsync(L0.k, hk, n * sizeof(Key128), hipMemcpyHostToDevice, sl.stream));
-    GraphShape sh{(int)depth, v, 1, dedup ? 1 : 0, e.bpc, s->tt, 0, wgCap, grid_limit(e, n, (int)depth)};
-    hipGraphExec_t exec;
-    int rc = get_graph(e, sl, sh, &exec);
+    const int rc = launch_search(e, sl, server_shape(e, s->tt, n, (int)depth, v, dedup, wgCap), n, L0, top, hb, hk, ss.hOut);
     if (rc) return rc;
-    Plan &h = *sl.hPlan;
-    memset(&h, 0, sizeof(Plan));
-    h.base = sl.region;
-    h.cap = sl.regionBytes;
-    h.top = top;
-    h.bias = e.bias;
-    h.lv[0] = L0;
-    HIP_TRY(hipMemcpyAsync(sl.dPlan, &h, sizeof(Plan), hipMemcpyHostToDevice, sl.stream));
-    HIP_TRY(hipEventRecord(sl.ev0, sl.stream));  // the batch's device time (pg_batch_stats.graph_ms)
-    HIP_TRY(hipGraphLaunch(exec, sl.stream));
-    HIP_TRY(hipEventRecord(sl.ev1, sl.stream));
-    HIP_TRY(hipMemcpyAsync(&h, sl.dPlan, sizeof(Plan), hipMemcpyDeviceToHost, sl.stream));
-    HIP_TRY(hipMemcpyAsync(ss.hOut, L0.perft, n * 8, hipMemcpyDeviceToHost, sl.stream));
     HIP_TRY(hipEventRecord(ss.done, sl.stream));
     ss.busy = true;
     ss.n = n;
@@ -735,7 +829,11 @@ int pg_server_poll(pg_server *s, uint32_t slot, uint64_t *out, pg_batch_stats *s
     ss.busy = false;
     Engine &e = *s->eng;
     Slot &sl = ss.slot;
-    const Plan &h = *sl.hPlan;
+    if (__atomic_load_n(&sl.link->seq, __ATOMIC_ACQUIRE) != sl.seq) {
+        set_error("served batch: the search ended without a result");
+        return PG_EHIP;
+    }
+    const Plan h = sl.link->plan;
     if (h.ovf) {
         set_error("served batch: a perft total does not fit 64 bits");
         return PG_EOVERFLOW;
@@ -745,19 +843,14 @@ int pg_server_poll(pg_server *s, uint32_t slot, uint64_t *out, pg_batch_stats *s
         return PG_EINVAL;
     }
     u64 items = h.leafItems, launches = 1, splits = 0, peak = h.peak;
-    float first = 0;
-    (void)hipEventElapsedTime(&first, sl.ev0, sl.ev1);  // read before a split reuses the events
-    double ms = first;
+    double ms = (double)sl.link->ticks * sl.tickMs;
     if (h.overflow) {
-        GraphShape sh{(int)ss.depth, ss.v, 1, ss.dedup ? 1 : 0, e.bpc, s->tt, 0, ss.wgCap,
-                      grid_limit(e, ss.n, (int)ss.depth)};
+        const GraphShape sh = server_shape(e, s->tt, ss.n, (int)ss.depth, ss.v, ss.dedup, ss.wgCap);
         (void)hipSetDevice(e.device);
         items = 0;
         launches = 0;
-        int rc = run_split(e, sl, sh, 0, ss.n, ss.L0, ss.top0, &items, &ms, &launches, &splits, &peak);
+        int rc = run_split(e, sl, sh, 0, ss.n, ss.L0, ss.top0, Staged{nullptr, nullptr, ss.hOut}, &items, &ms, &launches, &splits, &peak);
         if (rc) return rc;
-        HIP_TRY(hipMemcpyAsync(ss.hOut, ss.L0.perft, ss.n * 8, hipMemcpyDeviceToHost, sl.stream));
-        HIP_TRY(hipStreamSynchronize(sl.stream));
     }
     if (out)
         for (u64 i = 0; i < ss.n; i++) out[ss.order[i]] = ss.hOut[i];
@@ -782,17 +875,16 @@ int pg_server_prepare(pg_server *s, uint32_t depth, uint32_t max_roots, int slid
     const int v = slider == PG_SLIDER_AUTO ? e.slider : slider;
     if (v < 0 || v >= SL_COUNT) return PG_EINVAL;
     (void)hipSetDevice(e.device);
-    // the grids of the batch sizes 1..max_roots (grid_limit takes few values)
-    std::vector<int> limits;
+    // the shapes of the batch sizes 1..max_roots (few differ)
+    std::vector<pg::GraphShape> shapes;
     for (uint32_t n = 1; n <= max_roots; n++) {
-        const int g = grid_limit(e, n, (int)depth);
-        if (std::find(limits.begin(), limits.end(), g) == limits.end()) limits.push_back(g);
+        const pg::GraphShape sh = pg::server_shape(e, s->tt, n, (int)depth, v, dedup, (int)wg_per_cu);
+        if (std::find(shapes.begin(), shapes.end(), sh) == shapes.end()) shapes.push_back(sh);
     }
     uint32_t made = 0;
     for (auto &ss : s->slots) {
         if (ss.busy) continue;
-        for (const int g : limits) {
-            GraphShape sh{(int)depth, v, 1, dedup ? 1 : 0, e.bpc, s->tt, 0, (int)wg_per_cu, g};
+        for (const pg::GraphShape &sh : shapes) {
             const size_t before = ss.slot.graphs.size();
             hipGraphExec_t exec;
             const int rc = get_graph(e, ss.slot, sh, &exec);
