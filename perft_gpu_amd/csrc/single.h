@@ -61,9 +61,9 @@ struct SPlan {
     struct alignas(128) Bank {
         u64 acc, paths, items;          // of the last kernel; paths: of its ply
         u32 done;
+        u32 tile;                       // tiles of the bank taken
     } bank[S_BANKS];
     alignas(128) u32 done;              // banks that are complete
-    alignas(128) u32 tile;              // next tile of the last kernel
     alignas(128) u32 overflow, err, ovf;
 };
 
@@ -296,7 +296,7 @@ __device__ __forceinline__ void s_finish(SPlan *P, const SSum &sum, int depth, u
         paths = s_load(&L.paths);
         items = s_load(&L.items);
         L.acc = L.paths = L.items = 0;
-        L.done = 0;
+        L.done = L.tile = 0;
     }
     bool accWide = false, pathsWide = false;
     acc = s_wave_total(acc, &accWide);
@@ -315,7 +315,7 @@ __device__ __forceinline__ void s_finish(SPlan *P, const SSum &sum, int depth, u
         out->paths[l] = s_load(&P->paths[l]) + (l == depth - 1 ? paths : 0);
         P->nNode[l] = P->nList[l] = P->paths[l] = 0;
     }
-    P->overflow = P->err = P->ovf = P->done = P->tile = 0;
+    P->overflow = P->err = P->ovf = P->done = 0;
     __hip_atomic_store(&out->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -595,17 +595,21 @@ __global__ PG_LEAF_BOUNDS void ks_leaf(SPlan *P, SRegion rg, int depth, u64 bias
         SNode *node = (SNode *)rg.half[l & 1];
         const u32 T = leaf_tile_boards(n, waves);
         // the first tiles are dealt out, the others (if any) taken as waves
-        // get done: 3072 waves that ask for one at once wait 18 us
+        // get done, from as many counters as there are banks: with one, its
+        // atomics (12 ns each) were all that perft(8) from the start without
+        // merging waited for, 21.9 ms
+        const u32 banks = gridDim.x < S_BANKS ? gridDim.x : S_BANKS, bank = blockIdx.x % banks;
+        const u32 mine = ((gridDim.x - bank + banks - 1) / banks) * S_WAVES;  // the bank's waves
         const bool more = (u64)waves * T < n;
-        for (u64 tile = blockIdx.x * S_WAVES + wave; tile * T < n;) {
+        for (u64 tile = (u64)(blockIdx.x / banks * S_WAVES + wave) * banks + bank; tile * T < n;) {
             u32 next = 0;
-            if (more && lane == 0) next = atomicAdd(&P->tile, 1u) + waves;
+            if (more && lane == 0) next = atomicAdd(&P->bank[bank].tile, 1u) + mine;
             const u64 i = tile * T + lane;
             const bool live = lane < T && i < n;
             Pos b{};
             u64 w;
             if (live) b = s_board<LIST, false>(rg, A, node, i, &w, t);
-            tile = more ? (u32)__builtin_amdgcn_readfirstlane((int)next) : n;
+            tile = more ? (u64)(u32)__builtin_amdgcn_readfirstlane((int)next) * banks + bank : n;
             const u32 c = leaf_expand<V>(s, live, b, &P->err, t);
             w = 0;
             if (live) w = s_weight<LIST>(A, node, i);  // again: there is no register to keep it in
