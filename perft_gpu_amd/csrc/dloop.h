@@ -665,29 +665,26 @@ static __global__ __launch_bounds__(256) void kd_perft1(Plan *P, int l) {
     }
 }
 
-// level l+1 after its perfts are known: duplicates take their owner's value,
-// live children are stored (remaining depth rc)
-static __global__ __launch_bounds__(256) void kd_resolve(Plan *P, int l, TTView tt, int rc, TTCounters *ctr) {
-    const DLevel C = P->lv[l + 1];
-    if (P->overflow) return;
-    PG_GRID_LOOP(i, C.n) {
-        const u8 st = C.state[i];
-        bool stored = false;
-        if (st == ST_DUP) C.perft[i] = C.perft[C.dup[i]];
-        else if (st == ST_LIVE && C.k && rc >= 2 && tt.base[rc]) stored = tt_store(tt, rc, C.k[i], C.perft[i]);
-        if (ctr) ctr_count(ctr, rc, 2, stored);
-    }
-}
-
-static __global__ __launch_bounds__(256) void kd_segsum(Plan *P, int l) {
+// level l's perfts from those of level l+1 (see k_up; rc: its remaining depth)
+static __global__ __launch_bounds__(UP_WG) void kd_up(Plan *P, int l, TTView tt, int rc, TTCounters *ctr) {
     const DLevel L = P->lv[l];
     const DLevel C = P->lv[l + 1];
     if (P->overflow) return;
-    const u64 base = l == 0 ? P->bias : 0;
-    PG_GRID_LOOP(i, L.n) {
-        if (L.state[i] != ST_LIVE) continue;
-        L.perft[i] = sum_checked(C.perft, L.off[i], L.off[i + 1], base, &P->ovf);
-    }
+    const bool store = C.k && rc >= 2 && tt.base[rc];
+    sum_children(L.n, L.off, l == 0 ? P->bias : 0,
+        [&](u64 j) {
+            const u8 st = C.state[j];
+            const u64 v = C.perft[st == ST_DUP ? C.dup[j] : j];
+            bool stored = false;
+            if (store && st == ST_LIVE) stored = tt_store(tt, rc, C.k[j], v);
+            if (ctr) ctr_count(ctr, rc, 2, stored);
+            return v;
+        },
+        [&](u64 i, u64 s, bool wide) {
+            if (L.state[i] != ST_LIVE) return;
+            L.perft[i] = s;
+            if (wide) P->ovf = 1;
+        });
 }
 
 }  // namespace pg

@@ -227,8 +227,7 @@ static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, Link *H, con
         }
     }
     for (int l = lastExpand; l >= 0; l--) {
-        kd_resolve<<<gWork, 256, 0, s>>>(P, l, tt, D - l - 1, ctr);
-        kd_segsum<<<gWork, 256, 0, s>>>(P, l);
+        kd_up<<<gWork, UP_WG, 0, s>>>(P, l, tt, D - l - 1, ctr);
     }
     if (sh.tt) kd_root_store<<<gWork, 256, 0, s>>>(P, tt, D, ctr);
     kd_end<<<1, 1024, 0, s>>>(P, H);

@@ -34,19 +34,6 @@ __device__ __forceinline__ void add_checked(u64 *acc, u64 s, u32 *ovf) {
     if (old + s < old) atomicOr(ovf, 1u);
 }
 
-// sum of v[lo..hi) with a carry check
-__device__ __forceinline__ u64 sum_checked(const u64 *__restrict__ v, u64 lo, u64 hi, u64 base, u32 *ovf) {
-    u64 s = base;
-    bool carry = false;
-    for (u64 j = lo; j < hi; j++) {
-        const u64 x = v[j];
-        s += x;
-        carry |= s < x;
-    }
-    if (carry) *ovf = 1;
-    return s;
-}
-
 // per-call device state reset without memset nodes: total (with an optional
 // starting bias), consumed leaf items, error and overflow flags
 static __global__ void k_init_call(u64 *acc, u64 bias, u64 *items, u32 *err, u32 *ovf) {
@@ -266,6 +253,46 @@ __device__ __forceinline__ u64 block_excl_scan(u64 v, u64 *total) {
     __syncthreads();
     *total = tot;
     return base + incl - v;
+}
+
+// ---------------------------------------------------------------- way back up
+// done(i, base + sum of value(j) over i's children j, the sum passed 64 bits)
+// for parents [0, n), whose children lie one after the other at off[0..n].
+// Bound by memory: a work-group reads the children of 64 parents by
+// consecutive lanes into LDS, where each parent's lane adds up its own.  A
+// lane per parent that read its children itself, after a pass that copied the
+// owners' values to the duplicates, took 3.2 ms for the 136 M children of the
+// last level of 4096 positions at depth 5; this takes 1.1.
+constexpr int UP_WG = 256, UP_PARENTS = 64, UP_WINDOW = 2048;
+template <class Value, class Done>
+__device__ __forceinline__ void sum_children(u64 n, const u64 *__restrict__ off, u64 base, Value &&value, Done &&done) {
+    __shared__ u64 window[UP_WINDOW];
+    __shared__ u64 at[UP_PARENTS + 1];
+    const u32 tid = threadIdx.x;
+    for (u64 first = (u64)blockIdx.x * UP_PARENTS; first < n; first += (u64)gridDim.x * UP_PARENTS) {
+        const u32 np = n - first < UP_PARENTS ? (u32)(n - first) : UP_PARENTS;
+        if (tid <= np) at[tid] = off[first + tid];
+        __syncthreads();
+        const u64 lo = at[0], hi = at[np];
+        u64 s = base;
+        bool carry = false;
+        for (u64 c = lo; c < hi; c += UP_WINDOW) {
+            const u64 e = c + UP_WINDOW < hi ? c + UP_WINDOW : hi;
+            for (u64 j = c + tid; j < e; j += UP_WG) window[j - c] = value(j);
+            __syncthreads();
+            if (tid < np) {
+                const u64 from = at[tid] > c ? at[tid] : c, to = at[tid + 1] < e ? at[tid + 1] : e;
+                for (u64 j = from; j < to; j++) {
+                    const u64 x = window[j - c];
+                    s += x;
+                    carry |= s < x;
+                }
+            }
+            __syncthreads();
+        }
+        if (tid < np) done(first + tid, s, carry);
+        __syncthreads();
+    }
 }
 
 // ---------------------------------------------------------------- fused leaf

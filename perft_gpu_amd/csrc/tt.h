@@ -221,29 +221,31 @@ static __global__ __launch_bounds__(256) void k_dedup(Pos *__restrict__ children
     }
 }
 
-// After the children's perfts are known: duplicates copy their owner's value,
-// live children are stored in the table.
-static __global__ __launch_bounds__(256) void k_resolve_store(const Key128 *__restrict__ ckeys, u64 m, u64 *cperft,
-                                                       const u8 *__restrict__ state, const u32 *__restrict__ dup,
-                                                       TTView tt, int rc, TTCounters *ctr) {
-    PG_GRID_LOOP(i, m) {
-        const u8 st = state[i];
-        bool stored = false;
-        if (st == ST_DUP) cperft[i] = cperft[dup[i]];
-        else if (st == ST_LIVE && rc >= 2 && tt.base[rc]) stored = tt_store(tt, rc, ckeys[i], cperft[i]);  // no loads without a table
-        if (ctr) ctr_count(ctr, rc, 2, stored);
-    }
-}
-
-// P[i] = base + sum of the children's perfts of board i (children are
-// contiguous; base is 0 except under the count-bias test hook); boards
-// resolved before expansion keep their value.  A sum that wraps raises *ovf.
-static __global__ __launch_bounds__(256) void k_segsum(const Pos *__restrict__ boards, u64 n, const u64 *__restrict__ off,
-                                                const u64 *__restrict__ cperft, u64 *__restrict__ P, u64 base, u32 *ovf) {
-    PG_GRID_LOOP(i, n) {
-        if (!pos_valid(boards[i])) continue;
-        P[i] = sum_checked(cperft, off[i], off[i + 1], base, ovf);
-    }
+// The perfts of boards [0, n) from their children's: P[i] = base + the sum
+// over i's children (base is 0 except under the count-bias test hook).  A
+// duplicate counts as its owner, and a child that was counted is stored in
+// its depth's table.  Boards resolved before the expansion keep their value.
+// A sum that wraps raises *ovf.
+static __global__ __launch_bounds__(UP_WG) void k_up(const Pos *__restrict__ boards, u64 n, const u64 *__restrict__ off,
+                                                     const Key128 *__restrict__ ckeys, const u64 *__restrict__ cperft,
+                                                     const u8 *__restrict__ state, const u32 *__restrict__ dup,
+                                                     u64 *__restrict__ P, u64 base, u32 *ovf, TTView tt, int rc,
+                                                     TTCounters *ctr) {
+    const bool store = rc >= 2 && tt.base[rc];
+    sum_children(n, off, base,
+        [&](u64 j) {
+            const u8 st = state[j];
+            const u64 v = cperft[st == ST_DUP ? dup[j] : j];
+            bool stored = false;
+            if (store && st == ST_LIVE) stored = tt_store(tt, rc, ckeys[j], v);
+            if (ctr) ctr_count(ctr, rc, 2, stored);
+            return v;
+        },
+        [&](u64 i, u64 s, bool wide) {
+            if (!pos_valid(boards[i])) return;
+            P[i] = s;
+            if (wide) *ovf = 1;
+        });
 }
 
 // probe (store = 0) or store (store = 1) a single key, e.g. the root
@@ -275,7 +277,7 @@ static __global__ __launch_bounds__(256) void k_fill_random(ulonglong2 *p, u64 n
     }
 }
 
-// perft(1) of valid boards = their move counts (+ base, see k_segsum)
+// perft(1) of valid boards = their move counts (+ base, see k_up)
 static __global__ __launch_bounds__(256) void k_perft1(const Pos *__restrict__ boards, u64 n, const u32 *__restrict__ cnt, u64 *P,
                                                 u64 base, u32 *ovf) {
     PG_GRID_LOOP(i, n) {

@@ -170,9 +170,8 @@ int Engine::tt_bfs(int v, TTable &tt, Pos *B, Key128 *K, u64 n, u32 *cnt, int r,
         top = keep;  // moves, parents and the set are no longer needed
         rc = tt_bfs(v, tt, C, CK, m, Ccnt, rcd, CP, ply + 1);
         if (rc) return rc;
-        k_resolve_store<<<grid(m, 256), 256, 0, stream>>>(CK, m, CP, S, D, tt.view, rcd, tt.dCtr);
     }
-    k_segsum<<<grid(n, 256), 256, 0, stream>>>(B, n, off, CP, P, ply == 0 ? bias : 0, dOvf);
+    k_up<<<grid(n, UP_PARENTS), UP_WG, 0, stream>>>(B, n, off, CK, CP, S, D, P, ply == 0 ? bias : 0, dOvf, tt.view, rcd, tt.dCtr);
     HIP_TRY(hipGetLastError());
     top = mark;
     return PG_OK;
@@ -199,13 +198,16 @@ int Engine::tt_last(int v, TTable &tt, Pos *B, Key128 *K, u64 n, u32 *cnt, u64 *
     if (rc == PG_ENOMEM) { top = mark; return tt_split(v, tt, B, K, n, cnt, r, P, ply); }
     if (rc) return rc;
     if (m > 0xFFFFFFFFULL) { top = mark; return tt_split(v, tt, B, K, n, cnt, r, P, ply); }
+    Key128 *CK = nullptr;
     u64 *CP = nullptr;
+    u32 *D = nullptr;
+    u8 *S = nullptr;
     if (m) {
         const u64 chunks = (m + LIVE_CHUNK - 1) / LIVE_CHUNK;
-        Key128 *CK = (Key128 *)alloc(m * sizeof(Key128));
+        CK = (Key128 *)alloc(m * sizeof(Key128));
         CP = CK ? (u64 *)alloc(m * sizeof(u64)) : nullptr;
-        u32 *D = CP ? (u32 *)alloc(m * sizeof(u32)) : nullptr;
-        u8 *S = D ? (u8 *)alloc(m) : nullptr;
+        D = CP ? (u32 *)alloc(m * sizeof(u32)) : nullptr;
+        S = D ? (u8 *)alloc(m) : nullptr;
         u16 *mv = S ? (u16 *)alloc(m * sizeof(u16)) : nullptr;
         u32 *par = mv ? (u32 *)alloc(m * sizeof(u32)) : nullptr;
         u32 *chunkCount = par ? (u32 *)alloc(chunks * sizeof(u32)) : nullptr;
@@ -247,9 +249,8 @@ int Engine::tt_last(int v, TTable &tt, Pos *B, Key128 *K, u64 n, u32 *cnt, u64 *
         }
         stats.leaf_launches++;
         stats.leaf_parents += nLive;
-        k_resolve_store<<<grid(m, 256), 256, 0, stream>>>(CK, m, CP, S, D, tt.view, rcd, tt.dCtr);
     }
-    k_segsum<<<grid(n, 256), 256, 0, stream>>>(B, n, off, CP, P, ply == 0 ? bias : 0, dOvf);
+    k_up<<<grid(n, UP_PARENTS), UP_WG, 0, stream>>>(B, n, off, CK, CP, S, D, P, ply == 0 ? bias : 0, dOvf, tt.view, rcd, tt.dCtr);
     HIP_TRY(hipGetLastError());
     top = mark;
     return PG_OK;
