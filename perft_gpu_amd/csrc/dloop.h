@@ -3,14 +3,17 @@
 // captured once into a HIP graph and replayed.
 //
 // Sizes and array pointers of every level live in a Plan in device memory.
-// Single-thread planning kernels read the scan total, carve the next level's
-// arrays out of a bump region (stack discipline: transient move/parent/set
-// arrays are released after expansion) and publish the level's size; the
-// work kernels are persistent grid-stride loops that read their size from
-// the plan.  If a level does not fit, the planner raises `overflow` and
-// publishes size 0, every later kernel becomes a no-op, and the host reruns
-// the batch in halves.  Per-root results come back up the levels by
-// segmented sums (children of a board are contiguous), as in the TT path.
+// The work-group that ends a level's scan reads the total, carves the next
+// level's arrays out of a bump region (stack discipline: transient
+// move/parent/set arrays are released after expansion) and publishes the
+// level's size; the work kernels are persistent grid-stride loops that read
+// their size from the plan.  A kernel of a small level takes 4 to 5 us
+// whatever it does, so a level takes few: scan and plan; moves, their offsets
+// and the empty duplicate set; children; duplicates.  If a level does not
+// fit, the plan raises `overflow` and publishes size 0, every later kernel
+// becomes a no-op, and the host reruns the batch in halves.  Per-root results
+// come back up the levels by segmented sums (children of a board are
+// contiguous), as in the TT path.
 #pragma once
 #include "tt.h"
 
@@ -25,7 +28,8 @@ struct DLevel {
     u64 *perft;
     u8 *state;
     u32 *dup;
-    u64 *tiles;       // scan tile sums
+    u64 *tiles;       // children before each tile of GEN_WG boards
+    u64 kids;         // children of the level
     u32 *live;        // leaf level: the boards with moves (kd_live), when there was room
     u16 *mv;          // moves / parents of the children: transient, or kept (keep) when
     u32 *par;         //   the children's boards are not stored (the leaf makes them)
@@ -46,6 +50,7 @@ struct Plan {
     u64 peak;           // highest bump top reached (bytes of the region used)
     u64 liveN;          // entries of the leaf level's live list
     u64 began;          // device clock at the search's start
+    u32 arrived[TT_MAX_DEPTH];  // work-groups done with a level's kd_scan
     DLevel lv[TT_MAX_DEPTH];
 };
 
@@ -83,6 +88,16 @@ __device__ __forceinline__ void *plan_try_alloc(Plan *P, u64 bytes) {
 
 #define PG_GRID_LOOP_N(i, n) PG_GRID_LOOP(i, n)
 
+// room for the offsets of a level that will be expanded
+__device__ __forceinline__ void plan_offsets(Plan *P, DLevel &L) {
+    L.off = nullptr;
+    L.tiles = nullptr;
+    if (L.n == 0) return;
+    L.off = (u64 *)plan_alloc(P, (L.n + 1) * 8);
+    L.tiles = L.off ? (u64 *)plan_alloc(P, ((L.n + GEN_WG - 1) / GEN_WG) * 8) : nullptr;
+    if (!L.tiles) L.n = 0;
+}
+
 // The first kernel: the plan and the roots come from the host, the roots are
 // counted (deeper levels get their counts from the expansion) and the table
 // of depth D is probed: hits are resolved before the expansion.
@@ -94,7 +109,10 @@ __global__ __launch_bounds__(wg_size<V>()) void kd_begin(Plan *P, const Link *H,
         const u64 *from = (const u64 *)&H->plan;
         for (u32 i = threadIdx.x; i < sizeof(Plan) / 8; i += blockDim.x) ((u64 *)P)[i] = from[i];
         __syncthreads();
-        if (threadIdx.x == 0) P->began = wall_clock64();
+        if (threadIdx.x == 0) {
+            P->began = wall_clock64();
+            if (!small) plan_offsets(P, P->lv[0]);
+        }
     }
     const DLevel L = H->plan.lv[0];
     const u64 bias = H->plan.bias;
@@ -150,6 +168,7 @@ template <int V>
 __global__ __launch_bounds__(wg_size<V>()) void kd_count(Plan *P, Tables t) {
     stage_tables<V>(t);
     const DLevel L = P->lv[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) plan_offsets(P, P->lv[0]);
     PG_GRID_LOOP(i, L.n) L.cnt[i] = count_any<V>(L.b[i], t);
 }
 
@@ -173,75 +192,81 @@ __device__ __forceinline__ void release_level(Plan *P, int l) {
     L.set = nullptr;
 }
 
-// release level l-1's transient arrays (l > 0), then allocate the offsets
-// and scan tiles of level l
-static __global__ void kd_plan_scan(Plan *P, int l) {
-    if (threadIdx.x || blockIdx.x) return;
-    if (l > 0) release_level(P, l - 1);
-    DLevel &L = P->lv[l];
-    L.off = nullptr;
-    L.tiles = nullptr;
-    if (L.n == 0) return;
-    L.off = (u64 *)plan_alloc(P, (L.n + 1) * 8);
-    L.tiles = L.off ? (u64 *)plan_alloc(P, ((L.n + SCAN_TILE - 1) / SCAN_TILE) * 8) : nullptr;
-    if (!L.tiles) L.n = 0;
-}
+__device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int total, int expand);
 
-static __global__ __launch_bounds__(SCAN_WG) void kd_scan_reduce(Plan *P, int l) {
+// The children before each tile of GEN_WG boards of level l, and the plan of
+// level l + 1.  The work-group that arrives last scans the tile sums and
+// plans: what it reads was written by atomics that had returned before the
+// writer arrived.  (expand: level l + 1 will be expanded in its turn.)
+constexpr int PLAN_IPT = 8;
+static __global__ __launch_bounds__(GEN_WG) void kd_scan(Plan *P, int l, int wantKeys, int wantSet, int total, int expand) {
+    __shared__ u32 last;
+    constexpr u32 WAVES = GEN_WG / 64;
+    const u32 tid = threadIdx.x, lane = tid & 63;
     const DLevel L = P->lv[l];
-    const u64 tiles = (L.n + SCAN_TILE - 1) / SCAN_TILE;
-    for (u64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const u64 base = tile * SCAN_TILE + (u64)threadIdx.x * SCAN_IPT;
-        u32 v[SCAN_IPT];
-        load_tile(L.cnt, L.n, base, v);
-        u64 s = 0;
+    const u64 tiles = (L.n + GEN_WG - 1) / GEN_WG;
+    // work-groups without a tile do not take part (arrivals take 6 ns each)
+    const u64 need = tiles ? (tiles + WAVES - 1) / WAVES : 1;
+    const u32 members = need < gridDim.x ? (u32)need : gridDim.x;
+    if (blockIdx.x >= members) return;
+    for (u64 tile = (u64)blockIdx.x * WAVES + wave_number(); tile < tiles; tile += (u64)members * WAVES) {
+        u32 c = 0;
 #pragma unroll
-        for (int j = 0; j < SCAN_IPT; j++) s += v[j];
-        u64 tot;
-        block_excl_scan<SCAN_WG>(s, &tot);
-        if (threadIdx.x == 0) L.tiles[tile] = tot;
-    }
-}
-
-__device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int total);
-
-// scan of the tile sums; then one thread plans level l+1 from the total
-static __global__ __launch_bounds__(1024) void kd_scan_spine(Plan *P, int l, int wantKeys, int wantSet, int total) {
-    const DLevel L = P->lv[l];
-    if (L.n) {
-        const u64 tiles = (L.n + SCAN_TILE - 1) / SCAN_TILE;
-        u64 carry = 0;
-        for (u64 s = 0; s < tiles; s += 1024) {
-            const u64 i = s + threadIdx.x;
-            const u64 v = i < tiles ? L.tiles[i] : 0;
-            u64 tot;
-            const u64 ex = block_excl_scan<1024>(v, &tot);
-            if (i < tiles) L.tiles[i] = carry + ex;
-            carry += tot;
+        for (u32 k = 0; k < WAVES; k++) {
+            const u64 i = tile * GEN_WG + k * 64 + lane;
+            c += i < L.n ? L.cnt[i] : 0;
         }
-        if (threadIdx.x == 0) L.off[L.n] = carry;
+        const u64 sum = wave_sum32(c);
+        if (lane == 0) __hip_atomic_store(&L.tiles[tile], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (threadIdx.x == 0) plan_children(P, l, wantKeys, wantSet, total);
-}
-
-static __global__ __launch_bounds__(SCAN_WG) void kd_scan_down(Plan *P, int l) {
-    const DLevel L = P->lv[l];
-    const u64 tiles = (L.n + SCAN_TILE - 1) / SCAN_TILE;
-    for (u64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const u64 base = tile * SCAN_TILE + (u64)threadIdx.x * SCAN_IPT;
-        u32 v[SCAN_IPT];
-        load_tile(L.cnt, L.n, base, v);
-        u64 s = 0;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) last = atomicAdd(&P->arrived[l], 1u) + 1 == members;
+    __syncthreads();
+    if (!last) return;
+    u64 carry = 0;
+    for (u64 first = 0; first < tiles; first += GEN_WG * PLAN_IPT) {
+        const u64 at = first + tid * PLAN_IPT;
+        u64 v[PLAN_IPT], sum = 0;
 #pragma unroll
-        for (int j = 0; j < SCAN_IPT; j++) s += v[j];
-        u64 tot;
-        u64 run = L.tiles[tile] + block_excl_scan<SCAN_WG>(s, &tot);
+        for (int j = 0; j < PLAN_IPT; j++) {
+            v[j] = at + j < tiles ? __hip_atomic_load(&L.tiles[at + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+            sum += v[j];
+        }
+        u64 all;
+        u64 run = carry + block_excl_scan<GEN_WG>(sum, &all);
 #pragma unroll
-        for (int j = 0; j < SCAN_IPT; j++) {
-            if (base + j < L.n) L.off[base + j] = run;
+        for (int j = 0; j < PLAN_IPT; j++) {
+            if (at + j < tiles) L.tiles[at + j] = run;
             run += v[j];
         }
+        carry += all;
     }
+    if (tid == 0) {
+        P->lv[l].kids = carry;
+        if (l > 0) release_level(P, l - 1);
+        plan_children(P, l, wantKeys, wantSet, total, expand);
+    }
+}
+
+// The offsets of a tile's boards' children (all threads): this thread's board
+// is number first + threadIdx.x; returns its offset and *c, its count.
+__device__ __forceinline__ u64 tile_offsets(const DLevel &L, u64 first, u32 *c) {
+    const u64 i = first + threadIdx.x;
+    *c = i < L.n ? L.cnt[i] : 0;
+    u64 sum;
+    const u64 o = L.tiles[first / GEN_WG] + block_excl_scan<GEN_WG>(*c, &sum);
+    if (i < L.n) L.off[i] = o;
+    if (i + 1 == L.n) L.off[L.n] = o + *c;
+    return o;
+}
+// the offsets for the byte-lookup variant, whose tables leave the generate
+// kernel no room for a scan
+static __global__ __launch_bounds__(GEN_WG) void kd_offsets(Plan *P, int l) {
+    const DLevel L = P->lv[l];
+    if (P->lv[l + 1].n == 0) return;
+    u32 c;
+    for (u64 first = (u64)blockIdx.x * GEN_WG; first < L.n; first += (u64)gridDim.x * GEN_WG) (void)tile_offsets(L, first, &c);
 }
 
 // allocate level l+1 (children of l) and the transient arrays; a total-only
@@ -249,12 +274,12 @@ static __global__ __launch_bounds__(SCAN_WG) void kd_scan_down(Plan *P, int l) {
 // total == 3: the last level of a search with per-board results and keys
 // keeps no boards or counts, only keys, perfts, states and owners; the moves
 // and parents stay until the leaf, which makes the children from them.
-__device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int total) {
+__device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int total, int expand) {
     DLevel &L = P->lv[l];
     DLevel &C = P->lv[l + 1];
     memset(&C, 0, sizeof(C));
     L.keep = 0;
-    const u64 m = L.n ? L.off[L.n] : 0;
+    const u64 m = L.n ? L.kids : 0;
     if (m == 0 || m > 0xFFFFFFFFULL) {
         if (m) P->overflow = 1;
         return;
@@ -289,6 +314,8 @@ __device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int tot
         C.dup = (u32 *)plan_alloc(P, m * 4);
     }
     if (wantKeys) C.k = (Key128 *)plan_alloc(P, m * sizeof(Key128));
+    C.n = m;
+    if (expand) plan_offsets(P, C);
     L.release = P->top;
     L.mv = (u16 *)plan_alloc(P, m * 2);
     L.par = (u32 *)plan_alloc(P, m * 4);
@@ -305,11 +332,14 @@ __device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int tot
     C.n = m;
 }
 
+// the moves of level l, and its duplicate set emptied (graphs get no memset
+// nodes)
 template <int V>
 __global__ __launch_bounds__(wg_size<V>()) void kd_generate(Plan *P, int l, Tables t) {
     stage_tables<V>(t);
     const DLevel L = P->lv[l];
     if (P->lv[l + 1].n == 0) return;
+    if (L.set) PG_GRID_LOOP(i, L.setMask + 1) L.set[i] = 0;
     if constexpr (V == SL_BYTE) {
         PG_GRID_LOOP(i, L.n) {
             const u64 o = L.off[i];
@@ -320,7 +350,7 @@ __global__ __launch_bounds__(wg_size<V>()) void kd_generate(Plan *P, int l, Tabl
             for (u32 j = 0; j < room; j++) L.par[o + j] = (u32)i;
         }
     } else {
-        generate_tiles<V>(L.b, L.n, L.off, L.mv, L.par, &P->err, t);
+        generate_tiles<V>(L.b, L.n, L.mv, L.par, &P->err, t, [&](u64 first, u32 *c) { return tile_offsets(L, first, c); });
     }
 }
 
@@ -391,13 +421,6 @@ __device__ __forceinline__ bool same_child(const DLevel &L, u64 a, u64 b, const 
     make_any(pa, L.mv[a], t);
     make_any(pb, L.mv[b], t);
     return same_board(pa, pb);
-}
-
-// fill kernel for the duplicate set (graphs get no memset nodes)
-static __global__ __launch_bounds__(256) void kd_clear_set(Plan *P, int l) {
-    const DLevel L = P->lv[l];
-    if (!L.set || P->lv[l + 1].n == 0) return;
-    PG_GRID_LOOP(i, L.setMask + 1) L.set[i] = 0;
 }
 
 // one child after its first probe (kd_dedup): follow the probe sequence
@@ -670,8 +693,13 @@ static __global__ __launch_bounds__(UP_WG) void kd_up(Plan *P, int l, TTView tt,
     const DLevel L = P->lv[l];
     const DLevel C = P->lv[l + 1];
     if (P->overflow) return;
+    const u64 base = l == 0 ? P->bias : 0;
+    if (C.n == 0) {  // no moves at all, and no offsets
+        PG_GRID_LOOP(i, L.n) if (L.state[i] == ST_LIVE) L.perft[i] = base;
+        return;
+    }
     const bool store = C.k && rc >= 2 && tt.base[rc];
-    sum_children(L.n, L.off, l == 0 ? P->bias : 0,
+    sum_children(L.n, L.off, base,
         [&](u64 j) {
             const u8 st = C.state[j];
             const u64 v = C.perft[st == ST_DUP ? C.dup[j] : j];

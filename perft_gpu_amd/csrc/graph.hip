@@ -159,10 +159,8 @@ static void enqueue_total(const Engine &e, hipStream_t s, Plan *P, const GraphSh
     const int gWork = G.work, gScan = G.scan, gv = G.v;
     PG_VARIANT_CALL(v, cap_count, s, P, gv, e.dt);
     for (int l = 0; l <= D - 2; l++) {
-        kd_plan_scan<<<1, 64, 0, s>>>(P, l);
-        kd_scan_reduce<<<gScan, SCAN_WG, 0, s>>>(P, l);
-        kd_scan_spine<<<1, 1024, 0, s>>>(P, l, 0, 0, 1);
-        kd_scan_down<<<gScan, SCAN_WG, 0, s>>>(P, l);
+        kd_scan<<<std::min(gScan, 512), GEN_WG, 0, s>>>(P, l, 0, 0, 1, l + 1 <= D - 2);
+        kd_offsets<<<gScan, GEN_WG, 0, s>>>(P, l);
         PG_VARIANT_CALL(v, cap_generate, s, P, l, gv, e.dt);
         PG_VARIANT_CALL(v, cap_expand, s, P, l, TTView{}, D - l - 1, (TTCounters *)nullptr, gv, e.dt);
     }
@@ -197,20 +195,15 @@ static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, Link *H, con
         const int rc = D - l - 1;
         const int wantSet = sh.dedup && rc >= 2;
         const bool kl = keysLast && l == lastExpand;
-        kd_plan_scan<<<1, 64, 0, s>>>(P, l);
-        kd_scan_reduce<<<gScan, SCAN_WG, 0, s>>>(P, l);
-        kd_scan_spine<<<1, 1024, 0, s>>>(P, l, sh.keys, wantSet, kl ? 3 : 0);
-        kd_scan_down<<<gScan, SCAN_WG, 0, s>>>(P, l);
+        kd_scan<<<std::min(gScan, 512), GEN_WG, 0, s>>>(P, l, sh.keys, wantSet, kl ? 3 : 0, l + 1 <= lastExpand);
+        if (v == SL_BYTE) kd_offsets<<<gScan, GEN_WG, 0, s>>>(P, l);
         PG_VARIANT_CALL(v, cap_generate, s, P, l, gv, e.dt);
         if (kl) {
             PG_VARIANT_CALL(v, cap_expand_keys, s, P, l, tt, rc, ctr, gv, e.dt);
         } else {
             PG_VARIANT_CALL(v, cap_expand, s, P, l, tt, rc, ctr, gv, e.dt);
         }
-        if (wantSet) {
-            kd_clear_set<<<gWork, 256, 0, s>>>(P, l);
-            kd_dedup<<<gWork, 256, 0, s>>>(P, l, ctr, rc, sh.tt != nullptr, e.dt);
-        }
+        if (wantSet) kd_dedup<<<gWork, 256, 0, s>>>(P, l, ctr, rc, sh.tt != nullptr, e.dt);
     }
     const int last = lastExpand + 1;  // deepest materialized level
     if (D == 1 || v == SL_BYTE) {

@@ -139,22 +139,27 @@ static __global__ __launch_bounds__(256) void k_sum_u32(const u32 *__restrict__ 
 // (the two must agree for the level layout to be valid).
 constexpr int GEN_WG = 256, GEN_WINDOW = 8192;
 
-template <int V>
-__device__ __forceinline__ void generate_tiles(const Pos *__restrict__ b, u64 n, const u64 *__restrict__ off,
-                                               u16 *__restrict__ moves, u32 *__restrict__ parent, u32 *err,
-                                               const Tables &t) {
+// offsets(first, &c): the offset of board first + threadIdx.x and its count
+// (0: no moves, or resolved earlier)
+template <int V, class Offsets>
+__device__ __forceinline__ void generate_tiles(const Pos *__restrict__ b, u64 n, u16 *__restrict__ moves,
+                                               u32 *__restrict__ parent, u32 *err, const Tables &t, Offsets &&offsets) {
     __shared__ u32 word[GEN_WINDOW];
-    __shared__ u32 snext;
+    __shared__ u32 snext, stotal;
+    __shared__ u64 sbase;
     const int tid = threadIdx.x;
     for (u64 tile = blockIdx.x; tile * GEN_WG < n; tile += gridDim.x) {
         const u64 first = tile * GEN_WG;
-        const u64 last = first + GEN_WG < n ? first + GEN_WG : n;
         const u64 i = first + tid;
-        const bool live = i < n;
-        const u64 base = off[first];
-        const u32 pos = live ? (u32)(off[i] - base) : 0;
-        const u32 c = live ? (u32)(off[i + 1] - off[i]) : 0;  // 0: no moves, or resolved earlier
-        const u32 total = (u32)(off[last] - base);
+        u32 c;
+        const u64 off = offsets(first, &c);
+        if (tid == 0) sbase = off;
+        __syncthreads();
+        const u64 base = sbase;
+        const u32 pos = (u32)(off - base);
+        if (tid == GEN_WG - 1) stotal = pos + c;
+        __syncthreads();
+        const u32 total = stotal;
         u32 start = 0;
         while (start < total) {
             const u32 end = start + GEN_WINDOW;
@@ -195,7 +200,11 @@ __global__ __launch_bounds__(wg_size<V>()) void k_generate(const Pos *__restrict
             for (u32 j = 0; j < room; j++) parent[o + j] = (u32)i;
         }
     } else {
-        generate_tiles<V>(b, n, off, moves, parent, err, t);
+        generate_tiles<V>(b, n, moves, parent, err, t, [&](u64 first, u32 *c) {
+            const u64 i = first + threadIdx.x;
+            *c = i < n ? (u32)(off[i + 1] - off[i]) : 0;
+            return off[i < n ? i : n];
+        });
     }
 }
 
