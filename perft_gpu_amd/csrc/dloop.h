@@ -426,7 +426,7 @@ __device__ __forceinline__ bool same_child(const DLevel &L, u64 a, u64 b, const 
 // one child after its first probe (kd_dedup): follow the probe sequence
 // until the child owns a slot or finds its equal
 __device__ __forceinline__ void kd_dedup_finish(Plan *P, const DLevel &L, const DLevel &C, u64 i, bool live, u64 s,
-                                                u32 cur, TTCounters *ctr, int rc, int keyOnly, const Tables &t) {
+                                                u32 cur, bool look, TTCounters *ctr, int rc, int keyOnly, const Tables &t) {
     bool isDup = false;
     if (live) {
         for (u64 step = 0;; step++) {
@@ -440,7 +440,7 @@ __device__ __forceinline__ void kd_dedup_finish(Plan *P, const DLevel &L, const 
             }
             if (step >= L.setMask) { P->err = 3; break; }
             s = (s + 1) & L.setMask;
-            cur = atomicCAS(&L.set[s], 0u, (u32)i + 1);
+            cur = slot_claim(&L.set[s], look ? slot_look(&L.set[s]) : 0, (u32)i + 1);
         }
     }
     if (ctr) ctr_count(ctr, rc, 3, isDup);
@@ -459,15 +459,21 @@ static __global__ __launch_bounds__(256) void kd_dedup(Plan *P, int l, TTCounter
     const DLevel C = P->lv[l + 1];
     if (!L.set) return;
     const u64 stride = (u64)gridDim.x * blockDim.x;
+    // A set that the caches hold is claimed without a look first: the swap
+    // waits less there, and the look is one more access in a row (32 MB set,
+    // divide of an opening at depth 7: 1134 us per call without, 1170 with;
+    // 1 GB set, 4096 positions at depth 5: 46.0 ms without, 45.2 with).
+    const bool look = L.setMask >= 1u << 25;
     for (u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x; i0 < C.n; i0 += 2 * stride) {
         const u64 i1 = i0 + stride;
         const bool has1 = i1 < C.n;
         const bool l0 = C.state[i0] == ST_LIVE, l1 = has1 && C.state[i1] == ST_LIVE;
         const u64 s0 = (C.k[i0].lo >> 7) & L.setMask, s1 = l1 ? (C.k[i1].lo >> 7) & L.setMask : 0;
-        const u32 c0 = l0 ? atomicCAS(&L.set[s0], 0u, (u32)i0 + 1) : 0;
-        const u32 c1 = l1 ? atomicCAS(&L.set[s1], 0u, (u32)i1 + 1) : 0;
-        kd_dedup_finish(P, L, C, i0, l0, s0, c0, ctr, rc, keyOnly, t);
-        if (has1) kd_dedup_finish(P, L, C, i1, l1, s1, c1, ctr, rc, keyOnly, t);
+        u32 c0 = l0 && look ? slot_look(&L.set[s0]) : 0, c1 = l1 && look ? slot_look(&L.set[s1]) : 0;
+        if (l0) c0 = slot_claim(&L.set[s0], c0, (u32)i0 + 1);
+        if (l1) c1 = slot_claim(&L.set[s1], c1, (u32)i1 + 1);
+        kd_dedup_finish(P, L, C, i0, l0, s0, c0, look, ctr, rc, keyOnly, t);
+        if (has1) kd_dedup_finish(P, L, C, i1, l1, s1, c1, look, ctr, rc, keyOnly, t);
     }
 }
 

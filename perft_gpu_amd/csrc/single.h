@@ -493,7 +493,7 @@ static __global__ __launch_bounds__(S_COLLAPSE_WG) void ks_collapse(SPlan *P, SR
             const u64 h = s_hash(nd.b);
             const u64 id = (h << 48) | (u64)mv << 32 | par;
             at = __umul64hi(h, slots);
-            u64 cur = atomicCAS(&L.set[at].id, 0ULL, id);
+            u64 cur = slot_claim(&L.set[at].id, slot_look(&L.set[at].id), id);
             for (u64 step = 0; cur; step++) {
                 if ((cur ^ id) >> 48 == 0) {
                     const Pos q = s_child(L.node, (u32)cur, (u16)(cur >> 32), t);
@@ -506,7 +506,7 @@ static __global__ __launch_bounds__(S_COLLAPSE_WG) void ks_collapse(SPlan *P, SR
                 }
                 if (step >= slots) { P->err = 3; break; }
                 at = at + 1 < slots ? at + 1 : 0;
-                cur = atomicCAS(&L.set[at].id, 0ULL, id);
+                cur = slot_claim(&L.set[at].id, slot_look(&L.set[at].id), id);
             }
             nd.slot = (u32)at;
         }

@@ -192,7 +192,7 @@ __device__ __forceinline__ void dedup_finish(u64 i, bool live, u64 s, u32 cur, P
             }
             if (step >= setMask) { *err = 3; break; }
             s = (s + 1) & setMask;
-            cur = atomicCAS(&set[s], 0u, (u32)i + 1);
+            cur = slot_claim(&set[s], slot_look(&set[s]), (u32)i + 1);
         }
     }
     if (ctr) ctr_count(ctr, rc, 3, isDup);
@@ -214,8 +214,9 @@ static __global__ __launch_bounds__(256) void k_dedup(Pos *__restrict__ children
         const bool has1 = i1 < m;
         const bool l0 = state[i0] == ST_LIVE, l1 = has1 && state[i1] == ST_LIVE;
         const u64 s0 = (ckeys[i0].lo >> 7) & setMask, s1 = l1 ? (ckeys[i1].lo >> 7) & setMask : 0;
-        const u32 c0 = l0 ? atomicCAS(&set[s0], 0u, (u32)i0 + 1) : 0;
-        const u32 c1 = l1 ? atomicCAS(&set[s1], 0u, (u32)i1 + 1) : 0;
+        u32 c0 = l0 ? slot_look(&set[s0]) : 0, c1 = l1 ? slot_look(&set[s1]) : 0;
+        if (l0) c0 = slot_claim(&set[s0], c0, (u32)i0 + 1);
+        if (l1) c1 = slot_claim(&set[s1], c1, (u32)i1 + 1);
         dedup_finish(i0, l0, s0, c0, children, ckeys, cnt, state, dup, set, setMask, err, ctr, rc);
         if (has1) dedup_finish(i1, l1, s1, c1, children, ckeys, cnt, state, dup, set, setMask, err, ctr, rc);
     }
