@@ -467,18 +467,19 @@ __device__ __forceinline__ u64 s_hash(const Pos &p) {
 // node, the others add their weight to the slot.  A slot holds 32 bits of the
 // hash beside the owner's item, so only a probable match is compared: the
 // owner is made again from the list and compared board for board.  Bound by
-// the random accesses to the set (one line per board, two operations on it
-// for a merged one): about 110 ps per listed move once the set is past the
-// caches.  Every work-group reserves its nodes with one atomic per pass on one
-// counter, hence the largest work-group: 1024 lanes take 326 us for the 1.9e6
-// moves of an opening's ply 5, 512 take 363 and 256 take 414.
-constexpr int S_COLLAPSE_WG = 1024;
-static __global__ __launch_bounds__(S_COLLAPSE_WG) void ks_collapse(SPlan *P, SRegion rg, int l, Tables t) {
+// the random accesses to the set and to the owners' parents, and by their
+// latency: a work-group waits for its longest probe sequence before it
+// reserves its nodes with one atomic (all on one counter, hence large
+// work-groups), so two of 768 per CU, at 80 registers, beat one of 1024: 300
+// us against 330 for the 1.9e6 moves of an opening's ply 5, which is 160 ps
+// per move; 110 ps for the 30e6 of ply 6.
+constexpr int S_COLLAPSE_WG = 768;
+static __global__ __launch_bounds__(S_COLLAPSE_WG, 6) void ks_collapse(SPlan *P, SRegion rg, int l, Tables t) {
     if (s_stopped(P)) return;
     __shared__ u64 sBase;
-    const SLevel L = s_level(rg, l - 1, P->nNode[l - 1]);
+    const SLevel L = s_level(rg, l - 1, uniform64(P->nNode[l - 1]));
     SNode *out = (SNode *)rg.half[l & 1];
-    const u64 n = P->nList[l], slots = s_slots(n), cap = s_node_cap(rg);
+    const u64 n = uniform64(P->nList[l]), slots = s_slots(n), cap = s_node_cap(rg);
     for (u64 base = (u64)blockIdx.x * S_COLLAPSE_WG; base < n; base += (u64)gridDim.x * S_COLLAPSE_WG) {
         const u64 i = base + threadIdx.x;
         bool own = i < n;
