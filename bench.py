@@ -49,9 +49,9 @@ HBM_PEAK_GBS = 8000.0
 # Used only when the counters leg cannot run (no rocprofv3): VALU
 # instructions per counted board (SQ_INSTS_VALU x 64 / boards, one lane per
 # board) of k_leaf_moves<kogge_stone> measured by rocprofv3 on this workload
-# (profiles/k_leaf_moves_kogge_start_d7_d8_c2_d6.md)
-PROFILE_VALU_INSTS_PER_BOARD = 652
-PROFILE_SOURCE = "profiles/k_leaf_moves_kogge_start_d7_d8_c2_d6.md"
+# (profiles/leaf_by_difference.md)
+PROFILE_VALU_INSTS_PER_BOARD = 264
+PROFILE_SOURCE = "profiles/leaf_by_difference.md"
 LEAF_KERNEL = "k_leaf_moves<0>"
 COPY_BYTES = 1 << 30
 COPY_ITERS = 3
@@ -552,8 +552,8 @@ def main():
         kname, bnote = "k_leaf", "6 B per (parent, move) item + 48 B per parent board"
     hbm_gbs = bytes_per_launch / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
     boards_per_s = acc["items"] / (acc["ms"] * 1e-3) if acc["ms"] > 0 else 0.0
-    # VALU roofline: every counted board costs a fixed number of VALU wave
-    # instructions (64 lanes each); the vector peak is CUs x 128 lanes x clock,
+    # VALU roofline: a counted board costs some number of VALU wave
+    # instructions (64 lanes each; fewer for the moves that change nothing); the vector peak is CUs x 128 lanes x clock,
     # the published 157.3 TFLOP/s fp32 vector rate counted in lane operations
     # (an FMA is two flops).  Instructions per board come from the counters leg
     # of this run; without rocprofv3 the committed profile's figure is used.

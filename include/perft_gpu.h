@@ -257,7 +257,7 @@ int pg_set_dedup(pg_ctx *ctx, int on);
 
 typedef struct pg_batch_stats {
     double total_ms;        /* host wall time of the call */
-    double graph_ms;        /* HIP-event time of the graph launches */
+    double graph_ms;        /* device time of the searches, first kernel to last */
     uint64_t launches;      /* graph launches (1 unless the batch had to split) */
     uint64_t splits;        /* halvings forced by the region budget */
     uint64_t leaf_items;    /* (parent, move) items of the leaf level */
@@ -365,7 +365,7 @@ typedef struct pg_serve_stats {
     double submit_ms_max, submit_ms_total;   /* host time spent launching batches */
     uint64_t graphs;                         /* graphs instantiated by the slots so far */
     double device_ms;                        /* device time of the finished batches, summed (HIP
-                                                events around each batch's graph): over elapsed_ms,
+                                                clock over each batch): over elapsed_ms,
                                                 the mean number of batches running at once */
 } pg_serve_stats;
 typedef struct pg_serve pg_serve;
