@@ -553,22 +553,78 @@ __device__ __forceinline__ Pos s_board(const SRegion &rg, const SLevel &A, SNode
     }
 }
 
+// The moves of a few boards, each listed by a wave: up to S_FEW_BOARDS in a row
+// per wave, then one reservation for the work-group.  For so few boards the
+// kernel is one chain of latencies, and the listing by one lane each is the
+// longest link: 30 us for the 12000 boards of an opening's ply 3 against 37.
+constexpr u32 S_FEW_BOARDS = 4;
+template <int V, bool LIST>
+__device__ __forceinline__ void s_few_boards(u32 *word, const SRegion &rg, const SLevel &A, const SLevel &L, u64 n,
+                                             u64 *counter, SPlan *P, SSum &sum, const Tables &t) {
+    __shared__ u32 count[S_WAVES];
+    __shared__ u64 first;
+    const u32 wave = wave_number(), lane = threadIdx.x & 63;
+    u32 *const list = word + wave * S_FEW_BOARDS * 256;
+    const u32 each = s_tile_boards(n, S_RESIDENT * S_WAVES, 1, S_FEW_BOARDS);
+    for (u64 i0 = (u64)blockIdx.x * S_WAVES * each; i0 < n; i0 += (u64)gridDim.x * S_WAVES * each) {
+        const u64 mine = i0 + wave * each;
+        u32 m[S_FEW_BOARDS], total = 0;
+#pragma unroll
+        for (u32 k = 0; k < S_FEW_BOARDS; k++) {
+            m[k] = 0;
+            if (k < each && mine + k < n) {
+                u64 w;
+                const Pos b = uniform_pos(s_board<LIST, true>(rg, A, L.node, mine + k, &w, t));
+                m[k] = wave_words<V>(b, t, list + k * 256);
+                if (lane == 0) s_mad(&sum.paths, w, m[k], &sum.wide);
+            }
+            total += m[k];
+        }
+        if (lane == 0) count[wave] = total;
+        __syncthreads();
+        u32 before = 0, all = 0;
+        for (u32 v = 0; v < S_WAVES; v++) {
+            if (v < wave) before += count[v];
+            all += count[v];
+        }
+        if (threadIdx.x == 0) {
+            first = atomicAdd(counter, (u64)all);
+            if (first + all > L.cap) P->overflow = 1;
+        }
+        __syncthreads();
+        u64 at = first + before;
+        if (first + all <= L.cap)
+#pragma unroll
+            for (u32 k = 0; k < S_FEW_BOARDS; k++) {
+                for (u32 j = lane; j < m[k]; j += 64) {
+                    const u32 w = list[k * 256 + j];
+                    L.mv[at + j] = (u16)w;
+                    L.par[at + j] = (u32)(mine + k) | (u32)piece_code(w >> 24) << S_NODE_BITS;
+                }
+                at += m[k];
+            }
+        __syncthreads();
+    }
+}
+
 // ply l's boards to the list of ply l + 1
 template <int V, bool LIST>
 __global__ __launch_bounds__(LEAF_WG) void ks_level(SPlan *P, SRegion rg, int l, Tables t) {
     __shared__ ListTile s;
     if (s_stopped(P)) return;
-    const SLevel A = s_level(rg, l - 1, P->nNode[l - 1]);
-    const u64 n = LIST ? P->nList[l] : P->nNode[l];
+    const SLevel A = s_level(rg, l - 1, uniform64(P->nNode[l - 1]));
+    const u64 n = uniform64(LIST ? P->nList[l] : P->nNode[l]);
     if (LIST && n > s_node_cap(rg)) {
         if (threadIdx.x == 0) P->overflow = 1;
         return;
     }
     const SLevel L = s_level(rg, l, n);
     if (LIST && blockIdx.x == 0 && threadIdx.x == 0) P->nNode[l] = n;
-    const u32 T = s_tile_boards(n, S_RESIDENT, 8, LEAF_WG);
     SSum sum;
-    for (u64 tile = blockIdx.x; tile * T < n; tile += gridDim.x) {
+    const bool few = n <= (u64)S_RESIDENT * S_WAVES * S_FEW_BOARDS;
+    if (few) s_few_boards<V, LIST>(s.word, rg, A, L, n, &P->nList[l + 1], P, sum, t);
+    const u32 T = s_tile_boards(n, S_RESIDENT, 8, LEAF_WG);
+    for (u64 tile = blockIdx.x; !few && tile * T < n; tile += gridDim.x) {
         const u64 i = tile * T + threadIdx.x;
         const bool live = threadIdx.x < T && i < n;
         Pos b{};
