@@ -337,10 +337,11 @@ __device__ __forceinline__ void sum_children(u64 n, const u64 *__restrict__ off,
 // in the main loop they would hold up nearly every wave.
 //
 // Bound by the issue of VALU instructions.  From the start position,
-// perft(8) without merging (119 M boards, 2.4 G listed and counted moves of
-// ply 7) the kernel takes 21.9 ms; as a count of every reply from a board
-// that each lane made itself it took 50.1 ms, the same with the kin in LDS
-// 44.9 and with quiet moves as well 23.7.
+// perft(8) without merging (119 M boards, 3.2 G moves of ply 7) takes 20.1 ms,
+// 21.9 while all waves took their tiles from one counter, as in the figures
+// that follow.  As a count of every reply from a board that each lane made
+// itself it took 50.1 ms, the same with the kin in LDS 44.9, and with quiet
+// moves as well 23.7.
 //
 // No work-group barrier: working out the boards (a long chain, no listing)
 // and counting the replies overlap between the waves of a SIMD.  Four waves'
