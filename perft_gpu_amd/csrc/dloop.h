@@ -562,10 +562,10 @@ __global__ PG_LEAF_BOUNDS void kd_leaf_keys(
 template <int V, int D>
 __global__ __launch_bounds__(LEAF_WG) void kd_tiny(Plan *P, Tables t) {
     constexpr u32 WAVES = LEAF_WG / 64, PARTS = 32;
-    __shared__ u32 list[WAVES][3][256];
+    __shared__ u32 list[WAVES][3][WAVE_LIST];
     __shared__ u32 items;
     const u32 wave = wave_number(), lane = threadIdx.x & 63;
-    u32(&ls)[3][256] = list[wave];
+    u32(&ls)[3][WAVE_LIST] = list[wave];
     if (threadIdx.x == 0) items = 0;
     __syncthreads();
     const DLevel L = P->lv[0];
@@ -575,19 +575,19 @@ __global__ __launch_bounds__(LEAF_WG) void kd_tiny(Plan *P, Tables t) {
         const u64 ri = u / (units / L.n);
         const u32 part = (u32)(u % PARTS), part2 = (u32)(u / PARTS % PARTS);
         const Pos root = uniform_pos(L.b[ri]);
-        const u32 n = wave_words<V>(root, t, ls[0]);
+        const u32 n = wave_words<V>(root, t, ls[0], WAVE_LIST, &P->overflow);
         wave_sync();
         u32 sum = 0, moves;
         for (u32 i = part; i < n; i += PARTS) {
             const Pos c = wave_made(root, ls[0], i, t);
             if constexpr (D == 3) {
-                sum += wave_perft2<V>(c, ls[1], &moves, t);
+                sum += wave_perft2<V>(c, ls[1], &moves, &P->overflow, t);
                 listed += moves;
             } else {
-                const u32 m = wave_words<V>(c, t, ls[1]);
+                const u32 m = wave_words<V>(c, t, ls[1], WAVE_LIST, &P->overflow);
                 wave_sync();
                 for (u32 j = part2; j < m; j += PARTS) {
-                    sum += wave_perft2<V>(wave_made(c, ls[1], j, t), ls[2], &moves, t);
+                    sum += wave_perft2<V>(wave_made(c, ls[1], j, t), ls[2], &moves, &P->overflow, t);
                     listed += moves;
                 }
             }
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(2, 8)))
         u32 chunk = 0, rootMoves = 0;  // D == 4: the part's moves, 64 at a time, one in each lane
         do {
             if (D == 4) {
-                rootMoves = wave_words<V>(opaque_pos(uniform_pos(*rp)), t, s.word);
+                rootMoves = wave_words<V>(opaque_pos(uniform_pos(*rp)), t, s.word, LEAF_CAP, &P->overflow);
                 wave_sync();
                 lo = rootMoves * part / parts + chunk;
                 hi = rootMoves * (part + 1) / parts;
@@ -642,7 +642,7 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(2, 8)))
                         const u32 w = (u32)__builtin_amdgcn_readlane((int)mine, (int)lo);
                         p = made(p, (u16)w, piece_code(w >> 24), t);
                     }
-                    u32 m = wave_words<V>(p, t, s.word);
+                    u32 m = wave_words<V>(p, t, s.word, LEAF_CAP, &P->overflow);
                     wave_sync();
                     if (D == 3) {
                         if (at == 0) at = m * part / parts;

@@ -309,7 +309,7 @@ static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
     const Plan &h = sl.link->plan;
     *ms += (double)sl.link->ticks * sl.tickMs;
     *overflow = h.overflow != 0;
-    *leafItems += h.leafItems;
+    if (!*overflow) *leafItems += h.leafItems;  // (what did not fit is searched again)
     if (h.peak > *peak) *peak = h.peak;
     if (h.ovf) {
         set_error("batch: a perft total does not fit 64 bits");
@@ -329,6 +329,11 @@ static int run_split(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
     int rc = run_range(e, sl, sh, first, n, L0, top0, in, &over, leafItems, ms, peak);
     if (rc) return rc;
     if (!over) return PG_OK;
+    if (sh.small) {  // a board with more moves than the waves' lists hold: by levels
+        GraphShape general = sh;
+        general.small = 0;
+        return run_split(e, sl, general, first, n, L0, top0, Staged{nullptr, nullptr, in.out}, leafItems, ms, launches, splits, peak);
+    }
     if (n == 1) {
         set_error("one root does not fit the batch region (%zu bytes)", sl.regionBytes);
         return PG_ENOMEM;

@@ -409,15 +409,19 @@ __device__ __forceinline__ Pos opaque_pos(Pos p) {
 // lane works out the piece on its own square, an enemy slider's attacks or
 // one's own moves.  One lane that lists a board by itself (generate_words)
 // takes about four times as long, for it does one piece after the other.
+// Like every writer it counts on past its cap and stores nothing there.
 struct WaveSink {
     u32 *word;
-    u32 n, lane;
+    u32 cap, n, lane;
+    __device__ void put(u32 at, u32 w) {
+        if (at < cap) word[at] = w;
+    }
     __device__ void add(u32 m, u32 piece) {
-        if (lane == 0) word[n] = m | piece << 24;
+        if (lane == 0) put(n, m | piece << 24);
         n++;
     }
     template <class F> __device__ void squares(u64 m, u64, u32 piece, F &&f) {
-        if (m >> lane & 1) word[n + lanes_below(m)] = f((int)lane) | piece << 24;
+        if (m >> lane & 1) put(n + lanes_below(m), f((int)lane) | piece << 24);
         n += (u32)popc(m);
     }
     __device__ void skipped(u64) {}
@@ -461,28 +465,36 @@ __device__ __forceinline__ void wave_side_words(const Pos &p, const Tables &t, W
     const u32 piece = knight ? M_KNIGHT : (bishop ? M_BISHOP : 0u) | (rook ? M_ROOK : 0u);
     for (u64 left = __ballot(m != 0); left; left = __ballot(m != 0)) {
         if (m) {
-            o.word[o.n + lanes_below(left)] = mk_move((int)sq, ctz(m), MF_QUIET) | piece << 24;
+            o.put(o.n + lanes_below(left), mk_move((int)sq, ctz(m), MF_QUIET) | piece << 24);
             m &= m - 1;
         }
         o.n += (u32)popc(left);
     }
 }
-// out: room for the moves of any position
+// The number of words in out, which has room for cap.  A board with more moves
+// than that (218 are the most in a game, but a caller may set up one with more
+// queens than a game has) raises *full: the search is then to be run by the
+// kernels whose lists are sized by the counted moves.
+constexpr u32 WAVE_LIST = 256;
 template <int V>
-__device__ __forceinline__ u32 wave_words(const Pos &p, const Tables &t, u32 *out) {
-    WaveSink o{out, 0, threadIdx.x & 63};
+__device__ __forceinline__ u32 wave_words(const Pos &p, const Tables &t, u32 *out, u32 cap, u32 *full) {
+    WaveSink o{out, cap, 0, threadIdx.x & 63};
     if (pos_side(p)) wave_side_words<BLACK, V>(p, t, o);
     else wave_side_words<WHITE, V>(p, t, o);
-    return (u32)__builtin_amdgcn_readfirstlane((int)o.n);
+    const u32 n = (u32)__builtin_amdgcn_readfirstlane((int)o.n);
+    if (n <= cap) return n;
+    if (o.lane == 0) atomicOr(full, 1u);
+    return cap;
 }
 
-// perft(2) of one board by a whole wave: its moves are listed, then counted a
-// lane each.  Returns the lane's part; *moves: the board's moves.  About 5 us
+// perft(2) of one board by a whole wave: its moves are listed (list: WAVE_LIST
+// words), then counted a lane each.  Returns the lane's part; *moves: the
+// board's moves.  About 5 us
 // for a wave alone, where a tile of the fused leaf takes 25 and more, but
 // about ten times the instructions per board of a full tile.
 template <int V>
-__device__ __forceinline__ u32 wave_perft2(const Pos &b, u32 *list, u32 *moves, const Tables &t) {
-    const u32 m = wave_words<V>(b, t, list), lane = threadIdx.x & 63;
+__device__ __forceinline__ u32 wave_perft2(const Pos &b, u32 *list, u32 *moves, u32 *full, const Tables &t) {
+    const u32 m = wave_words<V>(b, t, list, WAVE_LIST, full), lane = threadIdx.x & 63;
     wave_sync();
     u32 sum = 0;
     for (u32 k = lane; k < m; k += 64) sum += count_any<V>(made(b, (u16)list[k], piece_code(list[k] >> 24), t), t);

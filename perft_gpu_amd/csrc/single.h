@@ -339,12 +339,12 @@ __global__ __launch_bounds__(LEAF_WG) void ks_one(SRoot r, SPlan *P, int depth, 
 constexpr u32 S_WAVES = LEAF_WG / 64;
 template <int V>
 __global__ __launch_bounds__(LEAF_WG) void ks_three(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ u32 list[S_WAVES][256];
+    __shared__ u32 list[S_WAVES][WAVE_LIST];
     SSum sum;
     const u32 wave = wave_number(), i = blockIdx.x * S_WAVES + wave;
     if (i < r.n) {
         u32 moves;
-        sum.total = wave_perft2<V>(uniform_pos(made(r.b, r.mv[i], r.piece[i], t)), list[wave], &moves, t);
+        sum.total = wave_perft2<V>(uniform_pos(made(r.b, r.mv[i], r.piece[i], t)), list[wave], &moves, &P->overflow, t);
         if ((threadIdx.x & 63) == 0) sum.items = sum.paths = moves;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
@@ -361,7 +361,7 @@ __device__ __forceinline__ Pos s_child_moves(u32 *list, const SRoot &r, SPlan *P
                                              const Tables &t) {
     const u32 i = blockIdx.x / parts, part = blockIdx.x % parts;
     const Pos c = uniform_pos(made(r.b, r.mv[i], r.piece[i], t));
-    const u32 n = wave_words<V>(c, t, list);
+    const u32 n = wave_words<V>(c, t, list, WAVE_LIST, &P->overflow);
     wave_sync();
     if (threadIdx.x == 0) {
         if (blockIdx.x == 0) atomicAdd(&P->paths[1], (u64)r.n);
@@ -376,14 +376,14 @@ __device__ __forceinline__ Pos s_child_moves(u32 *list, const SRoot &r, SPlan *P
 constexpr u32 S_FOUR_PARTS = 8, S_TOP_PARTS = 8;
 template <int V>
 __global__ __launch_bounds__(LEAF_WG) void ks_four(SRoot r, SPlan *P, u64 bias, SResult *out, u64 seq, Tables t) {
-    __shared__ u32 child[S_WAVES][256], list[S_WAVES][256];
+    __shared__ u32 child[S_WAVES][WAVE_LIST], list[S_WAVES][WAVE_LIST];
     SSum sum;
     const u32 wave = wave_number();
     u32 lo, hi;
     const Pos c = s_child_moves<V>(child[wave], r, P, S_FOUR_PARTS, &lo, &hi, t);
     for (u32 j = lo + wave; j < hi; j += S_WAVES) {
         u32 moves;
-        sum.total += wave_perft2<V>(wave_made(c, child[wave], j, t), list[wave], &moves, t);
+        sum.total += wave_perft2<V>(wave_made(c, child[wave], j, t), list[wave], &moves, &P->overflow, t);
         if ((threadIdx.x & 63) == 0) {
             sum.items += moves;
             sum.paths += moves;
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(LEAF_WG) void ks_four(SRoot r, SPlan *P, u64 bias, 
 // a wave per board of ply 2
 template <int V>
 __global__ __launch_bounds__(LEAF_WG) void ks_top(SRoot r, SPlan *P, SRegion rg, Tables t) {
-    __shared__ u32 child[S_WAVES][256], list[S_WAVES][256];
+    __shared__ u32 child[S_WAVES][WAVE_LIST], list[S_WAVES][WAVE_LIST];
     __shared__ u32 first, count[S_WAVES];
     __shared__ u64 base;
     const u32 wave = wave_number(), lane = threadIdx.x & 63;
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(LEAF_WG) void ks_top(SRoot r, SPlan *P, SRegion rg,
     u64 paths = 0;
     if (threadIdx.x == 0) first = lo < hi ? (u32)atomicAdd(&P->nNode[2], (u64)(hi - lo)) : 0;
     __syncthreads();
-    if (first + (hi - lo) > rg.node2) {  // cannot happen: node2 is the root's moves times the most a position has
+    if (first + (hi - lo) > rg.node2) {  // node2 is for games, in which no child has more than S_MOVES moves
         if (threadIdx.x == 0) P->overflow = 1;
         return;
     }
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(LEAF_WG) void ks_top(SRoot r, SPlan *P, SRegion rg,
         u32 m = 0;
         if (j < hi) {
             const Pos b = wave_made(c, child[wave], j, t);
-            m = wave_words<V>(b, t, list[wave]);
+            m = wave_words<V>(b, t, list[wave], WAVE_LIST, &P->overflow);
             if (lane == 0) L.node[node] = SNode{b, 1, S_NO_SLOT, 0};
         }
         if (lane == 0) count[wave] = m;
@@ -565,7 +565,8 @@ __device__ __forceinline__ void s_few_boards(u32 *word, const SRegion &rg, const
     __shared__ u32 count[S_WAVES];
     __shared__ u64 first;
     const u32 wave = wave_number(), lane = threadIdx.x & 63;
-    u32 *const list = word + wave * S_FEW_BOARDS * 256;
+    static_assert(S_WAVES * S_FEW_BOARDS * WAVE_LIST <= S_CAP, "the waves' lists share the window");
+    u32 *const list = word + wave * S_FEW_BOARDS * WAVE_LIST;
     const u32 each = s_tile_boards(n, S_RESIDENT * S_WAVES, 1, S_FEW_BOARDS);
     for (u64 i0 = (u64)blockIdx.x * S_WAVES * each; i0 < n; i0 += (u64)gridDim.x * S_WAVES * each) {
         const u64 mine = i0 + wave * each;
@@ -576,7 +577,7 @@ __device__ __forceinline__ void s_few_boards(u32 *word, const SRegion &rg, const
             if (k < each && mine + k < n) {
                 u64 w;
                 const Pos b = uniform_pos(s_board<LIST, true>(rg, A, L.node, mine + k, &w, t));
-                m[k] = wave_words<V>(b, t, list + k * 256);
+                m[k] = wave_words<V>(b, t, list + k * WAVE_LIST, WAVE_LIST, &P->overflow);
                 if (lane == 0) s_mad(&sum.paths, w, m[k], &sum.wide);
             }
             total += m[k];
@@ -598,7 +599,7 @@ __device__ __forceinline__ void s_few_boards(u32 *word, const SRegion &rg, const
 #pragma unroll
             for (u32 k = 0; k < S_FEW_BOARDS; k++) {
                 for (u32 j = lane; j < m[k]; j += 64) {
-                    const u32 w = list[k * 256 + j];
+                    const u32 w = list[k * WAVE_LIST + j];
                     L.mv[at + j] = (u16)w;
                     L.par[at + j] = (u32)(mine + k) | (u32)piece_code(w >> 24) << S_NODE_BITS;
                 }
