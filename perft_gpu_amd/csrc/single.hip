@@ -79,7 +79,7 @@ static void launch(Engine &e, const Single &s, const SRoot &r, const SRegion &rg
 }
 
 // perft of one root.  *fits is false (and nothing is returned) when a level
-// does not fit the arena.  collapse: merge the equal boards of each ply from
+// does not fit the arena, or a board's moves a list.  collapse: merge the equal boards of each ply from
 // the third on (two plies have no transpositions) of searches deep enough.
 int perft_single(Engine &e, const Pos &root, u32 depth, int v, bool collapse, u64 *out, bool *fits) {
     *fits = false;
@@ -94,10 +94,7 @@ int perft_single(Engine &e, const Pos &root, u32 depth, int v, bool collapse, u6
     r.b = root;
     u32 word[256];
     r.n = generate_words<SL_KOGGE>(root, ht->view(), word, 256, 0);
-    if (r.n > S_MOVES) {
-        set_error("the position has %u moves", r.n);
-        return PG_EINVAL;
-    }
+    if (r.n > S_MOVES) return PG_OK;  // more queens than a game has: the root's list does not hold them
     for (u32 i = 0; i < r.n; i++) {
         r.mv[i] = (u16)word[i];
         r.piece[i] = (u8)piece_code(word[i] >> 24);

@@ -24,6 +24,13 @@ def test_below_the_root(gdev, pg, v, depth):
     assert gdev.perft(W.CPW["start"], 5, v) == W.CPW_COUNTS["start"][5]
 
 
+@pytest.mark.parametrize("v", [0, 1, 2, 3])
+@pytest.mark.parametrize("depth", [1, 2, 3, 4])
+def test_at_the_root(gdev, pg, v, depth):
+    """More moves than pg_perft's kernels take of a root (218)."""
+    assert gdev.perft(WHITE, depth, v) == WHITE_COUNTS[depth]
+
+
 @pytest.mark.parametrize("n", [1, 3, 96, 130])
 @pytest.mark.parametrize("depth", [3, 4])
 def test_in_a_batch(gdev, pg, depth, n):
