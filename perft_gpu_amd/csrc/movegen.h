@@ -350,10 +350,16 @@ struct Sides {
     u64 occ, mine, enemy;
     u64 myPawns, myKnights, myBishops, myRooks, myKing;
     u64 ePawns, eKnights, eBishops, eRooks;
-    int k, ek;        // king squares, in range even for a board without a king
+    int k, ek;        // king squares, in range even for a board without a king (king_square)
     u32 castle, eCastle;  // castling rights of the side, of the enemy (2 bits each)
     u32 ep;               // en-passant file + 1
 };
+
+// The square of a king, or 31 if there is none (it was taken, on a board that
+// no game leads to).  ctz(0) is not defined: 31 is what it came to in the
+// kernels that hold a board per lane, but in scalar registers it is -1, the
+// compiler leaves out a mask after it, and tables were read 4 GB out of place.
+PG_HD int king_square(u64 kings) { return kings ? ctz(kings) : 31; }
 
 template <int C> PG_HD Sides sides_of(const Pos &p) {
     Sides s;
@@ -370,8 +376,8 @@ template <int C> PG_HD Sides sides_of(const Pos &p) {
     s.eKnights = side_of<1 - C>(p.knights, W);
     s.eBishops = side_of<1 - C>(p.bishopQueens, W);
     s.eRooks = side_of<1 - C>(p.rookQueens, W);
-    s.k = ctz(s.myKing) & 63;
-    s.ek = ctz(side_of<1 - C>(p.kings, W)) & 63;
+    s.k = king_square(s.myKing);
+    s.ek = king_square(side_of<1 - C>(p.kings, W));
     s.castle = (u32)(C == WHITE ? pos_wcastle(p) : pos_bcastle(p));
     s.eCastle = (u32)(C == WHITE ? pos_bcastle(p) : pos_wcastle(p));
     s.ep = (u32)pos_ep(p);
