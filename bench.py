@@ -52,7 +52,7 @@ HBM_PEAK_GBS = 8000.0
 # (profiles/leaf_by_difference.md)
 PROFILE_VALU_INSTS_PER_BOARD = 264
 PROFILE_SOURCE = "profiles/leaf_by_difference.md"
-LEAF_KERNEL = "k_leaf_moves<0>"
+LEAF_KERNEL = "k_leaf_moves<0, false>"
 COPY_BYTES = 1 << 30
 COPY_ITERS = 3
 

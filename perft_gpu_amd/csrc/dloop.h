@@ -52,6 +52,10 @@ struct Plan {
     u64 began;          // device clock at the search's start
     u32 arrived[TT_MAX_DEPTH];  // work-groups done with a level's kd_scan
     DLevel lv[TT_MAX_DEPTH];
+    // A root that no game leads to was seen (pos_regular): nothing is searched,
+    // and the host runs the search again with the plain leaf.  Kept from search
+    // to search: set by kd_begin, cleared by kd_end.
+    u64 irregular;
 };
 
 // A search's inputs and results in pinned host memory, which its first and
@@ -100,14 +104,15 @@ __device__ __forceinline__ void plan_offsets(Plan *P, DLevel &L) {
 
 // The first kernel: the plan and the roots come from the host, the roots are
 // counted (deeper levels get their counts from the expansion) and the table
-// of depth D is probed: hits are resolved before the expansion.
+// of depth D is probed: hits are resolved before the expansion.  check: the
+// leaf counts replies by difference, which not every root allows.
 template <int V>
 __global__ __launch_bounds__(wg_size<V>()) void kd_begin(Plan *P, const Link *H, TTView tt, int D, TTCounters *ctr,
-                                                         int small, Tables t) {
+                                                         int small, int check, Tables t) {
     stage_tables<V>(t);
     if (blockIdx.x == 0) {
         const u64 *from = (const u64 *)&H->plan;
-        for (u32 i = threadIdx.x; i < sizeof(Plan) / 8; i += blockDim.x) ((u64 *)P)[i] = from[i];
+        for (u32 i = threadIdx.x; i < offsetof(Plan, irregular) / 8; i += blockDim.x) ((u64 *)P)[i] = from[i];
         __syncthreads();
         if (threadIdx.x == 0) {
             P->began = wall_clock64();
@@ -124,6 +129,7 @@ __global__ __launch_bounds__(wg_size<V>()) void kd_begin(Plan *P, const Link *H,
             L.b[i] = b;
             if (L.k) L.k[i] = hk[i];
         }
+        if (check && !pos_regular(b)) atomicOr(&P->irregular, 1ULL);
         if (small) {
             L.perft[i] = bias;
             continue;
@@ -144,7 +150,7 @@ __global__ __launch_bounds__(wg_size<V>()) void kd_begin(Plan *P, const Link *H,
 }
 
 // The last kernel, one work-group: results and counters to the host.
-static __global__ __launch_bounds__(1024) void kd_end(const Plan *P, Link *H) {
+static __global__ __launch_bounds__(1024) void kd_end(Plan *P, Link *H) {
     const DLevel L = P->lv[0];
     u64 *const out = H->out;
     if (out)
@@ -156,6 +162,8 @@ static __global__ __launch_bounds__(1024) void kd_end(const Plan *P, Link *H) {
         h.ovf = P->ovf;
         h.leafItems = P->leafItems;
         h.peak = P->peak;
+        h.irregular = P->irregular;
+        P->irregular = 0;
         H->ticks = wall_clock64() - P->began;
     }
     __threadfence_system();
@@ -280,7 +288,7 @@ __device__ void plan_children(Plan *P, int l, int wantKeys, int wantSet, int tot
     memset(&C, 0, sizeof(C));
     L.keep = 0;
     const u64 m = L.n ? L.kids : 0;
-    if (m == 0 || m > 0xFFFFFFFFULL) {
+    if (m == 0 || m > 0xFFFFFFFFULL || P->irregular) {
         if (m) P->overflow = 1;
         return;
     }
@@ -488,6 +496,10 @@ static __global__ void kd_plan_live(Plan *P, int l) {
     if (threadIdx.x || blockIdx.x) return;
     if (l > 0) release_level(P, l - 1);  // the moves, parents and set that made level l
     DLevel &L = P->lv[l];
+    if (P->irregular) {
+        P->overflow = 1;
+        L.n = 0;
+    }
     P->liveN = 0;
     L.live = L.n && L.n <= 0xFFFFFFFFULL ? (u32 *)plan_try_alloc(P, L.n * 4) : nullptr;
 }
@@ -529,26 +541,26 @@ static __global__ __launch_bounds__(LIVE_WG) void kd_live(Plan *P, int l) {
 
 // perft(2) of the boards of level l, fused (see leaf_tiles), per board into
 // the level's perft array
-template <int V>
+template <int V, bool PLAIN>
 __global__ PG_LEAF_BOUNDS void kd_leaf(Plan *P, int l, Tables t) {
     const DLevel L = P->lv[l];
     const bool listed = L.live;
-    leaf_tiles<V, true>(L.b, L.cnt, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft, L.state,
-                        l == 0 ? P->bias : 0, &P->err, &P->ovf, t, listed ? L.live : nullptr);
+    leaf_tiles<V, true, false, PLAIN>(L.b, L.cnt, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft, L.state,
+                                      l == 0 ? P->bias : 0, &P->err, &P->ovf, t, listed ? L.live : nullptr);
 }
 
 // perft(2) of the children of level l-1 that form level l when level l keeps
 // keys only: the leaf makes each listed child from its parent and move (or,
 // without room for the list, every child, writing the live ones)
-template <int V>
+template <int V, bool PLAIN>
 __global__ PG_LEAF_BOUNDS void kd_leaf_keys(
     Plan *P, int l, Tables t) {
     const DLevel L = P->lv[l];
     const DLevel A = P->lv[l - 1];
     const bool listed = L.live != nullptr;
-    leaf_tiles<V, true, true>(A.b, nullptr, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft,
-                              listed ? nullptr : L.state, 0, &P->err, &P->ovf, t, listed ? L.live : nullptr, A.par,
-                              A.mv);
+    leaf_tiles<V, true, true, PLAIN>(A.b, nullptr, listed ? P->liveN : L.n, &P->acc, &P->leafItems, L.perft,
+                                     listed ? nullptr : L.state, 0, &P->err, &P->ovf, t, listed ? L.live : nullptr,
+                                     A.par, A.mv);
 }
 
 // Small searches without a table (depth 3 or 4): no levels in memory.  A wave
@@ -569,7 +581,7 @@ __global__ __launch_bounds__(LEAF_WG) void kd_tiny(Plan *P, Tables t) {
     if (threadIdx.x == 0) items = 0;
     __syncthreads();
     const DLevel L = P->lv[0];
-    const u64 units = uniform64(L.n) * (D == 3 ? PARTS : PARTS * PARTS);
+    const u64 n = P->irregular ? 0 : L.n, units = uniform64(n) * (D == 3 ? PARTS : PARTS * PARTS);
     u32 listed = 0;
     for (u64 u = blockIdx.x * WAVES + wave; u < units; u += gridDim.x * WAVES) {
         const u64 ri = u / (units / L.n);
@@ -608,7 +620,7 @@ __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(2, 8)))
     __shared__ LeafTile tiles[WAVES];
     const u32 wave = wave_number(), lane = threadIdx.x & 63;
     LeafTile &s = tiles[wave];
-    const u64 n = uniform64(P->lv[0].n);
+    const u64 n = uniform64(P->irregular ? 0 : P->lv[0].n);
     const u32 waves = gridDim.x * WAVES < LEAF_RESIDENT ? gridDim.x * WAVES : LEAF_RESIDENT;
     u32 parts = 1;
     while (parts < MOST && n * parts * 2 <= waves) parts *= 2;

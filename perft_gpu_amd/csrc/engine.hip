@@ -125,8 +125,9 @@ template <int V> static void launch_leaf_fused(Engine &c, const Pos *b, const u3
     if constexpr (V == SL_BYTE) {
         (void)c; (void)b; (void)cnt; (void)n;
     } else {
-        k_leaf_fused<V, false><<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(b, cnt, n, c.dAcc, c.dItems, nullptr, c.dErr,
-                                                                         c.dOvf, c.dt, nullptr);
+        const auto kernel = c.plainLeaf ? k_leaf_fused<V, false, true> : k_leaf_fused<V, false, false>;
+        kernel<<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(b, cnt, n, c.dAcc, c.dItems, nullptr, c.dErr, c.dOvf, c.dt,
+                                                         nullptr);
     }
 }
 
@@ -135,8 +136,8 @@ static void launch_leaf_moves(Engine &c, const Pos *gp, const u32 *par, const u1
     if constexpr (V == SL_BYTE) {
         (void)c; (void)gp; (void)par; (void)mv; (void)n;
     } else {
-        k_leaf_moves<V><<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(gp, par, mv, n, c.dAcc, c.dItems, c.dErr, c.dOvf,
-                                                                  c.dt);
+        const auto kernel = c.plainLeaf ? k_leaf_moves<V, true> : k_leaf_moves<V, false>;
+        kernel<<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(gp, par, mv, n, c.dAcc, c.dItems, c.dErr, c.dOvf, c.dt);
     }
 }
 
@@ -283,8 +284,10 @@ int Engine::perft(const Pos &root, u32 depth, int v, u64 *out) {
     // or the call must not allocate (its plan is created on first use).  The
     // collapsing search takes more arena per board of its last ply than the
     // plain one, so that is tried next; a search that fits neither way falls
-    // back to the host-driven loop below, which splits levels.
-    if (!timing && leafMode == 0 && graphPerft) {
+    // back to the host-driven loop below, which splits levels, and so does one
+    // from a root no game leads to.
+    plainLeaf = v != SL_BYTE && !pos_regular(root);
+    if (!timing && leafMode == 0 && graphPerft && !plainLeaf) {
         bool fits = false;
         int rc;
         if (v == SL_BYTE) {

@@ -28,9 +28,11 @@ struct GraphShape {
     int gmax;   // > 0: at most this many work-groups in any kernel (a small search's whole need)
     int leafMax;  // the same for the leaf, whose waves take a few boards each
     int small;  // searched without levels in memory: 1 kd_small, 2 kd_tiny
+    int plain;  // 1: the leaf makes each move (leaf_plain): a root no game leads to is among them
     bool operator==(const GraphShape &o) const {
         return depth == o.depth && v == o.v && keys == o.keys && dedup == o.dedup && bpc == o.bpc && tt == o.tt &&
-               total == o.total && cap == o.cap && gmax == o.gmax && leafMax == o.leafMax && small == o.small;
+               total == o.total && cap == o.cap && gmax == o.gmax && leafMax == o.leafMax && small == o.small &&
+               plain == o.plain;
     }
 };
 
@@ -97,7 +99,7 @@ static int leaf_need(const GraphShape &sh) { return sh.gmax * (sh.small == 2 ? 1
 // the graph of a served batch
 static GraphShape server_shape(const Engine &e, const TTable *tt, u64 n, int depth, int v, int dedup, int wgCap) {
     const int g = grid_limit(e, n, depth);
-    GraphShape sh{depth, v, 1, dedup ? 1 : 0, e.bpc, tt, 0, wgCap, g, 0, small_search(n, depth, v, tt)};
+    GraphShape sh{depth, v, 1, dedup ? 1 : 0, e.bpc, tt, 0, wgCap, g, 0, small_search(n, depth, v, tt), 0};
     sh.leafMax = leaf_need(sh);
     return sh;
 }
@@ -120,8 +122,8 @@ template <int V> static void cap_count(hipStream_t s, Plan *P, int g, const Tabl
     kd_count<V><<<g, wg_size<V>(), 0, s>>>(P, t);
 }
 template <int V> static void cap_begin(hipStream_t s, Plan *P, const Link *H, const TTView &tt, int D, TTCounters *ctr,
-                                       int small, int g, const Tables &t) {
-    kd_begin<V><<<g, wg_size<V>(), 0, s>>>(P, H, tt, D, ctr, small, t);
+                                       int small, int plain, int g, const Tables &t) {
+    kd_begin<V><<<g, wg_size<V>(), 0, s>>>(P, H, tt, D, ctr, small, V != SL_BYTE && D >= 2 && !plain, t);
 }
 template <int V> static void cap_generate(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
     kd_generate<V><<<g, wg_size<V>(), 0, s>>>(P, l, t);
@@ -130,15 +132,15 @@ template <int V> static void cap_expand(hipStream_t s, Plan *P, int l, const TTV
                                         const Tables &t) {
     kd_expand<V><<<g, wg_size<V>(), 0, s>>>(P, l, tt, rc, ctr, t);
 }
-template <int V> static void cap_leaf(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
-    if constexpr (V != SL_BYTE) kd_leaf<V><<<g, LEAF_WG, 0, s>>>(P, l, t);
+template <int V> static void cap_leaf(hipStream_t s, Plan *P, int l, int plain, int g, const Tables &t) {
+    if constexpr (V != SL_BYTE) (plain ? kd_leaf<V, true> : kd_leaf<V, false>)<<<g, LEAF_WG, 0, s>>>(P, l, t);
 }
 template <int V> static void cap_expand_keys(hipStream_t s, Plan *P, int l, const TTView &tt, int rc, TTCounters *ctr,
                                              int g, const Tables &t) {
     if constexpr (V != SL_BYTE) kd_expand_keys<V><<<g, wg_size<V>(), 0, s>>>(P, l, tt, rc, ctr, t);
 }
-template <int V> static void cap_leaf_keys(hipStream_t s, Plan *P, int l, int g, const Tables &t) {
-    if constexpr (V != SL_BYTE) kd_leaf_keys<V><<<g, LEAF_WG, 0, s>>>(P, l, t);
+template <int V> static void cap_leaf_keys(hipStream_t s, Plan *P, int l, int plain, int g, const Tables &t) {
+    if constexpr (V != SL_BYTE) (plain ? kd_leaf_keys<V, true> : kd_leaf_keys<V, false>)<<<g, LEAF_WG, 0, s>>>(P, l, t);
 }
 
 template <int V> static void cap_small(hipStream_t s, Plan *P, int depth, int tiny, int g, const Tables &t) {
@@ -178,7 +180,7 @@ static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, Link *H, con
         tt = sh.tt->view;
         ctr = sh.tt->dCtr;
     }
-    PG_VARIANT_CALL(v, cap_begin, s, P, H, tt, D, ctr, sh.small, gv, e.dt);
+    PG_VARIANT_CALL(v, cap_begin, s, P, H, tt, D, ctr, sh.small, sh.plain, gv, e.dt);
     if (sh.small) {
         PG_VARIANT_CALL(v, cap_small, s, P, D, sh.small == 2, gLeaf, e.dt);
         kd_end<<<1, 1024, 0, s>>>(P, H);
@@ -214,9 +216,9 @@ static void enqueue_search(const Engine &e, hipStream_t s, Plan *P, Link *H, con
         kd_plan_live<<<1, 64, 0, s>>>(P, last);
         kd_live<<<gWork, LIVE_WG, 0, s>>>(P, last);
         if (keysLast) {
-            PG_VARIANT_CALL(v, cap_leaf_keys, s, P, last, gLeaf, e.dt);
+            PG_VARIANT_CALL(v, cap_leaf_keys, s, P, last, sh.plain, gLeaf, e.dt);
         } else {
-            PG_VARIANT_CALL(v, cap_leaf, s, P, last, gLeaf, e.dt);
+            PG_VARIANT_CALL(v, cap_leaf, s, P, last, sh.plain, gLeaf, e.dt);
         }
     }
     for (int l = lastExpand; l >= 0; l--) {
@@ -292,9 +294,10 @@ struct Staged {
 };
 
 // Runs one batch (sub-range of the level-0 arrays; in.b: to be filled from
-// there); sets *overflow if it did not fit.
+// there); sets *overflow if it did not fit, *irregular if a root is among them
+// for which the leaf has to be the plain one.
 static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n, const DLevel &L0, size_t top0,
-                     const Staged &in, bool *overflow, u64 *leafItems, double *ms, u64 *peak) {
+                     const Staged &in, bool *overflow, bool *irregular, u64 *leafItems, double *ms, u64 *peak) {
     DLevel L = L0;
     L.b += first;
     if (L.k) L.k += first;
@@ -309,6 +312,8 @@ static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
     const Plan &h = sl.link->plan;
     *ms += (double)sl.link->ticks * sl.tickMs;
     *overflow = h.overflow != 0;
+    *irregular = h.irregular != 0;
+    if (*irregular) return PG_OK;
     if (!*overflow) *leafItems += h.leafItems;  // (what did not fit is searched again)
     if (h.peak > *peak) *peak = h.peak;
     if (h.ovf) {
@@ -324,14 +329,15 @@ static int run_range(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n
 
 static int run_split(Engine &e, Slot &sl, const GraphShape &sh, u64 first, u64 n, const DLevel &L0, size_t top0,
                      const Staged &in, u64 *leafItems, double *ms, u64 *launches, u64 *splits, u64 *peak) {
-    bool over = false;
+    bool over = false, irregular = false;
     (*launches)++;
-    int rc = run_range(e, sl, sh, first, n, L0, top0, in, &over, leafItems, ms, peak);
+    int rc = run_range(e, sl, sh, first, n, L0, top0, in, &over, &irregular, leafItems, ms, peak);
     if (rc) return rc;
-    if (!over) return PG_OK;
-    if (sh.small) {  // a board with more moves than the waves' lists hold: by levels
+    if (!over && !irregular) return PG_OK;
+    if (sh.small || irregular) {  // by levels: a board may have more moves than the waves' lists hold
         GraphShape general = sh;
         general.small = 0;
+        general.plain = irregular;
         return run_split(e, sl, general, first, n, L0, top0, Staged{nullptr, nullptr, in.out}, leafItems, ms, launches, splits, peak);
     }
     if (n == 1) {
@@ -353,6 +359,7 @@ int slot_init(Engine &e, Slot &sl, u8 *region, size_t bytes, hipStream_t stream)
     HIP_TRY(hipMalloc(&sl.dPlan, sizeof(Plan)));
     HIP_TRY(hipHostMalloc(&sl.link, sizeof(Link)));
     memset(sl.link, 0, sizeof(Link));
+    HIP_TRY(hipMemsetAsync(sl.dPlan, 0, sizeof(Plan), stream));
     int khz = 0;
     HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e.device));
     sl.tickMs = khz > 0 ? 1.0 / khz : 0;
@@ -408,7 +415,7 @@ int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fi
     h.top = 512;
     h.acc = e.bias;
     const int g = grid_limit(e, 1, (int)depth);
-    GraphShape sh{(int)depth, v, 0, 0, e.bpc, nullptr, 1, 0, g, g, 0};
+    GraphShape sh{(int)depth, v, 0, 0, e.bpc, nullptr, 1, 0, g, g, 0, 0};
     hipGraphExec_t exec;
     int rc = get_graph(e, sl, sh, &exec);
     if (rc) return rc;
@@ -508,7 +515,7 @@ int batch_perft(Engine &e, Slot &sl, TTable *tt, const Pos *roots, u64 n, u32 de
     // the default grid is the search's whole need; a set one holds for every kernel
     const int gmax = e.batchGrid >= 0 ? e.batchGrid : grid_limit(e, n, (int)depth);
     GraphShape sh{(int)depth, v, keys ? 1 : 0, dedup ? 1 : 0, bpc > 0 ? bpc : e.bpc, tt, 0, 0,
-                  gmax, 0, small_search(n, (int)depth, v, tt)};
+                  gmax, 0, small_search(n, (int)depth, v, tt), 0};
     sh.leafMax = e.batchGrid >= 0 ? gmax : leaf_need(sh);
     u64 leafItems = 0, launches = 0, splits = 0, peak = 0;
     double ms = 0;
@@ -831,18 +838,20 @@ int pg_server_poll(pg_server *s, uint32_t slot, uint64_t *out, pg_batch_stats *s
         return PG_EHIP;
     }
     const Plan h = sl.link->plan;
-    if (h.ovf) {
+    if (h.ovf && !h.irregular) {
         set_error("served batch: a perft total does not fit 64 bits");
         return PG_EOVERFLOW;
     }
-    if (h.err) {
+    if (h.err && !h.irregular) {
         set_error("device consistency check failed in served batch (flag %u)", h.err);
         return PG_EINVAL;
     }
     u64 items = h.leafItems, launches = 1, splits = 0, peak = h.peak;
     double ms = (double)sl.link->ticks * sl.tickMs;
-    if (h.overflow) {
-        const GraphShape sh = server_shape(e, s->tt, ss.n, (int)ss.depth, ss.v, ss.dedup, ss.wgCap);
+    if (h.overflow || h.irregular) {
+        GraphShape sh = server_shape(e, s->tt, ss.n, (int)ss.depth, ss.v, ss.dedup, ss.wgCap);
+        sh.plain = h.irregular != 0;
+        if (sh.plain) sh.small = 0;
         (void)hipSetDevice(e.device);
         items = 0;
         launches = 0;

@@ -14,6 +14,7 @@
 // All kernels are grid-stride loops sized to the CU count, so one launch
 // covers a level of any size; indices are 64-bit.
 #pragma once
+#include <type_traits>
 #include "movegen.h"
 
 namespace pg {
@@ -564,7 +565,7 @@ __device__ __forceinline__ u32 leaf_expand(LeafTile &s, bool live, const Pos &b,
         const u32 nCalm = n & 0xFFFF, nFull = n >> 16;
         wave_sync();
         for (u32 j = lane; j < nCalm; j += 64) {
-            const u32 w = s.word[j], o = w >> 16 & 255;
+            const u32 w = s.word[j], o = w >> 16 & (LEAF_TILE - 1);
             atomicAdd(&s.per[o], count_calm_any(s.k[o], w, t));
         }
         wave_sync();
@@ -587,7 +588,7 @@ __device__ __forceinline__ u32 leaf_expand(LeafTile &s, bool live, const Pos &b,
                 asides += (u32)__popcll(special);
             }
             if (j < nFull && !(w >> 31)) {
-                const u32 o = w >> 16 & 255;
+                const u32 o = w >> 16 & (LEAF_TILE - 1);
                 atomicAdd(&s.per[o], count_child_any<V>(s.k[o], w, t));
             }
         }
@@ -595,12 +596,48 @@ __device__ __forceinline__ u32 leaf_expand(LeafTile &s, bool live, const Pos &b,
         // those put aside, then (only if the list was full) the window's late ones
         const u32 m = asides < room ? asides : room, late = asides > room ? nFull : 0;
         for (u32 j = lane; j < m + late; j += 64) {
-            const u32 w = word[-(int)(j < m ? aside[j] : j - m)], o = w >> 16 & 255;
+            const u32 w = word[-(int)(j < m ? aside[j] : j - m)], o = w >> 16 & (LEAF_TILE - 1);
             if (j < m || (w & LEAF_LATE)) atomicAdd(&s.per[o], count_made<V>(s.k[o], w, t));
         }
         wave_sync();
     }
     return moves;
+}
+
+// The same by making every move and counting the replies from scratch, for
+// searches from a root no game leads to (pos_regular).  The window holds any
+// board's moves: a square is entered by sliders from at most eight sides, by
+// eight knights and by four pawn moves, three of which are four on the last
+// rank, and one king moves, which makes fewer than 1400.
+struct PlainTile {
+    Pos b[LEAF_TILE];
+    u32 word[LEAF_CAP];
+    u32 per[LEAF_TILE];
+};
+static_assert(LEAF_CAP >= 1400, "a board that does not fit the window would be put off for ever");
+template <int V>
+__device__ __forceinline__ u32 leaf_plain(PlainTile &s, bool live, const Pos &b, u32 *err, const Tables &t) {
+    const u32 lane = threadIdx.x & 63;
+    s.b[lane] = b;
+    s.per[lane] = 0;
+    const u32 c = live ? count_any<V>(b, t) : 0;
+    u32 total;
+    const u32 at = wave_excl_scan(c, &total);
+    for (u32 start = 0; start < total;) {
+        const bool due = c && at >= start, fits = due && at + c <= start + LEAF_CAP;
+        wave_sync();
+        if (fits && generate_words<V>(b, t, s.word + (at - start), c, lane) != c) atomicOr(err, 2u);
+        const u64 late = __ballot(due && !fits);
+        const u32 end = late ? __shfl(at, __builtin_ctzll(late), 64) : total;
+        wave_sync();
+        for (u32 j = start + lane; j < end; j += 64) {
+            const u32 w = s.word[j - start], o = w >> 16 & (LEAF_TILE - 1);
+            atomicAdd(&s.per[o], count_any<V>(made(s.b[o], (u16)w, piece_code(w >> 24), t), t));
+        }
+        start = end;
+    }
+    wave_sync();
+    return c;
 }
 
 // Boards per tile: too few boards for whole tiles on every CU are dealt out a
@@ -623,16 +660,18 @@ __device__ __forceinline__ u32 leaf_tile_boards(u64 n, u32 waves) {
 // them); the work-group makes each one and counts its moves itself, so the
 // level one above the leaf never goes to HBM.  With idx as well, the boards
 // made are those listed (j = idx[t]), and with PER their sums go to per[j].
-template <int V, bool PER, bool MOVES = false>
+// PLAIN: by leaf_plain.
+template <int V, bool PER, bool MOVES = false, bool PLAIN = false>
 __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const u32 *__restrict__ cnt, u64 n, u64 *acc,
                                            u64 *items, u64 *__restrict__ per, const u8 *__restrict__ state, u64 base,
                                            u32 *err, u32 *ovf, const Tables &t, const u32 *__restrict__ idx = nullptr,
                                            const u32 *__restrict__ par = nullptr, const u16 *__restrict__ mv = nullptr) {
     static_assert(V != SL_BYTE, "the byte-lookup tables leave no LDS for the move window");
     constexpr u32 WAVES = LEAF_WG / 64;
-    __shared__ LeafTile tiles[WAVES];
+    using Tile = std::conditional_t<PLAIN, PlainTile, LeafTile>;
+    __shared__ Tile tiles[WAVES];
     const u32 wave = wave_number();
-    LeafTile &s = tiles[wave];
+    Tile &s = tiles[wave];
     const u32 lane = threadIdx.x & 63;
     u64 sum = 0, itemSum = 0;
     n = uniform64(n);
@@ -653,7 +692,10 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
                 work = cnt[i] != 0;  // a board resolved earlier has count 0
             }
         }
-        itemSum += wave_sum32(leaf_expand<V>(s, work, b, err, t));
+        u32 c;
+        if constexpr (PLAIN) c = leaf_plain<V>(s, work, b, err, t);
+        else c = leaf_expand<V>(s, work, b, err, t);
+        itemSum += wave_sum32(c);
         if (live) {
             const u32 p = work ? s.per[lane] : 0;
             if constexpr (PER) {
@@ -678,28 +720,28 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
 // three waves per SIMD (see above); nothing spills at 168 registers
 #define PG_LEAF_BOUNDS __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(3, 8)))
 
-template <int V, bool PER>
+template <int V, bool PER, bool PLAIN>
 __global__ PG_LEAF_BOUNDS void k_leaf_fused(
     const Pos *__restrict__ boards, const u32 *__restrict__ cnt, u64 n, u64 *acc, u64 *items, u64 *__restrict__ per,
     u32 *err, u32 *ovf, Tables t, const u32 *__restrict__ idx) {
-    leaf_tiles<V, PER>(boards, cnt, n, acc, items, per, nullptr, 0, err, ovf, t, idx);
+    leaf_tiles<V, PER, false, PLAIN>(boards, cnt, n, acc, items, per, nullptr, 0, err, ovf, t, idx);
 }
 
 // the leaf over the children of `gp` listed by par/mv (see leaf_tiles, MOVES)
-template <int V>
+template <int V, bool PLAIN>
 __global__ PG_LEAF_BOUNDS void k_leaf_moves(
     const Pos *__restrict__ gp, const u32 *__restrict__ par, const u16 *__restrict__ mv, u64 n, u64 *acc, u64 *items,
     u32 *err, u32 *ovf, Tables t) {
-    leaf_tiles<V, false, true>(gp, nullptr, n, acc, items, nullptr, nullptr, 0, err, ovf, t, nullptr, par, mv);
+    leaf_tiles<V, false, true, PLAIN>(gp, nullptr, n, acc, items, nullptr, nullptr, 0, err, ovf, t, nullptr, par, mv);
 }
 
 // per-child sums over the children of `gp` listed by idx (see leaf_tiles,
 // MOVES with idx): perft(2) of each listed child into per[]
-template <int V>
+template <int V, bool PLAIN>
 __global__ PG_LEAF_BOUNDS void k_leaf_moves_per(
     const Pos *__restrict__ gp, const u32 *__restrict__ par, const u16 *__restrict__ mv, const u32 *__restrict__ idx,
     u64 n, u64 *items, u64 *__restrict__ per, u32 *err, u32 *ovf, Tables t) {
-    leaf_tiles<V, true, true>(gp, nullptr, n, nullptr, items, per, nullptr, 0, err, ovf, t, idx, par, mv);
+    leaf_tiles<V, true, true, PLAIN>(gp, nullptr, n, nullptr, items, per, nullptr, 0, err, ovf, t, idx, par, mv);
 }
 
 // ---------------------------------------------------------------- live list

@@ -1400,6 +1400,47 @@ PG_HD Key128 zobrist128(const Pos &p, const Tables &t) {
     return h;
 }
 
+// The men nearest to square k either way on a line through it.
+PG_HD u64 nearest(int k, u64 line, u64 occ) {
+    const u64 below = bit(k) - 1, up = line & occ & ~below & ~bit(k), down = line & occ & below;
+    return (up & (0 - up)) | (down & bit(63 - __builtin_clzll(down | 1)));
+}
+// Whether a board that pos_sane accepts is one that a game can be in, as far as
+// the moves go: one man per square, castling rights only where king and rook
+// stand at home, an en-passant field only behind an enemy pawn, and the side
+// not to move not in check.  Legal moves lead from such a board to such boards.
+// On others a king can be taken or a rook castle with no king, and the quiet
+// and calm moves are not what they are taken for: leaf_plain counts those.
+// (Straight through and without tables, for both sides: kd_begin asks it of
+// every root, and a batch waits for that.)
+PG_HD bool pos_regular(const Pos &p) {
+    const u64 occ = pos_occ(p), pawns = pos_pawns(p), sliders = p.bishopQueens | p.rookQueens;
+    const u64 twice = (pawns & (p.knights | sliders | p.kings)) | (p.knights & (sliders | p.kings)) | (sliders & p.kings);
+    // men that a castling right needs, and that are not there
+    const u64 rights = p.pawns & 15, wk = rights & 1, wq = rights >> 1 & 1, bk = rights >> 2 & 1, bq = rights >> 3;
+    const u64 rooks = p.rookQueens & ~p.bishopQueens;
+    const u64 away = ((wk | wq) << 4 & ~(p.kings & p.white)) | ((wk << 7 | wq) & ~(rooks & p.white)) |
+                     ((bk | bq) << 60 & ~(p.kings & ~p.white)) | ((bk << 63 | bq << 56) & ~(rooks & ~p.white));
+    const bool black = pos_side(p);
+    const u64 mine = black ? occ & ~p.white : p.white, king = p.kings & ~mine;
+    const int k = king_square(king);
+    const u64 checks = ((p.knights & knight_att(king)) | (p.kings & king_att(king)) |
+                        (pawns & (black ? pawn_att<WHITE>(king) : pawn_att<BLACK>(king))) |
+                        (p.rookQueens & (nearest(k, file_of(k), occ) | nearest(k, rank_of(k), occ))) |
+                        (p.bishopQueens & (nearest(k, diag_of(k), occ) | nearest(k, anti_of(k), occ)))) & mine;
+    u64 ep = 0;
+    if (const int f = pos_ep(p)) {
+        const u64 dst = black ? bit(15 + f) : bit(39 + f), pawn = black ? dst << 8 : dst >> 8;
+        ep = (occ & dst) | (pawn & ~(pawns & ~mine));
+        // a pawn that did not come by a double push may stand between a bishop
+        // and the king of the side that takes it
+        const int q = king_square(p.kings & mine);
+        const u64 seen = nearest(q, diag_of(q), occ & ~pawn) | nearest(q, anti_of(q), occ & ~pawn);
+        ep |= p.bishopQueens & ~mine & seen & ~(nearest(q, diag_of(q), occ) | nearest(q, anti_of(q), occ));
+    }
+    return (twice | away | checks | ep) == 0;
+}
+
 // side dispatch helpers
 template <int V>
 PG_HD u32 count_any(const Pos &p, const Tables &t) {

@@ -28,9 +28,10 @@ template <int V> static void launch_expand_tt(Engine &c, TTable &tt, const Pos *
 }
 template <int V>
 static void launch_leaf_per(Engine &c, const Pos *B, const u32 *cnt, u64 n, u64 *P, const u32 *idx) {
-    if constexpr (V != SL_BYTE)
-        k_leaf_fused<V, true><<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(B, cnt, n, c.dAcc, c.dItems, P, c.dErr, c.dOvf,
-                                                                        c.dt, idx);
+    if constexpr (V != SL_BYTE) {
+        const auto kernel = c.plainLeaf ? k_leaf_fused<V, true, true> : k_leaf_fused<V, true, false>;
+        kernel<<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(B, cnt, n, c.dAcc, c.dItems, P, c.dErr, c.dOvf, c.dt, idx);
+    }
 }
 template <int V> static void launch_expand_keys(Engine &c, TTable &tt, const Pos *B, const Key128 *K, const u32 *par,
                                                 const u16 *mv, u64 m, Key128 *CK, u64 *CP, u8 *S, int rc) {
@@ -41,9 +42,10 @@ template <int V> static void launch_expand_keys(Engine &c, TTable &tt, const Pos
 }
 template <int V>
 static void launch_leaf_moves_per(Engine &c, const Pos *B, const u32 *par, const u16 *mv, const u32 *idx, u64 n, u64 *P) {
-    if constexpr (V != SL_BYTE)
-        k_leaf_moves_per<V><<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(B, par, mv, idx, n, c.dItems, P, c.dErr, c.dOvf,
-                                                                      c.dt);
+    if constexpr (V != SL_BYTE) {
+        const auto kernel = c.plainLeaf ? k_leaf_moves_per<V, true> : k_leaf_moves_per<V, false>;
+        kernel<<<c.leaf_grid(n), LEAF_WG, 0, c.stream>>>(B, par, mv, idx, n, c.dItems, P, c.dErr, c.dOvf, c.dt);
+    }
 }
 template <int V> static void launch_gen(Engine &c, const Pos *b, u64 n, const u64 *off, u16 *mv, u32 *par) {
     constexpr int W = wg_size<V>();
@@ -265,6 +267,7 @@ int Engine::perft_tt(TTable &tt, const Pos &root, u32 depth, int v, u64 *out) {
     const HostTables *ht = host_tables(nullptr);
     if (!ht) return PG_ETABLE;
     const Key128 key = zobrist128(root, ht->view());
+    plainLeaf = v != SL_BYTE && !pos_regular(root);
     // device scratch: board, key, count, perft, probe result
     u8 *d = (u8 *)alloc(256);
     if (!d) return PG_ENOMEM;
