@@ -13,6 +13,7 @@ struct Single {
     SPlan *plan = nullptr;
     SResult *res = nullptr;  // pinned; the last kernel of a search writes it
     u64 seq = 0;
+    bool clear = false;      // the counters are zero: the last search ended with its last kernel
 };
 
 int single_init(Engine &e) {
@@ -21,7 +22,6 @@ int single_init(Engine &e) {
     HIP_TRY(hipMalloc(&s.plan, sizeof(SPlan)));
     HIP_TRY(hipHostMalloc(&s.res, sizeof(SResult)));
     memset(s.res, 0, sizeof(SResult));
-    HIP_TRY(hipMemset(s.plan, 0, sizeof(SPlan)));
     return PG_OK;
 }
 
@@ -107,11 +107,15 @@ int perft_single(Engine &e, const Pos &root, u32 depth, int v, bool collapse, u6
     if (collapse && depth >= 6)
         for (u32 l = 3; l + 2 <= depth; l++) rg.collapse |= 1ULL << l;
     if (depth >= 5 && rg.node2 * sizeof(SNode) > rg.bytes / 2) return PG_OK;
+    // before the first search, and after one that broke off
+    if (!s.clear) HIP_TRY(hipMemsetAsync(s.plan, 0, sizeof(SPlan), e.stream));
+    s.clear = false;
     s.seq++;
     PG_VARIANT_CALL_LDS(v, launch, e, s, r, rg, (int)depth, e.bias);
     HIP_TRY(hipGetLastError());
     const int rc = wait_result(e, s);
     if (rc) return rc;
+    s.clear = true;
     const SResult &h = *s.res;
     if (h.overflow) return PG_OK;
     if (h.ovf) {
