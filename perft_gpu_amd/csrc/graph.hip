@@ -392,17 +392,24 @@ void slot_forget_tt(Slot &sl, const TTable *tt) {
     }
 }
 
+// the context's own slot (nothing half made is kept)
+static int batch_slot(Engine &e) {
+    if (e.batchSlot) return PG_OK;
+    Slot *sl = new Slot();
+    const int rc = slot_init(e, *sl, e.arena, e.arenaBytes, e.stream);
+    if (rc) slot_delete(sl);
+    else e.batchSlot = sl;
+    return rc;
+}
+
 // perft of one root through a total-only graph on the context's batch slot
 // (the byte-lookup variant): no host round trip between levels.  *fits is false (and nothing is
 // returned) when a level does not fit the arena; the caller then runs the
 // host-driven search, which splits levels.
 int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fits) {
     *fits = false;
-    if (!e.batchSlot) {
-        e.batchSlot = new Slot();
-        const int rc = slot_init(e, *e.batchSlot, e.arena, e.arenaBytes, e.stream);
-        if (rc) return rc;
-    }
+    int rc = batch_slot(e);
+    if (rc) return rc;
     Slot &sl = *e.batchSlot;
     Plan &h = sl.link->plan;
     memset(&h, 0, sizeof(Plan));
@@ -417,7 +424,7 @@ int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fi
     const int g = grid_limit(e, 1, (int)depth);
     GraphShape sh{(int)depth, v, 0, 0, e.bpc, nullptr, 1, 0, g, g, 0, 0};
     hipGraphExec_t exec;
-    int rc = get_graph(e, sl, sh, &exec);
+    rc = get_graph(e, sl, sh, &exec);
     if (rc) return rc;
     HIP_TRY(hipMemcpyAsync(sl.dPlan, &h, sizeof(Plan), hipMemcpyHostToDevice, sl.stream));
     Pos *staged = reinterpret_cast<Pos *>(e.hostBuf + 8);
@@ -567,11 +574,8 @@ int pg_perft_batch(pg_ctx *ctx, const pg_pos48 *pos, uint32_t n, uint32_t depth,
             return PG_EINVAL;
         }
     (void)hipSetDevice(e->device);
-    if (!e->batchSlot) {
-        e->batchSlot = new Slot();
-        int rc = slot_init(*e, *e->batchSlot, e->arena, e->arenaBytes, e->stream);
-        if (rc) return rc;
-    }
+    const int rc = batch_slot(*e);
+    if (rc) return rc;
     return batch_perft(*e, *e->batchSlot, t, roots.data(), n, depth, v, dedup, blocks_per_cu,
                        reinterpret_cast<u64 *>(out), st);
 }

@@ -2,6 +2,7 @@
 // the slider variants whose tables leave the LDS to the fused leaf.
 #include <chrono>
 #include <cstring>
+#include <memory>
 #include "engine.h"
 #include "single.h"
 
@@ -16,20 +17,21 @@ struct Single {
     bool clear = false;      // the counters are zero: the last search ended with its last kernel
 };
 
-int single_init(Engine &e) {
-    e.single = new Single();
-    Single &s = *e.single;
-    HIP_TRY(hipMalloc(&s.plan, sizeof(SPlan)));
-    HIP_TRY(hipHostMalloc(&s.res, sizeof(SResult)));
-    memset(s.res, 0, sizeof(SResult));
-    return PG_OK;
-}
-
 void single_delete(Single *s) {
     if (!s) return;
     if (s->plan) (void)hipFree(s->plan);
     if (s->res) (void)hipHostFree(s->res);
     delete s;
+}
+
+// (nothing half made is kept)
+static int single_init(Engine &e) {
+    std::unique_ptr<Single, void (*)(Single *)> s(new Single(), single_delete);
+    HIP_TRY(hipMalloc(&s->plan, sizeof(SPlan)));
+    HIP_TRY(hipHostMalloc(&s->res, sizeof(SResult)));
+    memset(s->res, 0, sizeof(SResult));
+    e.single = s.release();
+    return PG_OK;
 }
 
 // Waits for the result: the last work-group writes it to pinned memory, which
