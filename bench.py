@@ -12,8 +12,9 @@ boards of a ply merged, which is what pg_perft does by default.
 
 Prints one JSON line: leaves/s over the timed steps, per-variant timings,
 the leaf kernel's roofline (integer VALU issue against the chip's vector
-peak, HBM bytes beside it) and the CPU baseline (the reference's own CPU
-perft compiled from its sources, timed on this host on a bounded sample).
+peak, HBM bytes beside it), the CPU baseline (the reference's own CPU
+perft compiled from its sources, timed on this host on a bounded sample) and
+the main figures of the legs, whose full results go to --report FILE.
 Legs beside the headline (--legs, comma list):
   counters   two rocprofv3 --pmc passes over one step of this workload plus
              the calib leg in a child process: VALU instructions per counted
@@ -283,6 +284,8 @@ def leg_counters(pg, dev=None):
     child = [sys.executable, os.path.join(ROOT, "bench.py"), "--steps", "1", "--warmup", "0", "--no-cpu",
              "--legs", "calib", "--variant", "0"]
     work = tempfile.mkdtemp(prefix="pg_counters_", dir="/tmp")
+    report = os.path.join(work, "report.json")
+    child += ["--report", report]
     sums, disp, child_line = {}, {}, None
     env = dict(os.environ, TMPDIR="/tmp")
     try:
@@ -292,9 +295,9 @@ def leg_counters(pg, dev=None):
                                                                           "csv", "--"] + child
             log("counters pass %d: %s" % (i + 1, " ".join(ctrs)))
             r = subprocess.run(cmd, capture_output=True, text=True, cwd="/tmp", env=env)
-            lines = [x for x in r.stdout.splitlines() if x.startswith("{")]
-            if lines:
-                child_line = json.loads(lines[-1])
+            if os.path.exists(report):
+                with open(report) as f:
+                    child_line = json.load(f)
             s_, d_ = _read_counters(out)
             if not s_:
                 return {"measured": False, "reason": "rocprofv3 pass %d gave no counters (rc %d): %s"
@@ -425,6 +428,49 @@ def leg_serve(pg, dev):
             "exact": True}
 
 
+def _pick(d, *keys):
+    return {k: d[k] for k in keys if k in d}
+
+
+def _round(x):
+    """Floats to six digits, throughout."""
+    if isinstance(x, float):
+        return float("%.6g" % x)
+    if isinstance(x, dict):
+        return {k: _round(v) for k, v in x.items()}
+    return [_round(v) for v in x] if isinstance(x, list) else x
+
+
+def summary(line):
+    """The result line of a full report: whole but for the legs, of which the
+    figures that are quoted stay (the report itself is 16 KB and more, too
+    long for a line that is read back; --report keeps it)."""
+    out = {k: v for k, v in line.items() if k not in ("counters", "calib", "batch", "tt", "serve", "leafmodes")}
+    roof = dict(line["roofline"])
+    roof["hbm"] = _pick(roof["hbm"], "achieved", "peak", "unit", "frac")
+    out["roofline"] = {k: v for k, v in roof.items() if not k.endswith("_note")}
+    if "counters" in line:
+        out["counters"] = _pick(line["counters"], "measured", "reason", "valu_insts_per_board",
+                                "valu_wave_insts_per_cu_per_cycle", "valu_busy_per_simd", "dual_issue_fraction",
+                                "lane_utilization", "hbm_bytes_per_launch", "algorithmic_bytes_per_launch")
+    if "calib" in line:
+        out["calib"] = {"copy_gb_per_s": line["calib"]["copy"]["gb_per_s_read_plus_write"], "cus": line["calib"]["cus"]}
+    if "batch" in line:
+        out["batch"] = _pick(line["batch"], "workload", "ms", "leaves_per_s", "autotuned", "speedup_vs_plain_loop", "exact")
+    if "tt" in line:
+        out["tt"] = {"workload": line["tt"]["workload"], "exact": line["tt"]["exact"],
+                     "runs": [_pick(r, "tt_gb", "depth", "s", "effective_leaves_per_s") for r in line["tt"]["runs"]]}
+    if "serve" in line:
+        s, row = line["serve"], ("rate_per_s", "queries", "leaves_per_s", "p50_ms", "p99_ms")
+        out["serve"] = {"rates": [dict(_pick(r, *row), p99_ms_by_depth={d: q["p99_ms"] for d, q in r["by_depth"].items()})
+                                  for r in s["rates"]],
+                        "burst_without_table": _pick(s["burst_without_table"], *row),
+                        "burst_vs_plain": s["burst_vs_plain"], "exact": s["exact"]}
+    if "leafmodes" in line:
+        out["leafmodes"] = [_pick(r, "leaf_mode", "slider", "depth", "s") for r in line["leafmodes"]["rows"]]
+    return _round(out)
+
+
 def cpu_model():
     try:
         out = subprocess.run(["lscpu"], capture_output=True, text=True).stdout
@@ -473,6 +519,7 @@ def main():
     ap.add_argument("--legs", default="counters,calib,batch,tt,serve",
                     help="legs beside the headline (comma list, or none): counters, calib, batch, tt, serve, leafmodes")
     ap.add_argument("--tt-gb", default="16,64", help="table sizes of the tt leg (GB, comma list)")
+    ap.add_argument("--report", help="file for the full report (the printed line holds its main figures)")
     ap.add_argument("--tt-depths", default="9,10", help="depths of the tt leg (comma list)")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
@@ -611,7 +658,10 @@ def main():
         r1k = [r for r in line["serve"]["rates"] if r["rate_per_s"] == 1000][0]
         line["served_p50_ms"] = r1k["p50_ms"]
         line["served_p99_ms"] = r1k["p99_ms"]
-    print(json.dumps(line))
+    if args.report:
+        with open(args.report, "w") as f:
+            json.dump(line, f)
+    print(json.dumps(summary(line)))
 
 
 if __name__ == "__main__":
