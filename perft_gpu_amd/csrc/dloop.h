@@ -90,8 +90,6 @@ __device__ __forceinline__ void *plan_try_alloc(Plan *P, u64 bytes) {
     return P->base + a;
 }
 
-#define PG_GRID_LOOP_N(i, n) PG_GRID_LOOP(i, n)
-
 // room for the offsets of a level that will be expanded
 __device__ __forceinline__ void plan_offsets(Plan *P, DLevel &L) {
     L.off = nullptr;
@@ -171,13 +169,12 @@ static __global__ __launch_bounds__(1024) void kd_end(Plan *P, Link *H) {
     if (threadIdx.x == 0) __hip_atomic_store(&H->seq, H->want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// level-0 move counts of a total-only search
-template <int V>
-__global__ __launch_bounds__(wg_size<V>()) void kd_count(Plan *P, Tables t) {
-    stage_tables<V>(t);
+// level-0 move counts of a total-only search (the byte-lookup variant)
+static __global__ __launch_bounds__(wg_size<SL_BYTE>()) void kd_count(Plan *P, Tables t) {
+    stage_tables<SL_BYTE>(t);
     const DLevel L = P->lv[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) plan_offsets(P, P->lv[0]);
-    PG_GRID_LOOP(i, L.n) L.cnt[i] = count_any<V>(L.b[i], t);
+    PG_GRID_LOOP(i, L.n) L.cnt[i] = count_any<SL_BYTE>(L.b[i], t);
 }
 
 static __global__ __launch_bounds__(256) void kd_root_store(Plan *P, TTView tt, int D, TTCounters *ctr) {

@@ -118,9 +118,6 @@ struct Slot {
     std::vector<BatchGraph> graphs;
 };
 
-template <int V> static void cap_count(hipStream_t s, Plan *P, int g, const Tables &t) {
-    kd_count<V><<<g, wg_size<V>(), 0, s>>>(P, t);
-}
 template <int V> static void cap_begin(hipStream_t s, Plan *P, const Link *H, const TTView &tt, int D, TTCounters *ctr,
                                        int small, int plain, int g, const Tables &t) {
     kd_begin<V><<<g, wg_size<V>(), 0, s>>>(P, H, tt, D, ctr, small, V != SL_BYTE && D >= 2 && !plain, t);
@@ -156,15 +153,15 @@ template <int V> static void cap_small(hipStream_t s, Plan *P, int depth, int ti
 // variant (the others run single.hip): per level just boards and counts (no
 // keys, table or per-board sums), down to the boards whose counts are summed.
 static void enqueue_total(const Engine &e, hipStream_t s, Plan *P, const GraphShape &sh) {
-    const int D = sh.depth, v = sh.v;
+    const int D = sh.depth;
     const Grids G = grids_for(e, sh);
     const int gWork = G.work, gScan = G.scan, gv = G.v;
-    PG_VARIANT_CALL(v, cap_count, s, P, gv, e.dt);
+    kd_count<<<gv, wg_size<SL_BYTE>(), 0, s>>>(P, e.dt);
     for (int l = 0; l <= D - 2; l++) {
         kd_scan<<<std::min(gScan, 512), GEN_WG, 0, s>>>(P, l, 0, 0, 1, l + 1 <= D - 2);
         kd_offsets<<<gScan, GEN_WG, 0, s>>>(P, l);
-        PG_VARIANT_CALL(v, cap_generate, s, P, l, gv, e.dt);
-        PG_VARIANT_CALL(v, cap_expand, s, P, l, TTView{}, D - l - 1, (TTCounters *)nullptr, gv, e.dt);
+        cap_generate<SL_BYTE>(s, P, l, gv, e.dt);
+        cap_expand<SL_BYTE>(s, P, l, TTView{}, D - l - 1, nullptr, gv, e.dt);
     }
     kd_sum_counts<<<gWork, 256, 0, s>>>(P, D - 1);
 }
