@@ -620,13 +620,14 @@ __device__ __forceinline__ u32 leaf_plain(PlainTile &s, bool live, const Pos &b,
     const u32 lane = threadIdx.x & 63;
     s.b[lane] = b;
     s.per[lane] = 0;
-    const u32 c = live ? count_any<V>(b, t) : 0;
+    wave_sync();
+    const u32 c = live ? count_any<V>(s.b[lane], t) : 0;
     u32 total;
     const u32 at = wave_excl_scan(c, &total);
     for (u32 start = 0; start < total;) {
         const bool due = c && at >= start, fits = due && at + c <= start + LEAF_CAP;
         wave_sync();
-        if (fits && generate_words<V>(b, t, s.word + (at - start), c, lane) != c) atomicOr(err, 2u);
+        if (fits && generate_words<V>(s.b[lane], t, s.word + (at - start), c, lane) != c) atomicOr(err, 2u);
         const u64 late = __ballot(due && !fits);
         const u32 end = late ? __shfl(at, __builtin_ctzll(late), 64) : total;
         wave_sync();
