@@ -415,7 +415,7 @@ __global__ __launch_bounds__(wg_size<V>()) void kd_expand_keys(Plan *P, int l, T
         }
         C.k[i] = h;
         C.state[i] = hit ? ST_HIT : ST_LIVE;
-        if (hit) C.perft[i] = v;  // the leaf writes the live children's, the resolve the duplicates'
+        if (hit) C.perft[i] = v;  // the leaf writes the live children's; duplicates have their owners'
     }
 }
 
@@ -560,14 +560,14 @@ __global__ PG_LEAF_BOUNDS void kd_leaf_keys(
                                      A.par, A.mv);
 }
 
-// Small searches without a table (depth 3 or 4): no levels in memory.  A wave
-// takes a part of a root's moves, lists the boards of ply D-2 below them, a
-// tile at a time (wave_words lists one board's moves), and hands the tile to
-// the fused leaf; kd_begin has set the results to the bias.  What the level
-// loop spends on such a search is mostly its kernels of 3 to 5 us each, ten
-// per level.
-// The same for so few roots that every board of ply D-2 can have a wave of its
-// own (wave_perft2).
+// Small searches without a table (depth 3 or 4): no levels in memory.  What the
+// level loop spends on such a search is mostly its kernels of 3 to 5 us each,
+// four per level and more.  kd_begin has set the results to the bias.  A board
+// with more moves than a wave's list holds raises overflow, and the host runs
+// the level loop.
+//
+// kd_tiny: so few roots that every board of ply D-2 can have a wave of its own
+// (wave_perft2).
 template <int V, int D>
 __global__ __launch_bounds__(LEAF_WG) void kd_tiny(Plan *P, Tables t) {
     constexpr u32 WAVES = LEAF_WG / 64, PARTS = 32;
@@ -610,6 +610,9 @@ __global__ __launch_bounds__(LEAF_WG) void kd_tiny(Plan *P, Tables t) {
     if (threadIdx.x == 0 && items) atomicAdd(&P->leafItems, (u64)items);
 }
 
+// kd_small: a wave takes a part of a root's moves, lists the boards of ply D-2
+// below them, a tile at a time (wave_words lists one board's moves), and hands
+// the tile to the fused leaf.
 template <int V, int D>
 __global__ __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(2, 8))) void kd_small(Plan *P, Tables t) {
     static_assert(D == 3 || D == 4, "two plies end in the leaf");

@@ -57,7 +57,7 @@ struct Engine {
     u64 *dAcc = nullptr;
     u64 *dItems = nullptr;   // items consumed by fused leaf launches
     int leafMode = 0;        // 0 fused last two plies, 1 materialized item list
-    bool graphPerft = true;  // pg_perft may run as one graph launch
+    bool graphPerft = true;  // pg_perft may run other than by host-driven levels (which allocates)
     bool plainLeaf = false;  // the search under way starts from a root no game leads to (pos_regular)
     int batchGrid = -1;      // work-groups per kernel of pg_perft_batch: -1 sized to the batch, 0 whole chip
     u32 *dErr = nullptr;

@@ -37,11 +37,12 @@ struct GraphShape {
 };
 
 // Whether n roots to `depth` are searched without levels in memory.  Measured
-// time of the graph in us, level loop / kd_small / kd_tiny: depth 3, 1 root
-// 79 / 34 / 21, 16 roots 98 / 39 / 25, 61 roots 111 / 38 / 28, 250 roots 127 /
-// 40 / -, 1000 roots 152 / 57 / -, 4096 roots 205 / 235 / -; depth 4, 1 root
-// 122 / 83 / 38, 4 roots 151 / 124 / 76, 61 roots 231 / 149 / -, 250 roots
-// 357 / 405 / -.
+// time of the graph in us, level loop / kd_small / kd_tiny, random positions of
+// plies 0 to 60: depth 3, 1 root 53 / 33 / 19, 16 roots 92 / 45 / 26, 128 roots
+// 107 / 40 / 36, 250 roots 108 / 41 / 55, 1536 roots 140 / 81 / 206; depth 4, 1
+// root 95 / 33 / 25, 6 roots 132 / 112 / 101, 61 roots 201 / 133 / 426, 96 roots
+// 205 / 132 / 536, 250 roots 305 / 343 / 1240.  (The upper lines leave a margin:
+// a few roots with many moves are one wave's each.)
 static int small_search(u64 n, int depth, int v, const TTable *tt) {
     if (tt || v == SL_BYTE || (depth != 3 && depth != 4)) return 0;
     if (n <= (depth == 3 ? 128 : 6)) return 2;
@@ -70,7 +71,8 @@ struct Grids {
 };
 static Grids grids_for(const Engine &e, const GraphShape &sh) {
     // a capped search keeps at most sh.cap work-groups per CU of each kernel
-    // resident (four fit per CU), so batches on other streams find room
+    // resident (four of most kernels fit per CU, three of the leaf), so batches
+    // on other streams find room
     const int wpc = sh.cap > 0 && sh.cap < sh.bpc ? sh.cap : sh.bpc;
     Grids g;
     g.work = e.cus * wpc;
@@ -400,9 +402,9 @@ static int batch_slot(Engine &e) {
 }
 
 // perft of one root through a total-only graph on the context's batch slot
-// (the byte-lookup variant): no host round trip between levels.  *fits is false (and nothing is
-// returned) when a level does not fit the arena; the caller then runs the
-// host-driven search, which splits levels.
+// (the byte-lookup variant): no host round trip between levels.  *fits is
+// false (and nothing is returned) when a level does not fit the arena; the
+// caller then runs the host-driven search, which splits levels.
 int perft_graph(Engine &e, const Pos &root, u32 depth, int v, u64 *out, bool *fits) {
     *fits = false;
     int rc = batch_slot(e);

@@ -490,9 +490,9 @@ __device__ __forceinline__ u32 wave_words(const Pos &p, const Tables &t, u32 *ou
 
 // perft(2) of one board by a whole wave: its moves are listed (list: WAVE_LIST
 // words), then counted a lane each.  Returns the lane's part; *moves: the
-// board's moves.  About 5 us
-// for a wave alone, where a tile of the fused leaf takes 25 and more, but
-// about ten times the instructions per board of a full tile.
+// board's moves.  A launch that does this takes 16 us (ks_three), where one
+// with a tile of the fused leaf takes 28, but it is about ten times the
+// instructions per board of a full tile.
 template <int V>
 __device__ __forceinline__ u32 wave_perft2(const Pos &b, u32 *list, u32 *moves, u32 *full, const Tables &t) {
     const u32 m = wave_words<V>(b, t, list, WAVE_LIST, full), lane = threadIdx.x & 63;
@@ -642,8 +642,8 @@ __device__ __forceinline__ u32 leaf_plain(PlainTile &s, bool live, const Pos &b,
 }
 
 // Boards per tile: too few boards for whole tiles on every CU are dealt out a
-// few at a time, for the time of the longest tile (a wave alone takes about
-// 15 us for one).
+// few at a time, for the time of the longest tile (a launch of one tile of 4
+// middle-game boards takes 28 us).
 constexpr u32 LEAF_RESIDENT = 3072;  // waves the chip holds
 __device__ __forceinline__ u32 leaf_tile_boards(u64 n, u32 waves) {
     if (waves > LEAF_RESIDENT) waves = LEAF_RESIDENT;
@@ -718,7 +718,8 @@ __device__ __forceinline__ void leaf_tiles(const Pos *__restrict__ boards, const
     }
 }
 
-// three waves per SIMD (see above); nothing spills at 168 registers
+// three waves per SIMD (see above): at 168 registers no vector register spills;
+// 5 to 67 scalar ones are kept in the lanes of vector registers
 #define PG_LEAF_BOUNDS __launch_bounds__(LEAF_WG) __attribute__((amdgpu_waves_per_eu(3, 8)))
 
 template <int V, bool PER, bool PLAIN>

@@ -771,7 +771,8 @@ PG_HD Gen gen_all(const Sides &s, const Tables &t) {
                castle_moves<C>(s, x)};
 }
 
-// Hands the legal moves of s that are not left out (at most 218) to the sink.
+// Hands the legal moves of s that are not left out to the sink (at most 218 in
+// a game; boards set up with 26 queens have 278).
 // Pawn captures carry the capture flag; other captures do not, as on the
 // reference's device path (MoveGeneratorBitboard.h:2525-2529).
 // First the king's and the pawns' moves and castling; false if the king alone

@@ -24,7 +24,7 @@
 namespace pg {
 
 constexpr int S_MAX_PLY = 16;
-constexpr int S_MOVES = 218;  // most moves of a position
+constexpr int S_MOVES = 218;  // most moves of a position in a game
 
 // A kept board: the paths that reach it are w, or, until the level kernel has
 // run, w + set[slot].w (the paths merged into it by the collapse).
@@ -465,9 +465,9 @@ __device__ __forceinline__ u64 s_hash(const Pos &p) {
 
 // Collapse of ply l: each listed move is made, and inserted in an
 // open-addressing set; the first of equal boards owns the slot and becomes a
-// node, the others add their weight to the slot.  A slot holds 32 bits of the
-// hash beside the owner's item, so only a probable match is compared: the
-// owner is made again from the list and compared board for board.  Bound by
+// node, the others add their weight to the slot.  A slot holds 16 bits of the
+// hash beside the owner's item, so that of the unequal boards met one in 65536
+// is compared: the owner is made again from the list and compared board for board.  Bound by
 // the random accesses to the set and to the owners' parents, and by their
 // latency: a work-group waits for its longest probe sequence before it
 // reserves its nodes with one atomic (all on one counter, hence large
