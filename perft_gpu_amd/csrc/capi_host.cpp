@@ -71,6 +71,11 @@ int parse_fen(const char *fen, Pos &p) {
 
 const HostTables *tables_or_null() { return host_tables(nullptr); }
 
+// room for the moves of any board: a square is entered by sliders from at most
+// eight sides, by eight knights and by four pawn moves, three of which are four
+// on the last rank, and one king moves
+constexpr u32 MOST_MOVES = 1400;
+
 u64 next_rand(u64 &s) {  // splitmix64
     u64 z = (s += 0x9E3779B97F4A7C15ULL);
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
@@ -195,8 +200,8 @@ namespace {
 u64 host_perft(const Pos &p, u32 depth, const Tables &t, bool *ovf) {
     if (depth == 0) return 1;
     if (depth == 1) return count_any<SL_FANCY>(p, t);
-    u16 mv[256];
-    const u32 n = generate_any<SL_FANCY>(p, t, mv, 256);
+    u16 mv[MOST_MOVES];
+    const u32 n = generate_any<SL_FANCY>(p, t, mv, MOST_MOVES);
     u64 s = 0;
     for (u32 i = 0; i < n && !*ovf; i++) {
         Pos q = p;
@@ -234,12 +239,12 @@ int pg_host_children(const pg_pos48 *pos, uint32_t n, pg_pos48 *out, uint64_t ca
     if (n && (!pos || !counts)) return PG_EINVAL;
     const Tables t = h->view();
     u64 w = 0;
-    u16 mv[256];
+    u16 mv[MOST_MOVES];
     for (uint32_t i = 0; i < n; i++) {
         Pos p;
         memcpy(&p, &pos[i], sizeof(p));
         if (!pos_sane(p)) return PG_EINVAL;
-        const u32 c = generate_any<SL_FANCY>(p, t, mv, 256);
+        const u32 c = generate_any<SL_FANCY>(p, t, mv, MOST_MOVES);
         counts[i] = c;
         if (w + c > cap) return PG_ENOMEM;
         for (u32 j = 0; j < c; j++) {

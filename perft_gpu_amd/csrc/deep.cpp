@@ -196,6 +196,10 @@ struct DeepWalk {
         pg_move moves[256];
         uint32_t n = 0;
         if ((rc = pg_host_generate_moves(&p, moves, &n)) != PG_OK) return 0;
+        if (n > 256) {  // more queens than a game has: the list holds the first 256
+            rc = PG_EINVAL;
+            return 0;
+        }
         // quiet moves first, as sortMoves orders them (launcher.h:367-391)
         std::stable_partition(moves, moves + n, [](pg_move m) { return (m >> 12) == 0; });
         u128 total = 0;
