@@ -51,11 +51,11 @@ struct Plan {
     u64 liveN;          // entries of the leaf level's live list
     u64 began;          // device clock at the search's start
     u32 arrived[TT_MAX_DEPTH];  // work-groups done with a level's kd_scan
-    DLevel lv[TT_MAX_DEPTH];
     // A root that no game leads to was seen (pos_regular): nothing is searched,
-    // and the host runs the search again with the plain leaf.  Kept from search
-    // to search: set by kd_begin, cleared by kd_end.
+    // and the host runs the search again with the plain leaf.  Not among what
+    // kd_begin copies: set by it, cleared by kd_end.
     u64 irregular;
+    DLevel lv[TT_MAX_DEPTH];
 };
 
 // A search's inputs and results in pinned host memory, which its first and
@@ -110,7 +110,8 @@ __global__ __launch_bounds__(wg_size<V>()) void kd_begin(Plan *P, const Link *H,
     stage_tables<V>(t);
     if (blockIdx.x == 0) {
         const u64 *from = (const u64 *)&H->plan;
-        for (u32 i = threadIdx.x; i < offsetof(Plan, irregular) / 8; i += blockDim.x) ((u64 *)P)[i] = from[i];
+        for (u32 i = threadIdx.x; i < sizeof(Plan) / 8; i += blockDim.x)
+            if (i != offsetof(Plan, irregular) / 8) ((u64 *)P)[i] = from[i];
         __syncthreads();
         if (threadIdx.x == 0) {
             P->began = wall_clock64();
